@@ -244,6 +244,16 @@ int qtx_resconv_metropolis(void* stream, const qtx_resconv_desc* d, const void* 
 int qtx_resconv_eloc(void* stream, const qtx_resconv_desc* d, const void* packed, const qtx_ham* H,
                      const int8_t* s, const double* logabs, int64_t ns, double* eloc, int32_t* nconn);
 
+/* The same with a workspace of qtx_resconv_eloc_ws_bytes(d, H, ns) bytes (0
+ * when none is needed; ws NULL: as qtx_resconv_eloc), in which the candidates
+ * of a sample are split over several workgroups when there are too few
+ * samples to fill the GPU.  Equal to qtx_resconv_eloc up to the order of the
+ * FP64 sum over candidates. */
+size_t qtx_resconv_eloc_ws_bytes(const qtx_resconv_desc* d, const qtx_ham* H, int64_t ns);
+int qtx_resconv_eloc_ws(void* stream, const qtx_resconv_desc* d, const void* packed, const qtx_ham* H,
+                        const int8_t* s, const double* logabs, int64_t ns, double* eloc, int32_t* nconn, void* ws,
+                        size_t ws_bytes);
+
 /* Per-sample log-derivatives O (ns, nparams) float32 via a per-sample
  * backward pass.  ws: qtx_resconv_jacobian_ws_bytes(d, ns) bytes. */
 size_t qtx_resconv_jacobian_ws_bytes(const qtx_resconv_desc* d, int64_t ns);

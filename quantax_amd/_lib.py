@@ -83,6 +83,9 @@ PROTOS = {
     "qtx_resconv_metropolis": (C.c_int, [vp, C.POINTER(QtxResConvDesc), vp, C.c_int, vp, i32, i32, vp, i32, i64,
                                          f64, f64, vp, vp, vp, vp]),
     "qtx_resconv_eloc": (C.c_int, [vp, C.POINTER(QtxResConvDesc), vp, C.POINTER(QtxHam), vp, vp, i64, vp, vp]),
+    "qtx_resconv_eloc_ws_bytes": (sz, [C.POINTER(QtxResConvDesc), C.POINTER(QtxHam), i64]),
+    "qtx_resconv_eloc_ws": (C.c_int, [vp, C.POINTER(QtxResConvDesc), vp, C.POINTER(QtxHam), vp, vp, i64, vp, vp, vp,
+                                      sz]),
     "qtx_resconv_jacobian_ws_bytes": (sz, [C.POINTER(QtxResConvDesc), i64]),
     "qtx_resconv_jacobian": (C.c_int, [vp, C.POINTER(QtxResConvDesc), vp, vp, i64, vp, vp, sz]),
     "qtx_resconv_jacobian_noalloc": (C.c_int, [vp, C.POINTER(QtxResConvDesc), vp, vp, i64, vp]),

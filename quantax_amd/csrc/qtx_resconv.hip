@@ -17,6 +17,7 @@
 //   BF16X3 : chunk j < C/8 = hi(channels 8j .. 8j+7), chunk C/8 + j = lo(...)
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include <string>
@@ -1534,8 +1535,11 @@ constexpr int RC_MAXCAND_WIN = 3072;  // 16 x 16 window kernels: keeps two workg
 
 template <int C, int MODE, int B, int NMAX, int MAXT, int W, int ROWS>
 __global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS == 3 ? 2 : (W == 8 ? 2 : 1)))) void rc_eloc_kernel(RcArgs a, qtx_ham H, const int8_t* __restrict__ s,
-                                                             const double* __restrict__ logabs, int64_t ns,
+                                                             const double* __restrict__ logabs, int S,
                                                              double* __restrict__ eloc, int32_t* __restrict__ nconn) {
+  // S workgroups per sample (virtual block n S + sp): workgroup sp evaluates
+  // the sp-th of S near-equal runs of candidates into eloc[n S + sp] (partial
+  // sums for rc_eloc_sum_kernel when S > 1, the local energy when S = 1)
   __shared__ __attribute__((aligned(16))) char act[(ROWS >= 2 ? 1 : 2) * B * NMAX * C * 4];
   __shared__ __attribute__((aligned(16))) char wst[ROWS == 2 ? rc_win_lds(B) : (ROWS == 3 ? rc32_tab_bytes(NMAX) : 16)];
   __shared__ int8_t s0[NMAX];
@@ -1548,7 +1552,8 @@ __global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS =
   __shared__ int16_t mv[4 * B];  // slot b: flips applied (2), flips of the next candidate (2)
   const int N = a.g.N;
   const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
-  const int64_t n = blockIdx.x;
+  const int64_t n = blockIdx.x / (unsigned)S;
+  const int sp = (int)(blockIdx.x % (unsigned)S);
   for (int i = threadIdx.x; i < N; i += (W * WAVE)) s0[i] = s[n * N + i];
   if constexpr (ROWS == 3) rc32_build_tab(a.g, reinterpret_cast<uint16_t*>(wst));
   __syncthreads();
@@ -1570,7 +1575,12 @@ __global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS =
     }
   }
   __syncthreads();
-  const int nvalid = nvalid_s;
+  const int nall = nvalid_s;
+  // runs start at multiples of B candidates
+  const int nbatch = (nall + B - 1) / B;
+  const int first = (int)((int64_t)nbatch * sp / S) * B;
+  const int last = (int)((int64_t)nbatch * (sp + 1) / S) * B;
+  const int nvalid = last < nall ? last : nall;  // end of this workgroup's run
   const double lp0 = logabs[n];
   // prop[b] holds s0 with candidate start + b applied: thread b < B undoes
   // the previous candidate's (at most two) flips and applies the next one's,
@@ -1580,8 +1590,8 @@ __global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS =
   if (threadIdx.x < B) {
     const int b = threadIdx.x;
     int na = -1, nb = -1;
-    if (b < nvalid) {
-      const int k = vlist[b];
+    if (first + b < nvalid) {
+      const int k = vlist[first + b];
       na = H.off_a[k];
       nb = H.off_b[k];
     }
@@ -1598,7 +1608,7 @@ __global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS =
     if (nb >= 0) pb[nb] = -s0[nb];
   }
   __syncthreads();
-  for (int start = 0; start < nvalid; start += B) {
+  for (int start = first; start < nvalid; start += B) {
     // thread b < B: the next candidate's sites and this candidate's coupling,
     // fetched before the forward and held in registers across it (their
     // global-memory latency hidden by the forward)
@@ -1636,11 +1646,20 @@ __global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS =
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    eloc[n] = diag_s + e_s;
-    if (nconn) nconn[n] = nvalid;
+    eloc[blockIdx.x] = (sp == 0) ? diag_s + e_s : e_s;
+    if (nconn && sp == 0) nconn[n] = nall;
   }
 }
 #undef RC_FWD
+
+// eloc[n] = sum of sample n's S partial sums, in order
+__global__ void rc_eloc_sum_kernel(const double* __restrict__ part, int64_t ns, int S, double* __restrict__ eloc) {
+  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= ns) return;
+  double e = 0.0;
+  for (int sp = 0; sp < S; ++sp) e += part[n * S + sp];
+  eloc[n] = e;
+}
 
 
 // ---------------------------------------------------------------- Jacobian
@@ -2081,8 +2100,32 @@ int qtx_resconv_metropolis(void* stream, const qtx_resconv_desc* d, const void* 
   return QTX_OK;
 }
 
-int qtx_resconv_eloc(void* stream, const qtx_resconv_desc* d, const void* packed, const qtx_ham* H,
-                     const int8_t* s, const double* logabs, int64_t ns, double* eloc, int32_t* nconn) {
+// Workgroups per sample of an E_loc launch.  One workgroup takes a sample's
+// candidates one batch after another, so a launch of few samples leaves the
+// card's 512 slots (256 CUs, two workgroups each) idle and one of a few
+// rounds ends in a nearly empty round: the candidates are split until the
+// launch has about 16 rounds, in runs of at least 8 batches (the scan that
+// lists a sample's candidates costs each workgroup about as much as one
+// forward of a small network).  A quarter of the table is the valid share of
+// an exchange Hamiltonian at Sz = 0; with a larger share the runs are longer.
+// Measured on J1-J2: 128 samples of 20 x 20, 32 channels, 16 blocks 219.6 ->
+// 65.3 ms; 2048 samples of 16 x 16, 8 blocks 53.2 -> 51.3 ms; 1000 samples of
+// 10 x 10, 4 blocks (FP32) 17.6 -> 17.0 ms.
+static int eloc_split(const RcLayout& L, int32_t noff, int64_t ns) {
+  const int64_t want = (16 * 512 + ns - 1) / ns;
+  const int64_t most = noff / 4 / ((L.C == 16 && L.N <= 256) ? 16 : 8);
+  return (int)std::max<int64_t>(1, std::min(want, most));
+}
+
+size_t qtx_resconv_eloc_ws_bytes(const qtx_resconv_desc* d, const qtx_ham* H, int64_t ns) {
+  if (rc_check(d) != QTX_OK || H == nullptr || H->noff < 0 || ns <= 0) return 0;
+  const int S = eloc_split(rc_layout(d), H->noff, ns);
+  return S > 1 ? (size_t)ns * S * sizeof(double) : 0;
+}
+
+int qtx_resconv_eloc_ws(void* stream, const qtx_resconv_desc* d, const void* packed, const qtx_ham* H,
+                        const int8_t* s, const double* logabs, int64_t ns, double* eloc, int32_t* nconn, void* ws,
+                        size_t ws_bytes) {
   int rc = rc_check(d);
   if (rc) return rc;
   QTX_REQUIRE(H != nullptr, "null qtx_ham");
@@ -2096,13 +2139,28 @@ int qtx_resconv_eloc(void* stream, const qtx_resconv_desc* d, const void* packed
   QTX_REQUIRE(packed && ns >= 0 && (ns == 0 || (s && logabs && eloc)), "bad arguments");
   if (ns == 0) return QTX_OK;
   QTX_REQUIRE(ns <= 0x7fffffff, "ns too large");
+  int S = 1;
+  if (ws != nullptr) {
+    S = eloc_split(L, H->noff, ns);
+    const size_t need = S > 1 ? (size_t)ns * S * sizeof(double) : 0;
+    if (ws_bytes < need)
+      return fail(QTX_EWORKSPACE, "workspace too small: need " + std::to_string(need) + " bytes");
+  }
   RcArgs a = rc_args(L, packed);
   hipStream_t st = as_stream(stream);
+  double* out = S > 1 ? (double*)ws : eloc;
   int per = 1;
-  RC_DISPATCH(rc_eloc_kernel, per, dim3((unsigned)ns), a, *H, s, logabs, ns, eloc, nconn);
+  RC_DISPATCH(rc_eloc_kernel, per, dim3((unsigned)(ns * S)), a, *H, s, logabs, S, out, nconn);
   (void)per;
+  if (S > 1)
+    hipLaunchKernelGGL(rc_eloc_sum_kernel, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, st, out, ns, S, eloc);
   QTX_LAUNCH_CHECK();
   return QTX_OK;
+}
+
+int qtx_resconv_eloc(void* stream, const qtx_resconv_desc* d, const void* packed, const qtx_ham* H,
+                     const int8_t* s, const double* logabs, int64_t ns, double* eloc, int32_t* nconn) {
+  return qtx_resconv_eloc_ws(stream, d, packed, H, s, logabs, ns, eloc, nconn, nullptr, 0);
 }
 
 static int64_t jac_chunk(int64_t ns) { return ns < 2048 ? ns : 2048; }

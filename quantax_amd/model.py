@@ -186,8 +186,11 @@ class ResConv(_Model):
         ns = s.shape[0]
         e = torch.empty(ns, dtype=torch.float64, device=s.device)
         nc = torch.empty(ns, dtype=torch.int32, device=s.device)
-        _lib.call("qtx_resconv_eloc", _lib.stream(), self.desc, self.packed.data_ptr(), H.device_tables(),
-                  s.data_ptr(), logabs.contiguous().data_ptr(), ns, e.data_ptr(), nc.data_ptr())
+        ham = H.device_tables()
+        wsb = int(_lib.lib().qtx_resconv_eloc_ws_bytes(self.desc, ham, ns))
+        ws = torch.empty(wsb, dtype=torch.uint8, device=s.device) if wsb else None
+        _lib.call("qtx_resconv_eloc_ws", _lib.stream(), self.desc, self.packed.data_ptr(), ham, s.data_ptr(),
+                  logabs.contiguous().data_ptr(), ns, e.data_ptr(), nc.data_ptr(), _lib.ptr(ws), wsb)
         return e, nc
 
     def jacobian(self, s: torch.Tensor, out_dtype=None):
