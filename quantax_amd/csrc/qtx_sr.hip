@@ -100,23 +100,9 @@ __global__ __launch_bounds__(1024) void ebar_kernel(const double* __restrict__ E
 }
 
 // ---------------------------------------------------------------- Gram T = A A^T
-// A = Obar (n x np) from O rows.  Workgroup: 256 threads = 2 x 2 waves, tile
-// 128 x 128 (each wave 64 x 64 = 4 x 4 MFMA 16x16 blocks); only tiles with
-// bi >= bj are computed and mirrored.  Output T is FP64 (n x n, symmetric).
-constexpr int GT = 128;
-
-template <int G>
-struct GramCfg;
-template <>
-struct GramCfg<QTX_GRAM_FP32> {
-  static constexpr int KC = 32;   // K elements staged per chunk
-  static constexpr int PAD = 1;   // LDS row padding (elements)
-};
-template <>
-struct GramCfg<QTX_GRAM_FP64> {
-  static constexpr int KC = 16;
-  static constexpr int PAD = 1;
-};
+// A = Obar (n x np) from O rows; only tiles with bi >= bj are computed and
+// mirrored.  Output T is FP64 (n x n, symmetric).
+constexpr int GT = 128;  // tile of the split-bf16 Gram
 
 __device__ __forceinline__ void tile_of(int bid, int& bi, int& bj) {
   // bid -> (bi, bj) with bj <= bi, row-major over the lower triangle
@@ -127,103 +113,150 @@ __device__ __forceinline__ void tile_of(int bid, int& bi, int& bj) {
   bj = bid - b * (b + 1) / 2;
 }
 
+// lower-triangle tile t of the XCD-contiguous order: workgroups are dealt to
+// the 8 XCDs round-robin, so block b runs on XCD b % 8; giving each XCD a
+// contiguous run of tiles (shared row panels) keeps them in its L2
+__device__ __forceinline__ int xcd_tile(int bid, int ntiles) {
+  const int per = ntiles / 8, rem = ntiles % 8, x = bid % 8, loc = bid / 8;
+  return x * per + (x < rem ? x : rem) + loc;
+}
+
+// FP64 / FP32 Gram on 16x16x4 MFMA.  The FP64 matrix pipe takes 64 cycles per
+// instruction, so LDS and L2 have room for a small tile: 64 x 64 per
+// workgroup (four waves of 32 x 32), four workgroups per CU, which leaves the
+// last round of a 4096-row Gram (2080 tiles on 256 CUs) 90 % full; a 128 x 128
+// tile would leave it at 69 %.  A thread stages four consecutive columns of
+// one row of each operand per 16-column chunk: one four-element load of O
+// (which needs only the element's own alignment, so any np takes it), fetched
+// one chunk ahead into registers, centred in FP64 and scaled by the row's
+// factor (formed once), then written to the other of two LDS buffers: one
+// barrier per chunk.  FP64, 4096 x 40400: 44.3 -> 13.5 ms (50 TFLOP/s; a
+// library f64 GEMM reaches 73); 4096 x 34952: 38.3 -> 11.5 ms.
+constexpr int GN_T = 64;    // tile
+constexpr int GN_KC = 16;   // columns per chunk
+constexpr int GN_LD = GN_KC + 1;
+
 template <typename TI, int G>
-__global__ __launch_bounds__(256) void gram_nt_kernel(const TI* __restrict__ O, const double* __restrict__ mean,
-                                                      const double* __restrict__ r, int64_t n, int64_t np,
-                                                      double inv_ns, double* __restrict__ T) {
-  constexpr int KC = GramCfg<G>::KC;
-  constexpr int LD = KC + GramCfg<G>::PAD;
+__global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ O, const double* __restrict__ mean,
+                                                         const double* __restrict__ r, int64_t n, int64_t np,
+                                                         double inv_ns, int ntiles, double* __restrict__ T) {
   using ST = typename std::conditional<G == QTX_GRAM_FP64, double, float>::type;
-  __shared__ ST As[1][GT * LD];
-  __shared__ ST Bs[1][GT * LD];
-
-  int bi, bj;
-  tile_of(blockIdx.x, bi, bj);
-  const int64_t i0 = (int64_t)bi * GT, j0 = (int64_t)bj * GT;
-  const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
-  const int wr = (wv / 2) * 64, wc = (wv % 2) * 64;  // wave's sub-tile origin
-
   using ACC = typename std::conditional<G == QTX_GRAM_FP64, v4d, v4f>::type;
-  ACC acc[4][4];
+  typedef TI vt4 __attribute__((ext_vector_type(4), aligned(sizeof(TI))));
+  __shared__ ST As[2][GN_T * GN_LD];
+  __shared__ ST Bs[2][GN_T * GN_LD];
+  int bi, bj;
+  tile_of(xcd_tile(blockIdx.x, ntiles), bi, bj);
+  const int64_t i0 = (int64_t)bi * GN_T, j0 = (int64_t)bj * GN_T;
+  const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
+  const int wr = (wv / 2) * 32, wc = (wv % 2) * 32;  // wave's sub-tile origin
+  // staging: row tid / 4, columns 4 (tid % 4) .. + 3; rows past n repeat row
+  // n - 1 (their outputs are not stored)
+  const int srow = tid / 4, sk = (tid % 4) * 4;
+  const int64_t ra = i0 + srow < n ? i0 + srow : n - 1, rb = j0 + srow < n ? j0 + srow : n - 1;
+  const TI* pa = O + ra * np;
+  const TI* pb = O + rb * np;
+  const double sa = sqrt((r ? r[ra] : 1.0) * inv_ns), sb = sqrt((r ? r[rb] : 1.0) * inv_ns);
+  TI av[4], bv[4];
+  double mv[4];
+  auto fetch = [&](int64_t k0) {
+    const int64_t k = k0 + sk;
+    if (k + 3 < np) {
+      const vt4 x = *reinterpret_cast<const vt4*>(pa + k), y = *reinterpret_cast<const vt4*>(pb + k);
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+      for (int q = 0; q < 4; ++q) {
+        av[q] = x[q];
+        bv[q] = y[q];
+        mv[q] = mean[k + q];
+      }
+    } else {
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = ACC{0, 0, 0, 0};
-  // the FP32 mode flushes its MFMA accumulators into FP64 every FLUSH chunks,
-  // so the rounding error does not grow with np
-  constexpr int FLUSH = 8;
+      for (int q = 0; q < 4; ++q) {
+        const bool ok = k + q < np;
+        av[q] = ok ? pa[k + q] : TI(0);
+        bv[q] = ok ? pb[k + q] : TI(0);
+        mv[q] = ok ? mean[k + q] : 0.0;
+      }
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      As[buf][srow * GN_LD + sk + q] = (ST)(((double)av[q] - mv[q]) * sa);
+      Bs[buf][srow * GN_LD + sk + q] = (ST)(((double)bv[q] - mv[q]) * sb);
+    }
+  };
+
+  ACC acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[a][b] = ACC{0, 0, 0, 0};
+  // the FP32 mode flushes its MFMA accumulators into FP64 every FLUSH chunks
+  // (256 columns), so the rounding error does not grow with np
+  constexpr int FLUSH = 256 / GN_KC;
   constexpr bool SHADOW = (G != QTX_GRAM_FP64);
-  v4d dacc[SHADOW ? 4 : 1][SHADOW ? 4 : 1];
+  v4d dacc[SHADOW ? 2 : 1][SHADOW ? 2 : 1];
   if constexpr (SHADOW) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) dacc[a][b] = v4d{0, 0, 0, 0};
+      for (int b = 0; b < 2; ++b) dacc[a][b] = v4d{0, 0, 0, 0};
   }
-  int chunk = 0;
 
-  for (int64_t k0 = 0; k0 < np; k0 += KC) {
-    // stage A rows [i0, i0+128) and B rows [j0, j0+128), columns [k0, k0+KC)
-    for (int e = tid; e < GT * KC; e += 256) {
-      int row = e / KC, kk = e % KC;
-      int64_t k = k0 + kk;
+  const int nchunks = (int)((np + GN_KC - 1) / GN_KC);
+  fetch(0);
+  stage(0);
+  __syncthreads();
+  for (int c = 0; c < nchunks; ++c) {
+    const ST* Ac = As[c & 1];
+    const ST* Bc = Bs[c & 1];
+    if (c + 1 < nchunks) fetch((int64_t)(c + 1) * GN_KC);
 #pragma unroll
-      for (int which = 0; which < 2; ++which) {
-        int64_t gr = (which == 0 ? i0 : j0) + row;
-        double v = 0.0;
-        if (gr < n && k < np) {
-          double sc = sqrt((r ? r[gr] : 1.0) * inv_ns);
-          v = ((double)O[gr * np + k] - mean[k]) * sc;
+    for (int ks = 0; ks < GN_KC; ks += 4) {
+      ST af[2], bf[2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        af[a] = Ac[(wr + a * 16 + lane % 16) * GN_LD + ks + lane / 16];
+        bf[a] = Bc[(wc + a * 16 + lane % 16) * GN_LD + ks + lane / 16];
+      }
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          if constexpr (G == QTX_GRAM_FP64)
+            acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[a], bf[b], acc[a][b], 0, 0, 0);
+          else
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[a], bf[b], acc[a][b], 0, 0, 0);
         }
-        ((which == 0) ? As[0] : Bs[0])[row * LD + kk] = (ST)v;
-      }
     }
-    __syncthreads();
-    {
-#pragma unroll
-      for (int ks = 0; ks < KC; ks += 4) {
-        ST av[4], bv[4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a) av[a] = As[0][(wr + a * 16 + lane % 16) * LD + ks + lane / 16];
-#pragma unroll
-        for (int b = 0; b < 4; ++b) bv[b] = Bs[0][(wc + b * 16 + lane % 16) * LD + ks + lane / 16];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            if constexpr (G == QTX_GRAM_FP64)
-              acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
-            else
-              acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a], bv[b], acc[a][b], 0, 0, 0);
-          }
-      }
-    }
-    __syncthreads();
     if constexpr (SHADOW) {
-      if (++chunk == FLUSH || k0 + KC >= np) {
-        chunk = 0;
+      if ((c + 1) % FLUSH == 0 || c + 1 == nchunks) {
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
+        for (int a = 0; a < 2; ++a)
 #pragma unroll
-          for (int b = 0; b < 4; ++b) {
+          for (int b = 0; b < 2; ++b) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) dacc[a][b][q] += (double)acc[a][b][q];
             acc[a][b] = ACC{0, 0, 0, 0};
           }
       }
     }
+    // the other buffer was last read before the previous barrier
+    if (c + 1 < nchunks) stage((c + 1) & 1);
+    __syncthreads();
   }
   // store, column lane%16 of each 16x16 block; rows of element q:
-  //   f32 / bf16 MFMA: 4 * (lane / 16) + q ;  f64 MFMA: lane / 16 + 4 * q
+  //   f32 MFMA: 4 * (lane / 16) + q ;  f64 MFMA: lane / 16 + 4 * q
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int rq = (G == QTX_GRAM_FP64) ? (lane / 16 + 4 * q) : (4 * (lane / 16) + q);
-        int64_t gi = i0 + wr + a * 16 + rq;
-        int64_t gj = j0 + wc + b * 16 + lane % 16;
+        const int64_t gi = i0 + wr + a * 16 + rq;
+        const int64_t gj = j0 + wc + b * 16 + lane % 16;
         // off-diagonal tiles are mirrored; inside diagonal tiles the lower
         // triangle is written to both halves so T is exactly symmetric
         if (gi < n && gj < n && (bi != bj || gi >= gj)) {
@@ -231,7 +264,7 @@ __global__ __launch_bounds__(256) void gram_nt_kernel(const TI* __restrict__ O, 
           if constexpr (SHADOW)
             v = dacc[a][b][q];
           else
-            v = (double)acc[a][b][q];
+            v = acc[a][b][q];
           T[gi * n + gj] = v;
           T[gj * n + gi] = v;
         }
@@ -270,14 +303,6 @@ __global__ __launch_bounds__(256) void split_bf16x3_kernel(const TI* __restrict_
     Hi[row * kpad + k] = hi;
     Lo[row * kpad + k] = (__bf16)(f - (float)hi);
   }
-}
-
-// lower-triangle tile t of the XCD-contiguous order: workgroups are dealt to
-// the 8 XCDs round-robin, so block b runs on XCD b % 8; giving each XCD a
-// contiguous run of tiles (shared row panels) keeps them in its L2
-__device__ __forceinline__ int xcd_tile(int bid, int ntiles) {
-  const int per = ntiles / 8, rem = ntiles % 8, x = bid % 8, loc = bid / 8;
-  return x * per + (x < rem ? x : rem) + loc;
 }
 
 typedef __attribute__((address_space(3))) void lds_void;
@@ -1268,10 +1293,14 @@ static int launch_gram_nt(hipStream_t st, int gram, const TI* O, const double* m
                        st, O, mean, r, n, np, kpad, bpr, nblocks, inv_ns, Hi, Lo);
     hipLaunchKernelGGL(gram_bf16x3_kernel, g, bl, 0, st, (const __bf16*)Hi, (const __bf16*)Lo, n, kpad, (int)ntiles,
                        T);
-  } else if (gram == QTX_GRAM_FP32) {
-    hipLaunchKernelGGL((gram_nt_kernel<TI, QTX_GRAM_FP32>), g, bl, 0, st, O, mean, r, n, np, inv_ns, T);
   } else {
-    hipLaunchKernelGGL((gram_nt_kernel<TI, QTX_GRAM_FP64>), g, bl, 0, st, O, mean, r, n, np, inv_ns, T);
+    const int64_t mt = (n + GN_T - 1) / GN_T, mtiles = mt * (mt + 1) / 2;
+    QTX_REQUIRE(mtiles < 0x7fffffff, "Gram too large");
+    const dim3 gm((unsigned)mtiles);
+    if (gram == QTX_GRAM_FP32)
+      hipLaunchKernelGGL((gram_nt_kernel<TI, QTX_GRAM_FP32>), gm, bl, 0, st, O, mean, r, n, np, inv_ns, (int)mtiles, T);
+    else
+      hipLaunchKernelGGL((gram_nt_kernel<TI, QTX_GRAM_FP64>), gm, bl, 0, st, O, mean, r, n, np, inv_ns, (int)mtiles, T);
   }
   QTX_LAUNCH_CHECK();
   return QTX_OK;
