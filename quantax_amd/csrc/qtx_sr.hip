@@ -121,6 +121,29 @@ __device__ __forceinline__ int xcd_tile(int bid, int ntiles) {
   return x * per + (x < rem ? x : rem) + loc;
 }
 
+// lower-triangle tile (bi, bj) of an mt x mt tile grid from its index t in the
+// order of 8 x 8 super-blocks (row-major over the triangle of super-blocks,
+// row-major inside each): tiles that run together share few row panels
+__device__ __forceinline__ void super_tile_of(int t, int mt, int& bi, int& bj) {
+  const int full = mt / 8;  // complete super-rows; super-row R starts at tile 32 R^2 + 4 R
+  int R = (int)((sqrt(16.0 + 128.0 * (double)t) - 4.0) / 64.0);
+  while (32LL * (R + 1) * (R + 1) + 4LL * (R + 1) <= t) ++R;
+  while (32LL * R * R + 4LL * R > t) --R;
+  if (R > full) R = full;
+  const int rem = t - (32 * R * R + 4 * R);
+  const int h = R < full ? 8 : mt - 8 * full;  // tile rows of this super-row
+  if (rem < 8 * h * R) {
+    const int sb = rem / (8 * h), in = rem - sb * 8 * h;
+    bi = 8 * R + in / 8;
+    bj = 8 * sb + in % 8;
+  } else {
+    int a, b;
+    tile_of(rem - 8 * h * R, a, b);
+    bi = 8 * R + a;
+    bj = 8 * R + b;
+  }
+}
+
 // FP64 / FP32 Gram on 16x16x4 MFMA.  The FP64 matrix pipe takes 64 cycles per
 // instruction, so LDS and L2 have room for a small tile: 64 x 64 per
 // workgroup (four waves of 32 x 32), four workgroups per CU, which leaves the
@@ -128,10 +151,12 @@ __device__ __forceinline__ int xcd_tile(int bid, int ntiles) {
 // tile would leave it at 69 %.  A thread stages four consecutive columns of
 // one row of each operand per 16-column chunk: one four-element load of O
 // (which needs only the element's own alignment, so any np takes it), fetched
-// one chunk ahead into registers, centred in FP64 and scaled by the row's
-// factor (formed once), then written to the other of two LDS buffers: one
-// barrier per chunk.  FP64, 4096 x 40400: 44.3 -> 13.5 ms (50 TFLOP/s; a
-// library f64 GEMM reaches 73); 4096 x 34952: 38.3 -> 11.5 ms.
+// one chunk ahead into registers and centred in FP64 (the rows' factors are
+// applied to the sums), then written to the other of two LDS buffers: one
+// barrier per chunk.  FP64, 4096 x 40400: 44.3 -> 12.9 ms; 4096 x 34952: 38.3
+// -> 11.2 ms; 16384 x 34952: 331 -> 156 ms (60 TFLOP/s, a library f64 GEMM
+// reaches 73).  The matrix pipe is busy 80 % of the time (SQ counters); the
+// FP64 conversions and subtractions, one per MFMA, are most of the rest.
 constexpr int GN_T = 64;    // tile
 constexpr int GN_KC = 16;   // columns per chunk
 constexpr int GN_LD = GN_KC + 1;
@@ -146,7 +171,7 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
   __shared__ ST As[2][GN_T * GN_LD];
   __shared__ ST Bs[2][GN_T * GN_LD];
   int bi, bj;
-  tile_of(xcd_tile(blockIdx.x, ntiles), bi, bj);
+  super_tile_of(xcd_tile(blockIdx.x, ntiles), (int)((n + GN_T - 1) / GN_T), bi, bj);
   const int64_t i0 = (int64_t)bi * GN_T, j0 = (int64_t)bj * GN_T;
   const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
   const int wr = (wv / 2) * 32, wc = (wv % 2) * 32;  // wave's sub-tile origin
@@ -156,7 +181,6 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
   const int64_t ra = i0 + srow < n ? i0 + srow : n - 1, rb = j0 + srow < n ? j0 + srow : n - 1;
   const TI* pa = O + ra * np;
   const TI* pb = O + rb * np;
-  const double sa = sqrt((r ? r[ra] : 1.0) * inv_ns), sb = sqrt((r ? r[rb] : 1.0) * inv_ns);
   TI av[4], bv[4];
   double mv[4];
   auto fetch = [&](int64_t k0) {
@@ -182,8 +206,8 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
   auto stage = [&](int buf) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      As[buf][srow * GN_LD + sk + q] = (ST)(((double)av[q] - mv[q]) * sa);
-      Bs[buf][srow * GN_LD + sk + q] = (ST)(((double)bv[q] - mv[q]) * sb);
+      As[buf][srow * GN_LD + sk + q] = (ST)((double)av[q] - mv[q]);
+      Bs[buf][srow * GN_LD + sk + q] = (ST)((double)bv[q] - mv[q]);
     }
   };
 
@@ -265,6 +289,7 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
             v = dacc[a][b][q];
           else
             v = acc[a][b][q];
+          v *= r ? sqrt(r[gi] * r[gj]) * inv_ns : inv_ns;
           T[gi * n + gj] = v;
           T[gj * n + gi] = v;
         }
