@@ -265,8 +265,8 @@ int qtx_resconv_jacobian(void* stream, const qtx_resconv_desc* d, const void* pa
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  The per-sample records live in a
  * 128 MiB file-scope device array of the library, one per GPU, held until the
- * process ends; samples run in launches of as many as it holds (e.g. 256 at
- * 16 x 16, 8 blocks, 16 channels).  Every call on a GPU shares that GPU's
+ * process ends; a launch has as many workgroups as it holds records for (e.g.
+ * 512 at 16 x 16, 8 blocks, 16 channels).  Every call on a GPU shares that GPU's
  * array: calls that overlap on one GPU (different streams or threads) race.
  * Returns QTX_EINVAL when one sample's records exceed the array. */
 int qtx_resconv_jacobian_noalloc(void* stream, const qtx_resconv_desc* d, const void* packed, const int8_t* s,

@@ -1,8 +1,7 @@
 // ResConv(nblocks, C, 3) on a periodic L0 x L1 grid: batched forward on MFMA
 // (FP32 16x16x4, or split-bf16 16x16x32 with FP32 accumulation), Metropolis
-// with one full forward per proposal, local energy over connected
-// configurations generated in LDS, and a per-sample backward for O whose
-// three convolution products per layer are FP32 MFMA GEMMs.
+// with one full forward per proposal and local energy over connected
+// configurations generated in LDS.
 //
 // Forward work unit ("item") = one 16-position tile of one configuration.
 // Convolution as an implicit GEMM per item: D[co, p] = sum_k W[co, k] X[k, p]
@@ -19,100 +18,12 @@
 
 #include <algorithm>
 #include <cmath>
-#include <mutex>
 #include <string>
 #include <type_traits>
 
-#include "common.hpp"
+#include "resconv.hpp"
 
 namespace qtx {
-
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
-typedef int v4i __attribute__((ext_vector_type(4)));
-
-constexpr int RC_WAVES = 4;
-constexpr int RC_THREADS = RC_WAVES * WAVE;
-constexpr int RC_MAXN = 1024;
-
-// ---------------------------------------------------------------- layout
-struct RcLayout {
-  int nb, C, L0, L1, N, mode, actk;
-  int win;                   // 16 x 16, C = 16: sliding-row-window forward and its K-step order
-  int64_t nparams;
-  int64_t off_l0w, off_l0b;  // first conv (Cin = 1): W (C, 9), b (C) in floats
-  int64_t off_frag;          // start of per-layer fragment blocks (bytes)
-  int64_t frag_bytes;        // bytes of one layer's fragments
-  int64_t bias_off;          // start of per-layer biases (floats, (2nb) x C)
-  int64_t total_bytes;
-};
-
-__host__ __device__ inline int64_t rc_nparams(int nb, int C) {
-  int64_t n = 0;
-  for (int i = 0; i < nb; ++i) {
-    int cin = (i == 0) ? 1 : C;
-    n += (int64_t)C * cin * 9 + C;                 // conv1 (+ bias)
-    n += (int64_t)C * C * 9 + ((i == nb - 1) ? 0 : C);  // conv2 (+ bias except last)
-  }
-  return n;
-}
-
-// offsets of layer l's weight/bias in the ravel_pytree vector
-__host__ __device__ inline void rc_theta_offsets(int nb, int C, int l, int64_t& w, int64_t& b) {
-  int64_t off = 0;
-  for (int ll = 0; ll < 2 * nb; ++ll) {
-    int i = ll / 2;
-    int cin = (ll == 0) ? 1 : C;
-    bool hb = !((ll % 2 == 1) && (i == nb - 1));
-    if (ll == l) {
-      w = off;
-      b = hb ? off + (int64_t)C * cin * 9 : -1;
-      return;
-    }
-    off += (int64_t)C * cin * 9 + (hb ? C : 0);
-  }
-  w = b = -1;
-}
-
-template <int C, int MODE>
-struct RcK {
-  static constexpr int CT = C / 16;                                   // output-channel tiles
-  static constexpr int KS = (MODE == QTX_CONV_FP32) ? (9 * C / 4) : (C == 16 ? 5 : 9);  // K steps
-  static constexpr int CH = C / 4;                                    // 16-byte chunks per position
-  static constexpr int FRAG_WORDS = (MODE == QTX_CONV_FP32) ? 1 : 8;  // 4-byte words per lane per (ct, ks)
-};
-
-inline RcLayout rc_layout(const qtx_resconv_desc* d) {
-  RcLayout L;
-  L.nb = d->nblocks;
-  L.C = d->channels;
-  L.L0 = d->L0;
-  L.L1 = d->L1;
-  L.N = d->L0 * d->L1;
-  L.mode = d->precision;
-  L.actk = d->activation;
-  L.win = (L.C == 16 && L.L0 == 16 && L.L1 == 16) ? 1 : 0;
-  L.nparams = rc_nparams(L.nb, L.C);
-  int64_t off = L.nparams * 4;  // raw theta copy first
-  off = (off + 255) & ~(int64_t)255;
-  L.off_l0w = off / 4;
-  off += (int64_t)L.C * 9 * 4;
-  L.off_l0b = off / 4;
-  off += (int64_t)L.C * 4;
-  off = (off + 255) & ~(int64_t)255;
-  L.bias_off = off / 4;
-  off += (int64_t)2 * L.nb * L.C * 4;
-  off = (off + 255) & ~(int64_t)255;
-  L.off_frag = off;
-  int ct = L.C / 16;
-  int ks = (L.mode == QTX_CONV_FP32) ? 9 * L.C / 4 : (L.C == 16 ? (L.win ? 6 : 5) : 9);
-  int words = (L.mode == QTX_CONV_FP32) ? 1 : 8;
-  L.frag_bytes = (int64_t)ct * ks * WAVE * words * 4;
-  off += L.frag_bytes * 2 * L.nb;  // slot per layer index (slot 0 unused)
-  L.total_bytes = off;
-  return L;
-}
 
 // ---------------------------------------------------------------- packing
 // one thread per (layer, ct, ks, lane) fragment for layers 1 .. 2nb-1
@@ -195,6 +106,27 @@ __global__ void rc_pack_frag_kernel(const float* __restrict__ theta, int nb, cha
   }
 }
 
+// The Jacobian's FP32 A fragments of layers 1 .. 2nb-1, whatever the forward's
+// precision: per layer and direction (0: forward, 1: input gradient, with the
+// two channel indices exchanged and the taps mirrored) [tap][row tile][column
+// half][lane][4]: row = 16 ct + lane % 16, column = 16 h + 4 (lane / 16) + j,
+// so a lane reads its four K values of a tap in one 16-byte load
+template <int C>
+__global__ void rc_pack_jac_kernel(const float* __restrict__ theta, int nb, float* __restrict__ dst) {
+  constexpr int CT = C / 16;
+  const int64_t per = (int64_t)C * C * 9;
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= (int64_t)(2 * nb - 1) * 2 * per) return;
+  const int l = 1 + (int)(idx / (2 * per)), dir = (int)(idx / per) & 1;
+  const int e = (int)(idx % per);
+  const int j = e % 4, lane = (e / 4) % WAVE, h = (e / 256) % CT, ct = (e / 256 / CT) % CT, tap = e / 256 / CT / CT;
+  const int row = 16 * ct + lane % 16, col = 16 * h + 4 * (lane / 16) + j;
+  int64_t w0, b0;
+  rc_theta_offsets(nb, C, l, w0, b0);
+  dst[((int64_t)l * 2 + dir) * per + e] =
+      dir == 0 ? theta[w0 + ((int64_t)row * C + col) * 9 + tap] : theta[w0 + ((int64_t)col * C + row) * 9 + (8 - tap)];
+}
+
 __global__ void rc_pack_misc_kernel(const float* __restrict__ theta, int nb, int C, int64_t nparams,
                                     float* __restrict__ packed, int64_t off_l0w, int64_t off_l0b, int64_t bias_off) {
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -210,31 +142,6 @@ __global__ void rc_pack_misc_kernel(const float* __restrict__ theta, int nb, int
     rc_theta_offsets(nb, C, l, w0, b0);
     packed[bias_off + j] = (b0 >= 0) ? theta[b0 + co] : 0.0f;
   }
-}
-
-// ---------------------------------------------------------------- math
-// Activations (qtx_resconv_desc.activation): QTX_ACT_GELU_TANH, the
-// reference's jax.nn.gelu default (model/conv_nets.py:85, 87),
-// QTX_ACT_GELU_ERF, and QTX_ACT_RELU (max(x, 0), derivative 0 at x <= 0, as
-// jax.nn.relu), an opt-in variant with no counterpart in the reference.
-// tanh form: 0.5 x (1 + tanh(k (x + 0.044715 x^3))) = x / (1 + 2^(x (A + B x^2)))
-// with A = -2 k log2(e), B = -2 k 0.044715 log2(e), k = sqrt(2 / pi); native exp2 and rcp
-__device__ __forceinline__ float act_f(float x, int actk) {
-  if (actk == QTX_ACT_RELU) return fmaxf(x, 0.0f);
-  if (actk == QTX_ACT_GELU_ERF) return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
-  constexpr float A = -2.0f * 0.79788456080286536f * 1.4426950408889634f;
-  constexpr float Bc = A * 0.044715f;
-  float e = __builtin_amdgcn_exp2f(x * fmaf(x * x, Bc, A));
-  return x * __builtin_amdgcn_rcpf(1.0f + e);
-}
-
-__device__ __forceinline__ float act_grad_f(float x, int actk) {
-  if (actk == QTX_ACT_RELU) return x > 0.0f ? 1.0f : 0.0f;
-  if (actk == QTX_ACT_GELU_ERF)
-    return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * __expf(-0.5f * x * x) * 0.39894228040143268f;
-  float u = 0.79788456080286536f * (x + 0.044715f * x * x * x);
-  float t = 1.0f - 2.0f / (1.0f + __expf(2.0f * u));
-  return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * 0.79788456080286536f * (1.0f + 0.134145f * x * x);
 }
 
 // v = hi + lo + O(2^-16 |v|): hi = bf16(v) (round to nearest even), lo =
@@ -267,19 +174,6 @@ __device__ __forceinline__ int swz_chunk(int p, int j) {
   // fall on distinct 16-byte bank groups
   constexpr int CH = C / 4;
   return j ^ ((p / (8 / CH)) & (CH - 1));
-}
-
-struct RcGeom {
-  int L0, L1, N, NT;
-  double log_cn;  // log(C N): the head's normalisation
-};
-
-__device__ __forceinline__ int tap_pos(const RcGeom& g, int y, int x, int tap) {
-  int dy = tap / 3 - 1, dx = tap % 3 - 1;
-  int ys = y + dy, xs = x + dx;
-  ys = ys < 0 ? ys + g.L0 : (ys >= g.L0 ? ys - g.L0 : ys);
-  xs = xs < 0 ? xs + g.L1 : (xs >= g.L1 ? xs - g.L1 : xs);
-  return ys * g.L1 + xs;
 }
 
 // Write 4 consecutive channels (c4 .. c4+3, c4 % 4 == 0) of position p.
@@ -1662,297 +1556,11 @@ __global__ void rc_eloc_sum_kernel(const double* __restrict__ part, int64_t ns, 
 }
 
 
-// ---------------------------------------------------------------- Jacobian
-// One workgroup (4 waves) per sample.  Every convolution of the forward
-// recompute and of the backward pass is an FP32-MFMA GEMM (16x16x4 f32) whose
-// operands are gathered from channel-major [c][p] activations in LDS through a
-// table of the 9 periodic neighbours of every site:
-//   forward   Z[co][p]     = sum_{ci,tap} W[co][ci][tap] X[ci][nb(p, tap)]
-//   input grad dX[ci][q]   = sum_{co,tap} W[co][ci][tap] dZ[co][nb(q, 8 - tap)]
-//   weight grad G[co][ci,tap] = sum_p dZ[co][p] X[ci][nb(p, tap)]
-// (MFMA lane l holds A[m0 + l%16][k0 + l/16], B[k0 + l/16][n0 + l%16]; result
-// element i of lane l is D[m0 + 4(l/16) + i][n0 + l%16].)  The forward records,
-// per block i, x_i (block input), y_i (conv1 input), z1_i (conv1 output) and
-// a1_i (conv2 input) in HBM workspace; the backward produces the O row in
-// ravel_pytree order (per layer weight (co, ci, tap), bias (co)).
-constexpr int JAC_THREADS = 256;
-
-__device__ __forceinline__ v4f mfma_f32_4(float a, float b, v4f c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// out[co][p] for all co < C, p < N; K = cin * 9; A fragments (weights) of a
-// 16-row tile held in registers across the wave's column tiles.
-template <int C, int KS, typename Epi>
-__device__ __forceinline__ void jac_conv_fwd_mfma(const float* __restrict__ in, const float* __restrict__ W,
-                                                  const int16_t* __restrict__ nbr, int N, int nmax, Epi epi) {
-  constexpr int K = (KS == 3) ? 9 : C * 9;  // cin * 9
-  const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
-  const int ntile = (N + 15) / 16;
-#pragma unroll
-  for (int m0 = 0; m0 < C; m0 += 16) {
-    float af[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int k = 4 * ks + lane / 16;
-      af[ks] = (k < K) ? W[(m0 + lane % 16) * K + k] : 0.0f;
-    }
-    for (int t = wv; t < ntile; t += JAC_THREADS / WAVE) {
-      const int p = 16 * t + lane % 16;
-      const int pc = p < N ? p : N - 1;
-      v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int k = 4 * ks + lane / 16;
-        const int ci = k / 9, tap = k - 9 * ci;
-        const float b = (k < K) ? in[ci * N + nbr[tap * nmax + pc]] : 0.0f;
-        acc = mfma_f32_4(af[ks], b, acc);
-      }
-      const int pw = 16 * t + lane % 16;
-      if (pw < N) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) epi(m0 + 4 * (lane / 16) + i, pw, acc[i]);
-      }
-    }
-  }
-}
-
-// din[ci][q] for all ci < C (input channels of a C -> C convolution)
-template <int C, typename Epi>
-__device__ __forceinline__ void jac_conv_bwd_in_mfma(const float* __restrict__ dz, const float* __restrict__ W,
-                                                     const int16_t* __restrict__ nbr, int N, int nmax, Epi epi) {
-  constexpr int KS = C * 9 / 4;
-  const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
-  const int ntile = (N + 15) / 16;
-#pragma unroll
-  for (int m0 = 0; m0 < C; m0 += 16) {
-    float af[KS];
-    const int ci = m0 + lane % 16;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int k = 4 * ks + lane / 16;
-      const int co = k / 9, tap = k - 9 * co;
-      af[ks] = W[(co * C + ci) * 9 + tap];
-    }
-    for (int t = wv; t < ntile; t += JAC_THREADS / WAVE) {
-      const int q = 16 * t + lane % 16;
-      const int qc = q < N ? q : N - 1;
-      v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int k = 4 * ks + lane / 16;
-        const int co = k / 9, tap = k - 9 * co;
-        acc = mfma_f32_4(af[ks], dz[co * N + nbr[(8 - tap) * nmax + qc]], acc);
-      }
-      if (q < N) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) epi(m0 + 4 * (lane / 16) + i, q, acc[i]);
-      }
-    }
-  }
-}
-
-// G[co][n], n = ci * 9 + tap < cin * 9, written to the O row; bias grads by VALU
-template <int C>
-__device__ __forceinline__ void jac_conv_grad_w_mfma(const float* __restrict__ dz, const float* __restrict__ x, int cin,
-                                                     const int16_t* __restrict__ nbr, int N, int nmax,
-                                                     float* __restrict__ Orow, int64_t w0, int64_t b0) {
-  const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
-  const int K9 = cin * 9;
-  const int ncol = (K9 + 15) / 16;
-  const int ntiles = (C / 16) * ncol;
-  const int ksteps = (N + 3) / 4;
-  for (int t = wv; t < ntiles; t += JAC_THREADS / WAVE) {
-    const int m0 = 16 * (t % (C / 16)), n0 = 16 * (t / (C / 16));
-    const int co = m0 + lane % 16;
-    const int n = n0 + lane % 16;
-    const bool nok = n < K9;
-    const int ci = nok ? n / 9 : 0, tap = nok ? n - 9 * (n / 9) : 0;
-    const float* xr = x + ci * N;
-    const int16_t* nr = nbr + tap * nmax;
-    const float* dr = dz + co * N;
-    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-    for (int ks = 0; ks < ksteps; ++ks) {
-      const int p = 4 * ks + lane / 16;
-      const bool pok = p < N;
-      const float a = pok ? dr[p] : 0.0f;
-      const float b = (pok && nok) ? xr[nr[pok ? p : 0]] : 0.0f;
-      acc = mfma_f32_4(a, b, acc);
-    }
-    if (nok) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) Orow[w0 + (int64_t)(m0 + 4 * (lane / 16) + i) * K9 + n] = acc[i];
-    }
-  }
-  if (b0 >= 0) {
-    for (int c = wv; c < C; c += JAC_THREADS / WAVE) {
-      float acc = 0.0f;
-      for (int p = lane; p < N; p += WAVE) acc += dz[c * N + p];
-      acc = wave_sum(acc);
-      if (lane == 0) Orow[b0 + c] = acc;
-    }
-  }
-}
-
-template <int C, int NMAX>
-__global__ __launch_bounds__(JAC_THREADS) void rc_jacobian_kernel(RcGeom g, int nb, int actk,
-                                                                  const float* __restrict__ theta,
-                                                                  const int8_t* __restrict__ s, int64_t s0,
-                                                                  int64_t ns_chunk, int64_t np,
-                                                                  float* __restrict__ O, float* __restrict__ ws) {
-  __shared__ float buf0[C * NMAX];
-  __shared__ float buf1[C * NMAX];
-  __shared__ float buf2[C * NMAX];
-  __shared__ int16_t nbr[9 * NMAX];
-  __shared__ float red[2 * JAC_THREADS / WAVE];
-  const int64_t nl = blockIdx.x;
-  if (nl >= ns_chunk) return;
-  const int64_t n = s0 + nl;
-  const int N = g.N;
-  const int64_t blk_f = (int64_t)4 * C * N;
-  float* rec = ws + nl * blk_f * nb;
-  float* Orow = O + n * np;
-  const float isq2 = 0.70710678118654752f;
-  float* bX = buf0;  // block input / running gradient
-  float* bA = buf1;
-  float* bB = buf2;
-
-  for (int e = threadIdx.x; e < 9 * N; e += JAC_THREADS) {
-    const int tap = e / N, p = e - tap * N;
-    nbr[tap * NMAX + p] = (int16_t)tap_pos(g, p / g.L1, p % g.L1, tap);
-  }
-  // ---- forward with record
-  for (int p = threadIdx.x; p < N; p += JAC_THREADS) bX[p] = (float)s[n * N + p];
-  __syncthreads();
-  for (int i = 0; i < nb; ++i) {
-    const int cin = (i == 0) ? 1 : C;
-    float* rx = rec + i * blk_f;
-    float* ry = rx + C * N;
-    float* rz = ry + C * N;
-    float* ra = rz + C * N;
-    const float sc = rsqrtf((float)(i + 1));
-    for (int e = threadIdx.x; e < cin * N; e += JAC_THREADS) {
-      float xv = bX[e];
-      rx[e] = xv;
-      float xin = xv * sc;
-      float yv = (i == 0) ? xin * isq2 : act_f(xin, actk);
-      bA[e] = yv;
-      ry[e] = yv;
-    }
-    __syncthreads();
-    int64_t w1, b1, w2, b2;
-    rc_theta_offsets(nb, C, 2 * i, w1, b1);
-    rc_theta_offsets(nb, C, 2 * i + 1, w2, b2);
-    {
-      const float* bias = theta + b1;
-      auto epi = [&](int co, int p, float v) {
-        v += bias[co];
-        rz[co * N + p] = v;
-        const float a = act_f(v, actk);
-        bB[co * N + p] = a;
-        ra[co * N + p] = a;
-      };
-      if (i == 0)
-        jac_conv_fwd_mfma<C, 3>(bA, theta + w1, nbr, N, NMAX, epi);
-      else
-        jac_conv_fwd_mfma<C, C * 9 / 4>(bA, theta + w1, nbr, N, NMAX, epi);
-    }
-    __syncthreads();
-    {
-      const float* bias = (b2 >= 0) ? theta + b2 : nullptr;
-      auto epi = [&](int co, int p, float v) {
-        if (bias) v += bias[co];
-        v += (cin == 1) ? bX[p] : bX[co * N + p];  // residual (block 0: the spin, broadcast)
-        bA[co * N + p] = v;
-      };
-      jac_conv_fwd_mfma<C, C * 9 / 4>(bB, theta + w2, nbr, N, NMAX, epi);
-    }
-    __syncthreads();
-    float* t = bX;
-    bX = bA;
-    bA = t;
-  }
-  // ---- head: dX = softmax(h) / sqrt(nb + 1), h = x / sqrt(nb + 1)
-  const float hs = rsqrtf((float)(nb + 1));
-  {
-    const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
-    float m = -INFINITY;
-    for (int e = threadIdx.x; e < C * N; e += JAC_THREADS) m = fmaxf(m, bX[e] * hs);
-    m = wave_max(m);
-    if (lane == 0) red[wv] = m;
-    __syncthreads();
-    m = -INFINITY;
-    for (int w = 0; w < JAC_THREADS / WAVE; ++w) m = fmaxf(m, red[w]);
-    float ssum = 0.0f;
-    for (int e = threadIdx.x; e < C * N; e += JAC_THREADS) ssum += expf(bX[e] * hs - m);
-    ssum = wave_sum(ssum);
-    __syncthreads();
-    if (lane == 0) red[wv] = ssum;
-    __syncthreads();
-    ssum = 0.0f;
-    for (int w = 0; w < JAC_THREADS / WAVE; ++w) ssum += red[w];
-    float inv = 1.0f / ssum;
-    for (int e = threadIdx.x; e < C * N; e += JAC_THREADS) bX[e] = expf(bX[e] * hs - m) * inv * hs;
-    __syncthreads();
-  }
-  // ---- backward
-  for (int i = nb - 1; i >= 0; --i) {
-    const int cin = (i == 0) ? 1 : C;
-    float* rx = rec + i * blk_f;
-    float* ry = rx + C * N;
-    float* rz = ry + C * N;
-    float* ra = rz + C * N;
-    int64_t w1, b1, w2, b2;
-    rc_theta_offsets(nb, C, 2 * i, w1, b1);
-    rc_theta_offsets(nb, C, 2 * i + 1, w2, b2);
-    // conv2: dz2 = dX; input a1
-    for (int e = threadIdx.x; e < C * N; e += JAC_THREADS) bA[e] = ra[e];
-    __syncthreads();
-    jac_conv_grad_w_mfma<C>(bX, bA, C, nbr, N, NMAX, Orow, w2, b2);
-    // da1 -> dz1 = da1 * act'(z1), into bB
-    jac_conv_bwd_in_mfma<C>(bX, theta + w2, nbr, N, NMAX, [&](int ci, int q, float v) {
-      bB[ci * N + q] = v * act_grad_f(rz[ci * N + q], actk);
-    });
-    __syncthreads();
-    // conv1: input y_i
-    for (int e = threadIdx.x; e < cin * N; e += JAC_THREADS) bA[e] = ry[e];
-    __syncthreads();
-    jac_conv_grad_w_mfma<C>(bB, bA, cin, nbr, N, NMAX, Orow, w1, b1);
-    __syncthreads();
-    if (i > 0) {
-      const float sc = rsqrtf((float)(i + 1));
-      jac_conv_bwd_in_mfma<C>(bB, theta + w1, nbr, N, NMAX, [&](int ci, int q, float v) {
-        const float xin = rx[ci * N + q] * sc;
-        bA[ci * N + q] = v * act_grad_f(xin, actk) * sc + bX[ci * N + q];
-      });
-      __syncthreads();
-      float* t = bX;
-      bX = bA;
-      bA = t;
-    }
-  }
-}
-
 }  // namespace qtx
 
 using namespace qtx;
 
 // ================================================================ C ABI
-static int rc_check(const qtx_resconv_desc* d) {
-  QTX_REQUIRE(d != nullptr, "null qtx_resconv_desc");
-  QTX_REQUIRE(d->channels == 16 || d->channels == 32, "channels must be 16 or 32");
-  QTX_REQUIRE(d->nblocks >= 1 && d->nblocks <= 64, "nblocks out of range (1..64)");
-  QTX_REQUIRE(d->L0 >= 1 && d->L1 >= 1 && d->L0 * d->L1 <= RC_MAXN, "L0 * L1 out of range (1..1024)");
-  QTX_REQUIRE(d->precision == QTX_CONV_FP32 || d->precision == QTX_CONV_BF16X3, "unknown precision");
-  QTX_REQUIRE(d->activation == QTX_ACT_GELU_TANH || d->activation == QTX_ACT_GELU_ERF ||
-                  d->activation == QTX_ACT_RELU,
-              "unknown activation");
-  if (d->channels == 16) QTX_REQUIRE(d->L0 * d->L1 <= 512, "channels = 16 needs L0 * L1 <= 512");
-  if (d->channels == 32) QTX_REQUIRE(d->L0 * d->L1 <= 400, "channels = 32 needs L0 * L1 <= 400");
-  return QTX_OK;
-}
-
 static RcArgs rc_args(const RcLayout& L, const void* packed) {
   RcArgs a;
   a.g = RcGeom{L.L0, L.L1, L.N, (L.N + 15) / 16, std::log((double)L.C * (double)L.N)};
@@ -2035,6 +1643,12 @@ int qtx_resconv_pack(void* stream, const qtx_resconv_desc* d, const float* theta
   int64_t misc = L.nparams + (int64_t)L.C * 10 + (int64_t)2 * L.nb * L.C;
   hipLaunchKernelGGL(rc_pack_misc_kernel, dim3((unsigned)((misc + 255) / 256)), dim3(256), 0, st, theta, L.nb, L.C,
                      L.nparams, (float*)packed, L.off_l0w, L.off_l0b, L.bias_off);
+  const int64_t jac = (int64_t)(2 * L.nb - 1) * 2 * L.C * L.C * 9;
+  float* jf = (float*)((char*)packed + L.off_jac);
+  if (L.C == 16)
+    hipLaunchKernelGGL(rc_pack_jac_kernel<16>, dim3((unsigned)((jac + 255) / 256)), dim3(256), 0, st, theta, L.nb, jf);
+  else
+    hipLaunchKernelGGL(rc_pack_jac_kernel<32>, dim3((unsigned)((jac + 255) / 256)), dim3(256), 0, st, theta, L.nb, jf);
   int ct = L.C / 16;
   int ks = (L.mode == QTX_CONV_FP32) ? 9 * L.C / 4 : (L.C == 16 ? (L.win ? 6 : 5) : 9);
   int64_t total = (int64_t)ct * ks * WAVE * (2 * L.nb - 1);
@@ -2161,100 +1775,6 @@ int qtx_resconv_eloc_ws(void* stream, const qtx_resconv_desc* d, const void* pac
 int qtx_resconv_eloc(void* stream, const qtx_resconv_desc* d, const void* packed, const qtx_ham* H,
                      const int8_t* s, const double* logabs, int64_t ns, double* eloc, int32_t* nconn) {
   return qtx_resconv_eloc_ws(stream, d, packed, H, s, logabs, ns, eloc, nconn, nullptr, 0);
-}
-
-static int64_t jac_chunk(int64_t ns) { return ns < 2048 ? ns : 2048; }
-
-size_t qtx_resconv_jacobian_ws_bytes(const qtx_resconv_desc* d, int64_t ns) {
-  if (rc_check(d) != QTX_OK || ns <= 0) return 0;
-  int64_t N = (int64_t)d->L0 * d->L1;
-  return (size_t)(jac_chunk(ns) * (int64_t)d->nblocks * 4 * d->channels * N * 4);
-}
-
-int qtx_resconv_jacobian(void* stream, const qtx_resconv_desc* d, const void* packed, const int8_t* s, int64_t ns,
-                         float* O, void* ws, size_t ws_bytes) {
-  int rc = rc_check(d);
-  if (rc) return rc;
-  QTX_REQUIRE(packed && ns >= 0 && (ns == 0 || (s && O)), "bad arguments");
-  if (ns == 0) return QTX_OK;
-  size_t need = qtx_resconv_jacobian_ws_bytes(d, ns);
-  if (ws == nullptr || ws_bytes < need)
-    return fail(QTX_EWORKSPACE, "workspace too small: need " + std::to_string(need) + " bytes");
-  RcLayout L = rc_layout(d);
-  RcGeom g{L.L0, L.L1, L.N, (L.N + 15) / 16, std::log((double)L.C * (double)L.N)};
-  hipStream_t st = as_stream(stream);
-  const float* theta = (const float*)packed;  // raw theta copy at offset 0
-  int64_t chunk = jac_chunk(ns);
-  for (int64_t s0 = 0; s0 < ns; s0 += chunk) {
-    int64_t nc = (ns - s0) < chunk ? (ns - s0) : chunk;
-    if (L.C == 16 && L.N <= 256)
-      hipLaunchKernelGGL((rc_jacobian_kernel<16, 256>), dim3((unsigned)nc), dim3(JAC_THREADS), 0, st, g, L.nb,
-                         L.actk, theta, s, s0, nc, L.nparams, O, (float*)ws);
-    else if (L.C == 16)
-      hipLaunchKernelGGL((rc_jacobian_kernel<16, 512>), dim3((unsigned)nc), dim3(JAC_THREADS), 0, st, g, L.nb,
-                         L.actk, theta, s, s0, nc, L.nparams, O, (float*)ws);
-    else
-      hipLaunchKernelGGL((rc_jacobian_kernel<32, 400>), dim3((unsigned)nc), dim3(JAC_THREADS), 0, st, g, L.nb,
-                         L.actk, theta, s, s0, nc, L.nparams, O, (float*)ws);
-    QTX_LAUNCH_CHECK();
-  }
-  return QTX_OK;
-}
-
-// ---------------------------------------------------------------- allocation-free Jacobian
-// The per-sample forward records of qtx_resconv_jacobian_noalloc live in this
-// file-scope device array (one copy per GPU, held until the process ends)
-// instead of a caller workspace; samples run in launches of as many as the
-// array holds.  Host code uses the per-device address from
-// hipGetSymbolAddress, never the array's name (a host-side stand-in).
-constexpr size_t RC_JAC_SCRATCH_BYTES = (size_t)128 << 20;
-static __device__ __align__(256) char scratch[RC_JAC_SCRATCH_BYTES];
-
-namespace {
-constexpr int RC_MAX_DEVICES = 64;
-std::mutex g_scratch_mu;
-void* g_scratch_ptr[RC_MAX_DEVICES] = {};
-
-// the calling thread's current device's copy of scratch
-int jac_scratch(void** out) {
-  int dev = 0;
-  QTX_HIP(hipGetDevice(&dev));
-  QTX_REQUIRE(dev >= 0 && dev < RC_MAX_DEVICES, "device index out of range");
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (g_scratch_ptr[dev] == nullptr) {
-    void* p = nullptr;
-    QTX_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-    QTX_REQUIRE(p != nullptr, "hipGetSymbolAddress returned no address for the Jacobian scratch");
-    g_scratch_ptr[dev] = p;
-  }
-  *out = g_scratch_ptr[dev];
-  return QTX_OK;
-}
-}  // namespace
-
-int qtx_resconv_jacobian_noalloc(void* stream, const qtx_resconv_desc* d, const void* packed, const int8_t* s,
-                                 int64_t ns, float* O) {
-  int rc = rc_check(d);
-  if (rc) return rc;
-  QTX_REQUIRE(packed && ns >= 0 && (ns == 0 || (s && O)), "bad arguments");
-  void* ws = nullptr;
-  rc = jac_scratch(&ws);
-  if (rc) return rc;
-  if (ns == 0) return QTX_OK;
-  const size_t per_sample = qtx_resconv_jacobian_ws_bytes(d, 1);
-  if (per_sample > RC_JAC_SCRATCH_BYTES)
-    return fail(QTX_EINVAL, "one sample's Jacobian records need " + std::to_string(per_sample) +
-                                " bytes, more than the " + std::to_string(RC_JAC_SCRATCH_BYTES) +
-                                "-byte scratch of the allocation-free entry point");
-  const int64_t per_launch = (int64_t)(RC_JAC_SCRATCH_BYTES / per_sample);
-  for (int64_t s0 = 0; s0 < ns; s0 += per_launch) {
-    const int64_t nc = (ns - s0) < per_launch ? (ns - s0) : per_launch;
-    // the kernel indexes samples from the start of the pointers it is given
-    rc = qtx_resconv_jacobian(stream, d, packed, s + s0 * (int64_t)d->L0 * d->L1, nc,
-                              O + s0 * qtx_resconv_nparams(d), ws, per_launch * per_sample);
-    if (rc) return rc;
-  }
-  return QTX_OK;
 }
 
 }  // extern "C"
