@@ -142,6 +142,18 @@ __global__ __launch_bounds__(JAC_THREADS, WPS) void rc_jacobian_kernel(RcGeom g,
     // the swizzle key of site 16 t + l16 depends on l16 alone
     if (site(k) < N) *reinterpret_cast<v4f*>(buf + (wv + 4 * k) * (16 * C * 4) + put_off[ct]) = v;
   };
+  // Wait out the last MFMA of acc: the compiler counts the wait states from an
+  // MFMA to the first read of its result along the fall-through path only, so
+  // a short branch over a block that rewrites the same registers (an optional
+  // bias) read element 3 three instructions after the MFMA instead of ten.
+  // The asm statements keep their order, and each use of acc follows its own.
+  auto settle = [&](v4f (&acc)[MAXT][CT]) {
+    asm volatile("s_nop 15" : "+v"(acc[0][0]));
+#pragma unroll
+    for (int k = 0; k < MAXT; ++k)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) asm volatile("" : "+v"(acc[k][ct]));
+  };
   // acc[k][ct] += the 3 x 3 convolution of the positions in buf with layer l's fragments
   auto conv = [&](const char* buf, int l, int dir, v4f (&acc)[MAXT][CT]) {
     const v4f* fr = reinterpret_cast<const v4f*>(jf + ((int64_t)l * 2 + dir) * per) + lane;
@@ -172,9 +184,8 @@ __global__ __launch_bounds__(JAC_THREADS, WPS) void rc_jacobian_kernel(RcGeom g,
           }
         }
       }
-      // 32 channels, four tiles: one tap's operands live at a time (else 22 spills)
-      if constexpr (CT == 2 && MAXT == 4) __builtin_amdgcn_sched_barrier(0);
     }
+    settle(acc);
   };
   auto zero = [&](v4f (&acc)[MAXT][CT]) {
 #pragma unroll
