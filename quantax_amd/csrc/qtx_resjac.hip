@@ -207,8 +207,7 @@ __global__ __launch_bounds__(JAC_THREADS, WPS) void rc_jacobian_kernel(RcGeom g,
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float v = t[i];
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
+        v = row_sum(v);
         if (l16 == 0) sred[wv * C + 16 * ct + 4 * gq + i] = v;
       }
     }
