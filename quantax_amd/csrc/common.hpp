@@ -78,9 +78,27 @@ __device__ __forceinline__ T wave_sum(T v) {
   return wave_butterfly(v, [](T a, T b) { return a + b; });
 }
 
+// wave_sum(a * b) with the first step fused, a b + (a b of lane ^ 32): what the
+// product form of the butterfly rounds to under FP contraction
+__device__ __forceinline__ float wave_sum_prod(float a, float b) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, a * b);
+  const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const uint32_t other = (threadIdx.x % WAVE) < 32 ? (uint32_t)h[1] : (uint32_t)h[0];
+  uint32_t v = __builtin_bit_cast(uint32_t, fmaf(a, b, __builtin_bit_cast(float, other)));
+  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return row_sum(__builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_max(T v) {
   return wave_butterfly(v, [](T a, T b) { return (T)fmax(a, b); });
+}
+
+// Orders this wave's LDS writes before its later LDS reads (other lanes' data)
+// for the compiler; the hardware runs a wave's LDS instructions in order.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
 // ---------------------------------------------------------------- math

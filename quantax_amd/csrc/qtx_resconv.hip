@@ -962,7 +962,7 @@ __device__ __attribute__((always_inline)) inline void rc_forward_win(
       m_l = mn;
     });
     const float m_w = wave_max(m_l);
-    const float s_w = wave_sum(s_l * __expf(m_l - m_w));
+    const float s_w = wave_sum_prod(s_l, __expf(m_l - m_w));
     if (lane == 0) {
       red[wv * 2] = m_w;
       red[wv * 2 + 1] = s_w;
