@@ -1302,6 +1302,8 @@ __global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS =
   __shared__ double lp_cur[B];
   __shared__ int mv_a[B], mv_b[B], mv_upd[B], nhop[B], nacc[B], nnear[B];
   __shared__ double mv_thr[B];
+  __shared__ uint2 wq[B][WAVE];   // proposal words of 64 steps
+  __shared__ double tq[B][WAVE];  // and their acceptance thresholds
   const int N = a.g.N;
   const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
   const int64_t c0 = xcd_block(blockIdx.x, gridDim.x) * B;  // per-chain Philox words of a step share lines
@@ -1324,35 +1326,40 @@ __global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS =
     if (lane == 0) nhop[b] = cnt;
   }
   __syncthreads();
-  // with at least two waves per chain, the FP64 acceptance threshold of
-  // chain b is computed by wave B + b while wave b draws the move
-  constexpr bool kThrWave = (2 * B <= W);
   static_assert(W >= B, "one wave per chain at most");
-  // the step's Philox words are fetched one step ahead (their HBM latency
-  // hidden by the forward): waves 0 .. B - 1 draw chain wv's move, waves
-  // B .. 2 B - 1 its acceptance threshold
-  const int cbw = (wv < B) ? wv : ((kThrWave && wv < 2 * B) ? wv - B : -1);
-  const int64_t cw = c0 + cbw;
-  const bool wok = cbw >= 0 && cw < ns;
-  uint4 wn = make_uint4(0u, 0u, 0u, 0u);
-  if (wok && nsteps > 0) wn = reinterpret_cast<const uint4*>(words)[cw];
-  for (int t = 0; t < nsteps; ++t) {
-    const uint4 wcur = wn;
-    if (wok && t + 1 < nsteps) wn = reinterpret_cast<const uint4*>(words)[(int64_t)(t + 1) * ns + cw];
+  // A proposal that leaves the spins unchanged (an exchange of equal spins: a
+  // third to a half of them at Sz = 0) is never accepted, so its forward is
+  // not run: wave b < B draws chain b's moves until one changes the spins, and
+  // the chains of a workgroup may be at different steps.  The Philox words of
+  // 64 steps are fetched at once, lane l step t0 + l, and each lane evaluates
+  // its step's FP64 threshold.  512 steps of 4096 chains, 16 x 16, 8 blocks:
+  // 104.6 -> 57.3 ms.
+  int tc = 0;  // next step of the wave's chain
+  for (;;) {
     // the lane index through an opaque move, as in the forwards: the step's
     // per-lane LDS addresses are formed here, not held across the loop
     int lane = threadIdx.x % WAVE;
     asm volatile("" : "+v"(lane));
-    // proposals: one wave per chain
-    for (int b = wv; b < B; b += W) {
-      int64_t c = c0 + b;
+    if (wv < B) {
+      const int b = wv;
+      const int64_t c = c0 + b;
       int fa = -1, fb = -1;
       bool upd = false;
       double thr = 0.0;
-      if (c < ns) {
-        const uint4 w = wcur;
+      while (c < ns && tc < nsteps && !upd) {
+        const int q = tc % WAVE;
+        if (q == 0) {
+          if (tc + lane < nsteps) {
+            const uint4 w = reinterpret_cast<const uint4*>(words)[(int64_t)(tc + lane) * ns + c];
+            wq[b][lane] = make_uint2(w.x, w.y);
+            tq[b][lane] = accept_threshold(w.z, w.w);
+          }
+          wave_lds_fence();
+        }
+        const uint2 w = wq[b][q];
         propose_move(kind, cur + b * N, N, nbr, width, hopping, nhop[b], w.x, w.y, lane, fa, fb, upd);
-        if constexpr (!kThrWave) thr = accept_threshold(w.z, w.w);
+        thr = tq[b][q];
+        ++tc;
       }
       for (int i = lane; i < N; i += WAVE) {
         int8_t v = cur[b * N + i];
@@ -1363,19 +1370,14 @@ __global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS =
         mv_a[b] = fa;
         mv_b[b] = fb;
         mv_upd[b] = upd ? 1 : 0;
-        if constexpr (!kThrWave) mv_thr[b] = thr;
-      }
-    }
-    if constexpr (kThrWave) {
-      if (wv >= B && wv < 2 * B) {
-        const int b = wv - B;
-        const int64_t c = c0 + b;
-        double thr = 0.0;
-        if (c < ns) thr = accept_threshold(wcur.z, wcur.w);
-        if (lane == 0) mv_thr[b] = thr;
+        mv_thr[b] = thr;
       }
     }
     __syncthreads();
+    int any = 0;
+#pragma unroll
+    for (int b = 0; b < B; ++b) any |= mv_upd[b];
+    if (!any) break;  // every chain has run its steps
     RC_FWD(prop, lp_new);
     // accept / reject (rc_forward ends with a barrier)
     for (int b = wv; b < B; b += W) {
