@@ -3,15 +3,14 @@
 // with one full forward per proposal and local energy over connected
 // configurations generated in LDS.
 //
-// Forward work unit ("item") = one 16-position tile of one configuration.
-// Convolution as an implicit GEMM per item: D[co, p] = sum_k W[co, k] X[k, p]
-// with k = (tap, ci); A = weights (rows = output channels, register
-// resident per layer), B = activations read from LDS at the tap-shifted
-// position.  The residual stream stays in registers in the MFMA output
-// layout (lane l: channel 16 ct + 4 (l / 16) + q, position 16 t + l % 16).
+// The 16 x 16 window kernels and the large 32-channel split-bf16 ones are here,
+// every other shape in resconv_wave.hpp.  The residual stream stays in
+// registers in the MFMA output layout (lane l: channel 16 ct + 4 (l / 16) + q,
+// site 16 t + l % 16).
 //
-// LDS activations: per configuration, per position, C/4 chunks of 16 bytes,
-// XOR-swizzled so 16 consecutive positions hit distinct banks.
+// LDS activations: per configuration, per site, C/4 chunks of 16 bytes,
+// XOR-swizzled so the eight lanes a ds_read_b128 serves at a time (eight
+// consecutive sites) hit distinct 16-byte bank groups.
 //   FP32   : chunk j = channels 4j .. 4j+3 (float)
 //   BF16X3 : chunk j < C/8 = hi(channels 8j .. 8j+7), chunk C/8 + j = lo(...)
 #include <hip/hip_runtime.h>
@@ -21,7 +20,7 @@
 #include <string>
 #include <type_traits>
 
-#include "resconv.hpp"
+#include "resconv_wave.hpp"
 
 namespace qtx {
 
@@ -30,9 +29,8 @@ namespace qtx {
 template <int C, int MODE, int WIN>
 __global__ void rc_pack_frag_kernel(const float* __restrict__ theta, int nb, char* __restrict__ packed,
                                     int64_t off_frag, int64_t frag_bytes) {
-  using K0 = RcK<C, MODE>;
-  constexpr int KCT = K0::CT;
-  constexpr int KKS = (WIN && MODE == QTX_CONV_BF16X3) ? 6 : K0::KS;
+  constexpr int KCT = C / 16;
+  constexpr int KKS = (MODE == QTX_CONV_FP32) ? 9 * C / 4 : (C == 16 ? (WIN ? 6 : 5) : 9);
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int64_t per_layer = (int64_t)KCT * KKS * WAVE;
   int64_t total = per_layer * (2 * nb - 1);
@@ -121,8 +119,7 @@ __global__ void rc_pack_jac_kernel(const float* __restrict__ theta, int nb, floa
   const int e = (int)(idx % per);
   const int j = e % 4, lane = (e / 4) % WAVE, h = (e / 256) % CT, ct = (e / 256 / CT) % CT, tap = e / 256 / CT / CT;
   const int row = 16 * ct + lane % 16, col = 16 * h + 4 * (lane / 16) + j;
-  int64_t w0, b0;
-  rc_theta_offsets(nb, C, l, w0, b0);
+  const int64_t w0 = 10 * C + (int64_t)(l - 1) * (per + C);  // layer l >= 1 of rc_theta_offsets
   dst[((int64_t)l * 2 + dir) * per + e] =
       dir == 0 ? theta[w0 + ((int64_t)row * C + col) * 9 + tap] : theta[w0 + ((int64_t)col * C + row) * 9 + (8 - tap)];
 }
@@ -144,506 +141,7 @@ __global__ void rc_pack_misc_kernel(const float* __restrict__ theta, int nb, int
   }
 }
 
-// v = hi + lo + O(2^-16 |v|): hi = bf16(v) (round to nearest even), lo =
-// bf16(v - hi).  v - hi is formed by v_dot2c_f32_bf16 from the packed hi
-// pair, (hi0, hi1) . (-1, 0) + v0 and (hi0, hi1) . (0, -1) + v1, exact
-// (bf16 products are exact in FP32 and v - hi is representable), so hi is
-// never widened back to FP32 by bit moves.
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void split_bf16x4(v4f v, v4bf& hi, v4bf& lo) {
-  const v2bf h01 = {(__bf16)v[0], (__bf16)v[1]}, h23 = {(__bf16)v[2], (__bf16)v[3]};
-  // the selectors come from registers: an inline constant here (the
-  // compiler encodes e0 as "-1.0") is not read as (bf16 -1, 0) by the hardware
-  uint32_t u0 = 0x0000bf80u, u1 = 0xbf800000u;
-  asm("" : "+v"(u0), "+v"(u1));
-  const v2bf e0 = __builtin_bit_cast(v2bf, u0), e1 = __builtin_bit_cast(v2bf, u1);
-  const float l0 = __builtin_amdgcn_fdot2_f32_bf16(h01, e0, v[0], false);
-  const float l1 = __builtin_amdgcn_fdot2_f32_bf16(h01, e1, v[1], false);
-  const float l2 = __builtin_amdgcn_fdot2_f32_bf16(h23, e0, v[2], false);
-  const float l3 = __builtin_amdgcn_fdot2_f32_bf16(h23, e1, v[3], false);
-  const v2bf l01 = {(__bf16)l0, (__bf16)l1}, l23 = {(__bf16)l2, (__bf16)l3};
-  hi = v4bf{h01[0], h01[1], h23[0], h23[1]};
-  lo = v4bf{l01[0], l01[1], l23[0], l23[1]};
-}
-
-// ---------------------------------------------------------------- forward core
-template <int C>
-__device__ __forceinline__ int swz_chunk(int p, int j) {
-  // a ds_read_b128 is served eight lanes (128 bytes, 32 banks) at a time and
-  // the eight lanes read eight consecutive sites: the key makes their chunks
-  // fall on distinct 16-byte bank groups
-  constexpr int CH = C / 4;
-  return j ^ ((p / (8 / CH)) & (CH - 1));
-}
-
-// Write 4 consecutive channels (c4 .. c4+3, c4 % 4 == 0) of position p.
-template <int C, int MODE>
-__device__ __forceinline__ void act_store4(char* act_cfg, int p, int c4, v4f v) {
-  constexpr int CH = C / 4;
-  if constexpr (MODE == QTX_CONV_FP32) {
-    int j = c4 / 4;
-    *reinterpret_cast<v4f*>(act_cfg + ((int64_t)p * CH + swz_chunk<C>(p, j)) * 16) = v;
-  } else {
-    v4bf hi, lo;
-    split_bf16x4(v, hi, lo);
-    int j = c4 / 8, half = (c4 % 8) / 4;
-    char* base = act_cfg + (int64_t)p * CH * 16;
-    *reinterpret_cast<v4bf*>(base + swz_chunk<C>(p, j) * 16 + half * 8) = hi;
-    *reinterpret_cast<v4bf*>(base + swz_chunk<C>(p, C / 8 + j) * 16 + half * 8) = lo;
-  }
-}
-
-// Accumulate one conv layer (C -> C) for one item into acc[CT].
-template <int C, int MODE>
-__device__ __forceinline__ void conv_item(const char* act_cfg, const RcGeom& g, int p, int y, int x, int lane,
-                                          const float* wf, const v8bf* wh, const v8bf* wl, v4f* acc) {
-  using K = RcK<C, MODE>;
-  constexpr int CH = K::CH;
-  const int gq = lane / 16;
-  if constexpr (MODE == QTX_CONV_FP32) {
-#pragma unroll
-    for (int tap = 0; tap < 9; ++tap) {
-      int ps = tap_pos(g, y, x, tap);
-      const char* base = act_cfg + (int64_t)ps * CH * 16;
-#pragma unroll
-      for (int h = 0; h < C / 16; ++h) {
-        int j = 4 * h + gq;
-        v4f bv = *reinterpret_cast<const v4f*>(base + swz_chunk<C>(ps, j) * 16);
-#pragma unroll
-        for (int jp = 0; jp < 4; ++jp) {
-          int ks = tap * (C / 4) + 4 * h + jp;
-#pragma unroll
-          for (int ct = 0; ct < K::CT; ++ct)
-            acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[ct * K::KS + ks], bv[jp], acc[ct], 0, 0, 0);
-        }
-      }
-    }
-  } else {
-#pragma unroll
-    for (int ks = 0; ks < K::KS; ++ks) {
-      int tap, c0;
-      if (C == 16) {
-        tap = 2 * ks + (gq >> 1);
-        c0 = 8 * (gq & 1);
-      } else {
-        tap = ks;
-        c0 = 8 * gq;
-      }
-      int ps = (tap < 9) ? tap_pos(g, y, x, tap) : p;
-      const char* base = act_cfg + (int64_t)ps * CH * 16;
-      int jh = c0 / 8;
-      v8bf bh = *reinterpret_cast<const v8bf*>(base + swz_chunk<C>(ps, jh) * 16);
-      v8bf bl = *reinterpret_cast<const v8bf*>(base + swz_chunk<C>(ps, C / 8 + jh) * 16);
-#pragma unroll
-      for (int ct = 0; ct < K::CT; ++ct) {
-        acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wl[ct * K::KS + ks], bh, acc[ct], 0, 0, 0);
-        acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wh[ct * K::KS + ks], bl, acc[ct], 0, 0, 0);
-        acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wh[ct * K::KS + ks], bh, acc[ct], 0, 0, 0);
-      }
-    }
-  }
-}
-
-// Forward of B configurations whose spins are in sp[b * N + i] (LDS int8).
-// Result: lp_out[b] (LDS double).  All threads of the block must call it.
-// act: two LDS activation buffers of B * N * C * 4 bytes each (ping-pong: a
-// layer reads one and writes the other, so one barrier per layer suffices).
-// red: >= 2 * B * W floats.  Items of wave w: w + W * k, k < MAXT.
-template <int C, int MODE, int B, int MAXT, int W>
-__device__ __attribute__((always_inline)) inline void rc_forward(const RcGeom& g, int nb, int actk, const char* __restrict__ packed,
-                           int64_t off_l0w, int64_t off_l0b, int64_t bias_off, int64_t off_frag, int64_t frag_bytes,
-                           const int8_t* sp, char* act, float* red, double* lp_out) {
-  using K = RcK<C, MODE>;
-  constexpr int CT = K::CT;
-  int tid = threadIdx.x;
-  asm volatile("" : "+v"(tid));  // per-lane addresses formed inside the forward
-  const int lane = tid % WAVE, wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  const int gq = lane / 16;
-  const int nitems = B * g.NT;
-  const int64_t act_cfg_bytes = (int64_t)g.N * C * 4;
-  const int64_t buf_bytes = act_cfg_bytes * B;
-  const float* pf = reinterpret_cast<const float*>(packed);
-
-  v4f res[MAXT][CT];
-
-  // ---- layer 0: conv (Cin = 1) of s / sqrt(2) on VALU, GELU, into buffer 0
-  {
-    const float* W0 = pf + off_l0w;
-    const float* b0 = pf + off_l0b;
-#pragma unroll
-    for (int k = 0; k < MAXT; ++k) {
-      int it = wv + W * k;
-      if (it < nitems) {
-        int b = it / g.NT, t = it % g.NT;
-        int p = 16 * t + lane % 16;
-        bool pv = p < g.N;
-        int pc = pv ? p : 0;
-        int y = pc / g.L1, x = pc % g.L1;
-        const int8_t* s = sp + b * g.N;
-        float sv[9];
-#pragma unroll
-        for (int tap = 0; tap < 9; ++tap) sv[tap] = (float)s[tap_pos(g, y, x, tap)] * 0.70710678118654752f;
-        float spin = (float)s[pc];
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-          v4f z;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            int co = 16 * ct + 4 * gq + q;
-            float a = b0[co];
-#pragma unroll
-            for (int tap = 0; tap < 9; ++tap) a += W0[co * 9 + tap] * sv[tap];
-            z[q] = act_f(a, actk);
-          }
-          res[k][ct] = v4f{spin, spin, spin, spin};
-          if (pv) act_store4<C, MODE>(act + b * act_cfg_bytes, p, 16 * ct + 4 * gq, z);
-        }
-      }
-    }
-  }
-  __syncthreads();
-
-  // ---- layers 1 .. 2nb-1 on MFMA
-  int cur = 0;
-  for (int l = 1; l < 2 * nb; ++l) {
-    float wf[(MODE == QTX_CONV_FP32) ? CT * K::KS : 1];
-    v8bf wh[(MODE == QTX_CONV_FP32) ? 1 : CT * K::KS];
-    v8bf wl[(MODE == QTX_CONV_FP32) ? 1 : CT * K::KS];
-    const char* fr = packed + off_frag + (int64_t)l * frag_bytes;
-    if constexpr (MODE == QTX_CONV_FP32) {
-#pragma unroll
-      for (int i = 0; i < CT * K::KS; ++i) wf[i] = reinterpret_cast<const float*>(fr)[i * WAVE + lane];
-    } else {
-#pragma unroll
-      for (int i = 0; i < CT * K::KS; ++i) {
-        const v8bf* src = reinterpret_cast<const v8bf*>(fr) + ((int64_t)i * WAVE + lane) * 2;
-        wh[i] = src[0];
-        wl[i] = src[1];
-      }
-    }
-    const float* bias = pf + bias_off + (int64_t)l * C;
-    const char* in = act + cur * buf_bytes;
-    char* out = act + (cur ^ 1) * buf_bytes;
-    const bool is_conv2 = (l % 2) == 1;
-    const int blk = l / 2;
-    const bool last = (l == 2 * nb - 1);
-    const float scale = last ? rsqrtf((float)(nb + 1)) : (is_conv2 ? rsqrtf((float)(blk + 2)) : 1.0f);
-    float m_b[B], s_b[B];
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-      m_b[b] = -INFINITY;
-      s_b[b] = 0.0f;
-    }
-#pragma unroll
-    for (int k = 0; k < MAXT; ++k) {
-      int it = wv + W * k;
-      if (it < nitems) {
-        int b = it / g.NT, t = it % g.NT;
-        int p = 16 * t + lane % 16;
-        int pc = p < g.N ? p : 0;
-        int y = pc / g.L1, x = pc % g.L1;
-        v4f acc[CT];
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-          int cb = 16 * ct + 4 * gq;
-          acc[ct] = v4f{bias[cb], bias[cb + 1], bias[cb + 2], bias[cb + 3]};
-        }
-        conv_item<C, MODE>(in + b * act_cfg_bytes, g, pc, y, x, lane, wf, wh, wl, acc);
-        if (!last) {
-#pragma unroll
-          for (int ct = 0; ct < CT; ++ct) {
-            v4f o;
-            if (is_conv2) {
-              v4f xr = acc[ct] + res[k][ct];
-              res[k][ct] = xr;
-#pragma unroll
-              for (int q = 0; q < 4; ++q) o[q] = act_f(xr[q] * scale, actk);
-            } else {
-#pragma unroll
-              for (int q = 0; q < 4; ++q) o[q] = act_f(acc[ct][q], actk);
-            }
-            if (p < g.N) act_store4<C, MODE>(out + b * act_cfg_bytes, p, 16 * ct + 4 * gq, o);
-          }
-        } else {
-          // head: h = (z2 + r) / sqrt(nb + 1); running logsumexp per configuration
-          float m = -INFINITY;
-          float hv[CT * 4];
-#pragma unroll
-          for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              float h = (acc[ct][q] + res[k][ct][q]) * scale;
-              hv[ct * 4 + q] = h;
-              if (p < g.N) m = fmaxf(m, h);
-            }
-          m = wave_max(m);
-          float sacc = 0.0f;
-          if (p < g.N) {
-#pragma unroll
-            for (int i = 0; i < CT * 4; ++i) sacc += __expf(hv[i] - m);
-          }
-          sacc = wave_sum(sacc);
-#pragma unroll
-          for (int bb = 0; bb < B; ++bb) {
-            if (bb == b) {
-              float mm = fmaxf(m_b[bb], m);
-              s_b[bb] = s_b[bb] * __expf(m_b[bb] - mm) + sacc * __expf(m - mm);
-              m_b[bb] = mm;
-            }
-          }
-        }
-      }
-    }
-    if (!last) {
-      __syncthreads();
-      cur ^= 1;
-    } else {
-      if (lane == 0) {
-#pragma unroll
-        for (int b = 0; b < B; ++b) {
-          red[(b * W + wv) * 2] = m_b[b];
-          red[(b * W + wv) * 2 + 1] = s_b[b];
-        }
-      }
-      __syncthreads();
-      if (threadIdx.x < B) {
-        // waves' (max, sum) merged in FP32 (the sums are FP32 already): FP64
-        // exp / log here would hold the workgroup at the barrier below
-        int b = threadIdx.x;
-        float m = -INFINITY;
-        for (int w = 0; w < W; ++w) m = fmaxf(m, red[(b * W + w) * 2]);
-        float ssum = 0.0f;
-        for (int w = 0; w < W; ++w) {
-          const float mw = red[(b * W + w) * 2];
-          if (mw > -INFINITY) ssum += red[(b * W + w) * 2 + 1] * __expf(mw - m);
-        }
-        lp_out[b] = (double)m + (double)logf(ssum) - g.log_cn;
-      }
-      __syncthreads();
-    }
-  }
-}
-
-}  // namespace qtx
-
-namespace qtx {
-
-// Row-tile forward for C = 16 on L0 x 16 grids (L0 <= 16): an item is one
-// lattice row of one configuration, so the 16 lanes of a fragment are the 16
-// columns and every tap address is a wave-uniform row offset plus a per-lane
-// column constant computed once.  Same LDS layout and results as rc_forward.
-template <int MODE, int B, int MAXT, int W>
-__device__ __attribute__((always_inline)) inline void rc_forward_rows(const RcGeom& g, int nb, int actk, const char* __restrict__ packed,
-                                int64_t off_l0w, int64_t off_l0b, int64_t bias_off, int64_t off_frag,
-                                int64_t frag_bytes, const int8_t* sp, char* act, float* red, double* lp_out) {
-  constexpr int C = 16;
-  using K = RcK<C, MODE>;
-  constexpr int ROWB = 16 * 64;  // bytes of one lattice row (16 positions x 16 channels x 4 B)
-  const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
-  const int gq = lane / 16, x = lane % 16;
-  const int L0 = g.L0;
-  const int nitems = B * L0;
-  const int cfg_bytes = L0 * ROWB;
-  const int buf_bytes = cfg_bytes * B;
-  const float* pf = reinterpret_cast<const float*>(packed);
-
-  // per-lane column constants (swizzle key of column c is (c >> 1) & 3)
-  int xoff[3];
-#pragma unroll
-  for (int dx = 0; dx < 3; ++dx) {
-    int xs = (x + dx + 15) & 15;
-    xoff[dx] = xs * 64 + ((gq ^ ((xs >> 1) & 3)) << 4);
-  }
-  int kdy[5], khi[5], klo[5];
-#pragma unroll
-  for (int ks = 0; ks < 5; ++ks) {
-    int tap = 2 * ks + (gq >> 1);
-    bool valid = tap < 9;
-    int dy = valid ? tap / 3 : 1, dx = valid ? tap % 3 : 1;
-    int xs = (x + dx + 15) & 15, key = (xs >> 1) & 3, jh = gq & 1;
-    kdy[ks] = dy;
-    khi[ks] = xs * 64 + ((jh ^ key) << 4);
-    klo[ks] = xs * 64 + (((2 + jh) ^ key) << 4);
-  }
-  const int key0 = (x >> 1) & 3;
-  const int st_f32 = x * 64 + ((gq ^ key0) << 4);
-  const int st_hi = x * 64 + (((gq >> 1) ^ key0) << 4) + (gq & 1) * 8;
-  const int st_lo = x * 64 + (((2 + (gq >> 1)) ^ key0) << 4) + (gq & 1) * 8;
-
-  auto store4 = [&](char* row_base, v4f v) {
-    if constexpr (MODE == QTX_CONV_FP32) {
-      *reinterpret_cast<v4f*>(row_base + st_f32) = v;
-    } else {
-      v4bf hi, lo;
-      split_bf16x4(v, hi, lo);
-      *reinterpret_cast<v4bf*>(row_base + st_hi) = hi;
-      *reinterpret_cast<v4bf*>(row_base + st_lo) = lo;
-    }
-  };
-  auto wrap = [&](int r) { return r < 0 ? r + L0 : (r >= L0 ? r - L0 : r); };
-
-  v4f res[MAXT];
-
-  // ---- layer 0: conv (Cin = 1) of s / sqrt(2) on VALU, GELU, into buffer 0
-  {
-    const float* W0 = pf + off_l0w;
-    const float* b0 = pf + off_l0b;
-#pragma unroll
-    for (int k = 0; k < MAXT; ++k) {
-      int it = wv + W * k;
-      if (it < nitems) {
-        int b = it / L0, y = it % L0;
-        const int8_t* s = sp + b * 16 * L0;
-        float sv[9];
-#pragma unroll
-        for (int tap = 0; tap < 9; ++tap)
-          sv[tap] = (float)s[wrap(y + tap / 3 - 1) * 16 + ((x + tap % 3 + 15) & 15)] * 0.70710678118654752f;
-        float spin = (float)s[y * 16 + x];
-        v4f z;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          int co = 4 * gq + q;
-          float a = b0[co];
-#pragma unroll
-          for (int tap = 0; tap < 9; ++tap) a += W0[co * 9 + tap] * sv[tap];
-          z[q] = act_f(a, actk);
-        }
-        res[k] = v4f{spin, spin, spin, spin};
-        store4(act + b * cfg_bytes + y * ROWB, z);
-      }
-    }
-  }
-  __syncthreads();
-
-  int cur = 0;
-  for (int l = 1; l < 2 * nb; ++l) {
-    float wf[(MODE == QTX_CONV_FP32) ? K::KS : 1];
-    v8bf wh[(MODE == QTX_CONV_FP32) ? 1 : K::KS];
-    v8bf wl[(MODE == QTX_CONV_FP32) ? 1 : K::KS];
-    const char* fr = packed + off_frag + (int64_t)l * frag_bytes;
-    if constexpr (MODE == QTX_CONV_FP32) {
-#pragma unroll
-      for (int i = 0; i < K::KS; ++i) wf[i] = reinterpret_cast<const float*>(fr)[i * WAVE + lane];
-    } else {
-#pragma unroll
-      for (int i = 0; i < K::KS; ++i) {
-        const v8bf* src = reinterpret_cast<const v8bf*>(fr) + ((int64_t)i * WAVE + lane) * 2;
-        wh[i] = src[0];
-        wl[i] = src[1];
-      }
-    }
-    const float* bias = pf + bias_off + (int64_t)l * C;
-    const v4f bias4 = v4f{bias[4 * gq], bias[4 * gq + 1], bias[4 * gq + 2], bias[4 * gq + 3]};
-    const char* in = act + cur * buf_bytes;
-    char* out = act + (cur ^ 1) * buf_bytes;
-    const bool is_conv2 = (l % 2) == 1;
-    const int blk = l / 2;
-    const bool last = (l == 2 * nb - 1);
-    const float scale = last ? rsqrtf((float)(nb + 1)) : (is_conv2 ? rsqrtf((float)(blk + 2)) : 1.0f);
-    float m_b[B], s_b[B];
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-      m_b[b] = -INFINITY;
-      s_b[b] = 0.0f;
-    }
-#pragma unroll
-    for (int k = 0; k < MAXT; ++k) {
-      int it = wv + W * k;
-      if (it < nitems) {
-        int b = it / L0, y = it % L0;
-        const char* base = in + b * cfg_bytes;
-        v4f acc = bias4;
-        if constexpr (MODE == QTX_CONV_FP32) {
-#pragma unroll
-          for (int dy = 0; dy < 3; ++dy) {
-            const char* rb = base + wrap(y + dy - 1) * ROWB;
-#pragma unroll
-            for (int dx = 0; dx < 3; ++dx) {
-              v4f bv = *reinterpret_cast<const v4f*>(rb + xoff[dx]);
-              const int tap = 3 * dy + dx;
-#pragma unroll
-              for (int jp = 0; jp < 4; ++jp)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[tap * 4 + jp], bv[jp], acc, 0, 0, 0);
-            }
-          }
-        } else {
-#pragma unroll
-          for (int ks = 0; ks < 5; ++ks) {
-            const char* rb = base + wrap(y + kdy[ks] - 1) * ROWB;
-            v8bf bh = *reinterpret_cast<const v8bf*>(rb + khi[ks]);
-            v8bf bl = *reinterpret_cast<const v8bf*>(rb + klo[ks]);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wl[ks], bh, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wh[ks], bl, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wh[ks], bh, acc, 0, 0, 0);
-          }
-        }
-        if (!last) {
-          v4f o;
-          if (is_conv2) {
-            v4f xr = acc + res[k];
-            res[k] = xr;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) o[q] = act_f(xr[q] * scale, actk);
-          } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) o[q] = act_f(acc[q], actk);
-          }
-          store4(out + b * cfg_bytes + y * ROWB, o);
-          // keep one item's fragments live at a time (bounds VGPR use)
-          __builtin_amdgcn_sched_barrier(0);
-        } else {
-          float hv[4], m = -INFINITY;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            hv[q] = (acc[q] + res[k][q]) * scale;
-            m = fmaxf(m, hv[q]);
-          }
-          m = wave_max(m);
-          float sacc = 0.0f;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) sacc += __expf(hv[q] - m);
-          sacc = wave_sum(sacc);
-#pragma unroll
-          for (int bb = 0; bb < B; ++bb) {
-            if (bb == b) {
-              float mm = fmaxf(m_b[bb], m);
-              s_b[bb] = s_b[bb] * __expf(m_b[bb] - mm) + sacc * __expf(m - mm);
-              m_b[bb] = mm;
-            }
-          }
-        }
-      }
-    }
-    if (!last) {
-      __syncthreads();
-      cur ^= 1;
-    } else {
-      if (lane == 0) {
-#pragma unroll
-        for (int b = 0; b < B; ++b) {
-          red[(b * W + wv) * 2] = m_b[b];
-          red[(b * W + wv) * 2 + 1] = s_b[b];
-        }
-      }
-      __syncthreads();
-      if (threadIdx.x < B) {
-        // waves' (max, sum) merged in FP32 (the sums are FP32 already): FP64
-        // exp / log here would hold the workgroup at the barrier below
-        int b = threadIdx.x;
-        float m = -INFINITY;
-        for (int w = 0; w < W; ++w) m = fmaxf(m, red[(b * W + w) * 2]);
-        float ssum = 0.0f;
-        for (int w = 0; w < W; ++w) {
-          const float mw = red[(b * W + w) * 2];
-          if (mw > -INFINITY) ssum += red[(b * W + w) * 2 + 1] * __expf(mw - m);
-        }
-        lp_out[b] = (double)m + (double)logf(ssum) - g.log_cn;
-      }
-      __syncthreads();
-    }
-  }
-}
-
+// ---------------------------------------------------------------- forwards
 // Sliding-row-window forward for C = 16 on a 16 x 16 grid.  Workgroup:
 // WPC B waves, B configurations; wave w owns the RPW = 16 / WPC rows
 // RPW (w % WPC) .. of configuration w / WPC and walks them in order keeping
@@ -1228,13 +726,6 @@ __device__ __forceinline__ void rc32_build_tab(const RcGeom& g, uint16_t* tab) {
 }
 
 // ---------------------------------------------------------------- kernels
-struct RcArgs {
-  RcGeom g;
-  int nb, actk;
-  const char* packed;
-  int64_t off_l0w, off_l0b, bias_off, off_frag, frag_bytes;
-};
-
 #define RC_FWD(SP, LP)                                                                                        \
   do {                                                                                                        \
     if constexpr (ROWS == 3) {                                                                                \
@@ -1250,22 +741,16 @@ struct RcArgs {
         rc_forward_t32<MAXT, W, RC32_CTW, QTX_ACT_GELU_TANH>(a.g, a.nb, a.packed, a.off_l0w, a.off_l0b,        \
                                                              a.bias_off, a.off_frag, a.frag_bytes, SP, act,    \
                                                              tab_, red, LP);                                   \
-    } else if constexpr (ROWS == 2)                                                                           \
+    } else                                                                                                    \
       rc_forward_win<MODE, B, W / B>(a.g, a.nb, a.actk, a.packed, a.off_l0w, a.off_l0b, a.bias_off, a.off_frag, \
                            a.frag_bytes, SP, act, wst, red, LP);                                              \
-    else if constexpr (ROWS == 1)                                                                             \
-      rc_forward_rows<MODE, B, MAXT, W>(a.g, a.nb, a.actk, a.packed, a.off_l0w, a.off_l0b, a.bias_off,   \
-                                        a.off_frag, a.frag_bytes, SP, act, red, LP);                          \
-    else                                                                                                      \
-      rc_forward<C, MODE, B, MAXT, W>(a.g, a.nb, a.actk, a.packed, a.off_l0w, a.off_l0b, a.bias_off,     \
-                                      a.off_frag, a.frag_bytes, SP, act, red, LP);                            \
   } while (0)
 
 template <int C, int MODE, int B, int NMAX, int MAXT, int W, int ROWS>
-__global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS == 3 ? 2 : (W == 8 ? 2 : 1)))) void rc_logpsi_kernel(RcArgs a, const int8_t* __restrict__ s, int64_t ns,
+__global__ __launch_bounds__(W * 64, 2) void rc_logpsi_kernel(RcArgs a, const int8_t* __restrict__ s, int64_t ns,
                                                                double* __restrict__ logabs) {
-  __shared__ __attribute__((aligned(16))) char act[(ROWS >= 2 ? 1 : 2) * B * NMAX * C * 4];
-  __shared__ __attribute__((aligned(16))) char wst[ROWS == 2 ? rc_win_lds(B) : (ROWS == 3 ? rc32_tab_bytes(NMAX) : 16)];
+  __shared__ __attribute__((aligned(16))) char act[B * NMAX * C * 4];
+  __shared__ __attribute__((aligned(16))) char wst[ROWS == 2 ? rc_win_lds(B) : rc32_tab_bytes(NMAX)];
   __shared__ int8_t sp[B * NMAX];
   __shared__ float red[2 * B * W];
   __shared__ double lp[B];
@@ -1281,20 +766,13 @@ __global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS =
   if (threadIdx.x < B && c0 + threadIdx.x < ns) logabs[c0 + threadIdx.x] = lp[threadIdx.x];
 }
 
-// log(u) of the acceptance test (metropolis.py:291-322) in FP64, kept out of
-// line: inlined, the constants of FP64 log1p would be hoisted into VGPRs for
-// the whole kernel
-__device__ __noinline__ double accept_threshold(uint32_t w2, uint32_t w3) {
-  return log1p(-words_to_uniform(w2, w3));
-}
-
 template <int C, int MODE, int B, int NMAX, int MAXT, int W, int ROWS>
-__global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS == 3 ? 2 : (W == 8 ? 2 : 1)))) void rc_metropolis_kernel(
+__global__ __launch_bounds__(W * 64, 2) void rc_metropolis_kernel(
     RcArgs a, int kind, const int32_t* __restrict__ nbr, int width, int hopping, const uint32_t* __restrict__ words,
     int nsteps, int64_t ns, double reweight, double tie_tol, int8_t* __restrict__ s, double* __restrict__ logabs,
     int32_t* __restrict__ n_accept, int32_t* __restrict__ n_near) {
-  __shared__ __attribute__((aligned(16))) char act[(ROWS >= 2 ? 1 : 2) * B * NMAX * C * 4];
-  __shared__ __attribute__((aligned(16))) char wst[ROWS == 2 ? rc_win_lds(B) : (ROWS == 3 ? rc32_tab_bytes(NMAX) : 16)];
+  __shared__ __attribute__((aligned(16))) char act[B * NMAX * C * 4];
+  __shared__ __attribute__((aligned(16))) char wst[ROWS == 2 ? rc_win_lds(B) : rc32_tab_bytes(NMAX)];
   __shared__ int8_t cur[B * NMAX];
   __shared__ int8_t prop[B * NMAX];
   __shared__ float red[2 * B * W];
@@ -1411,33 +889,18 @@ __global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS =
   }
 }
 
-// psi(s') / psi(s) = e^d for the local energy: 2^t, t = d log2(e), split
-// into an integer k applied exactly by ldexp and f = t - k in [-1/2, 1/2]
-// whose 2^f is one FP32 exp2 (about 1 ulp); the FP64 product d log2(e) and
-// the FP32 rounding of f keep the relative error near 1e-7 for any d, where
-// an FP32 exp of d itself would lose |d| * 2^-24 to the rounding of d alone.
-// |t| >= 2100 is exp's overflow (+inf) or underflow (0) outright, and NaN
-// stays NaN: no FP64 exp, whose polynomial constants would otherwise occupy
-// VGPRs for the whole kernel.
-__device__ __forceinline__ double exp_ratio(double d) {
-  const double t = d * 1.4426950408889634;
-  if (!(fabs(t) < 2100.0)) return d > 0.0 ? HUGE_VAL : (d < 0.0 ? 0.0 : d);  // exp's overflow / underflow; NaN stays
-  const double k = rint(t);
-  return ldexp((double)__builtin_amdgcn_exp2f((float)(t - k)), (int)k);
-}
-
 constexpr int RC_MAXCAND = 4096;
 constexpr int RC_MAXCAND_WIN = 3072;  // 16 x 16 window kernels: keeps two workgroups' LDS within a CU
 
 template <int C, int MODE, int B, int NMAX, int MAXT, int W, int ROWS>
-__global__ __launch_bounds__(W * 64, (ROWS == 2 ? (W == 4 * B ? 3 : 2) : (ROWS == 3 ? 2 : (W == 8 ? 2 : 1)))) void rc_eloc_kernel(RcArgs a, qtx_ham H, const int8_t* __restrict__ s,
+__global__ __launch_bounds__(W * 64, 2) void rc_eloc_kernel(RcArgs a, qtx_ham H, const int8_t* __restrict__ s,
                                                              const double* __restrict__ logabs, int S,
                                                              double* __restrict__ eloc, int32_t* __restrict__ nconn) {
   // S workgroups per sample (virtual block n S + sp): workgroup sp evaluates
   // the sp-th of S near-equal runs of candidates into eloc[n S + sp] (partial
   // sums for rc_eloc_sum_kernel when S > 1, the local energy when S = 1)
-  __shared__ __attribute__((aligned(16))) char act[(ROWS >= 2 ? 1 : 2) * B * NMAX * C * 4];
-  __shared__ __attribute__((aligned(16))) char wst[ROWS == 2 ? rc_win_lds(B) : (ROWS == 3 ? rc32_tab_bytes(NMAX) : 16)];
+  __shared__ __attribute__((aligned(16))) char act[B * NMAX * C * 4];
+  __shared__ __attribute__((aligned(16))) char wst[ROWS == 2 ? rc_win_lds(B) : rc32_tab_bytes(NMAX)];
   __shared__ int8_t s0[NMAX];
   __shared__ int8_t prop[B * NMAX];
   __shared__ float red[2 * B * W];
@@ -1574,53 +1037,30 @@ static RcArgs rc_args(const RcLayout& L, const void* packed) {
   a.bias_off = L.bias_off;
   a.off_frag = L.off_frag;
   a.frag_bytes = L.frag_bytes;
+  a.off_jac = L.off_jac;
   return a;
 }
 
-// Kernel configurations: (C, B, NMAX, MAXT) with B * ceil(NMAX/16) <= 4 * MAXT
-// (C = 16: N <= 256 -> 2 configurations per workgroup, N <= 512 -> 1; C = 32: N <= 400 -> 1).
-#define RC_DISPATCH(KERNEL, NS_PER_BLOCK_OUT, GRID_FROM_B, ...)                                        \
+// The 16 x 16 window kernels (two configurations per workgroup) and the large
+// 32-channel split-bf16 ones (one); every other shape runs the kernels of
+// resconv_wave.hpp
+static bool rc_own_kernel(const RcLayout& L) {
+  return L.win || (L.C == 32 && L.mode == QTX_CONV_BF16X3 && (L.N + 15) / 16 > 16);
+}
+
+#define RC_DISPATCH(KERNEL, GRID_FROM_B, ...)                                                          \
   do {                                                                                                 \
     if (L.win) {                                                                                       \
       constexpr int B_ = 2;                                                                            \
-      NS_PER_BLOCK_OUT = B_;                                                                           \
       dim3 grid_ = GRID_FROM_B;                                                                        \
       if (L.mode == QTX_CONV_FP32)                                                                     \
         hipLaunchKernelGGL((KERNEL<16, QTX_CONV_FP32, 2, 256, 4, 4, 2>), grid_, dim3(256), 0, st, __VA_ARGS__); \
       else                                                                                             \
         hipLaunchKernelGGL((KERNEL<16, QTX_CONV_BF16X3, 2, 256, 4, 4, 2>), grid_, dim3(256), 0, st, __VA_ARGS__); \
-    } else if (L.C == 16 && L.L1 == 16 && L.L0 <= 16) {                                                \
-      constexpr int B_ = 2;                                                                            \
-      NS_PER_BLOCK_OUT = B_;                                                                           \
-      dim3 grid_ = GRID_FROM_B;                                                                        \
-      if (L.mode == QTX_CONV_FP32)                                                                     \
-        hipLaunchKernelGGL((KERNEL<16, QTX_CONV_FP32, 2, 256, 4, 8, 1>), grid_, dim3(512), 0, st, __VA_ARGS__); \
-      else                                                                                             \
-        hipLaunchKernelGGL((KERNEL<16, QTX_CONV_BF16X3, 2, 256, 4, 8, 1>), grid_, dim3(512), 0, st, __VA_ARGS__); \
-    } else if (L.C == 16 && L.N <= 256) {                                                              \
-      constexpr int B_ = 2;                                                                            \
-      NS_PER_BLOCK_OUT = B_;                                                                           \
-      dim3 grid_ = GRID_FROM_B;                                                                        \
-      if (L.mode == QTX_CONV_FP32)                                                                     \
-        hipLaunchKernelGGL((KERNEL<16, QTX_CONV_FP32, 2, 256, 8, 4, 0>), grid_, dim3(256), 0, st, __VA_ARGS__); \
-      else                                                                                             \
-        hipLaunchKernelGGL((KERNEL<16, QTX_CONV_BF16X3, 2, 256, 8, 4, 0>), grid_, dim3(256), 0, st, __VA_ARGS__); \
-    } else if (L.C == 16) {                                                                            \
-      constexpr int B_ = 1;                                                                            \
-      NS_PER_BLOCK_OUT = B_;                                                                           \
-      dim3 grid_ = GRID_FROM_B;                                                                        \
-      if (L.mode == QTX_CONV_FP32)                                                                     \
-        hipLaunchKernelGGL((KERNEL<16, QTX_CONV_FP32, 1, 512, 8, 4, 0>), grid_, dim3(256), 0, st, __VA_ARGS__); \
-      else                                                                                             \
-        hipLaunchKernelGGL((KERNEL<16, QTX_CONV_BF16X3, 1, 512, 8, 4, 0>), grid_, dim3(256), 0, st, __VA_ARGS__); \
     } else {                                                                                           \
       constexpr int B_ = 1;                                                                            \
-      NS_PER_BLOCK_OUT = B_;                                                                           \
       dim3 grid_ = GRID_FROM_B;                                                                        \
-      if (L.mode == QTX_CONV_FP32)                                                                     \
-        hipLaunchKernelGGL((KERNEL<32, QTX_CONV_FP32, 1, 400, 7, 4, 0>), grid_, dim3(256), 0, st, __VA_ARGS__); \
-      else                                                                                             \
-        hipLaunchKernelGGL((KERNEL<32, QTX_CONV_BF16X3, 1, RC32_MAXN, 7, 4, 3>), grid_, dim3(256), 0, st, __VA_ARGS__); \
+      hipLaunchKernelGGL((KERNEL<32, QTX_CONV_BF16X3, 1, RC32_MAXN, 7, 4, 3>), grid_, dim3(256), 0, st, __VA_ARGS__); \
     }                                                                                                  \
   } while (0)
 
@@ -1685,9 +1125,9 @@ int qtx_resconv_logpsi(void* stream, const qtx_resconv_desc* d, const void* pack
   RcLayout L = rc_layout(d);
   RcArgs a = rc_args(L, packed);
   hipStream_t st = as_stream(stream);
-  int per = 1;
-  RC_DISPATCH(rc_logpsi_kernel, per, dim3((unsigned)((ns + B_ - 1) / B_)), a, s, ns, logabs);
-  (void)per;
+  if (!rc_own_kernel(L))
+    return RW_CALL(rw_logpsi, L, st, L, a, s, ns, logabs);
+  RC_DISPATCH(rc_logpsi_kernel, dim3((unsigned)((ns + B_ - 1) / B_)), a, s, ns, logabs);
   QTX_LAUNCH_CHECK();
   return QTX_OK;
 }
@@ -1708,10 +1148,11 @@ int qtx_resconv_metropolis(void* stream, const qtx_resconv_desc* d, const void* 
   RcLayout L = rc_layout(d);
   RcArgs a = rc_args(L, packed);
   hipStream_t st = as_stream(stream);
-  int per = 1;
-  RC_DISPATCH(rc_metropolis_kernel, per, dim3((unsigned)((ns + B_ - 1) / B_)), a, kind, nbr, width, hopping, words,
+  if (!rc_own_kernel(L))
+    return RW_CALL(rw_metropolis, L, st, L, a, kind, nbr, width, hopping, words, nsteps, ns, reweight, tie_tol, s,
+                   logabs, n_accept, n_near);
+  RC_DISPATCH(rc_metropolis_kernel, dim3((unsigned)((ns + B_ - 1) / B_)), a, kind, nbr, width, hopping, words,
               nsteps, ns, reweight, tie_tol, s, logabs, n_accept, n_near);
-  (void)per;
   QTX_LAUNCH_CHECK();
   return QTX_OK;
 }
@@ -1729,7 +1170,8 @@ int qtx_resconv_metropolis(void* stream, const qtx_resconv_desc* d, const void* 
 // 10 x 10, 4 blocks (FP32) 17.6 -> 17.0 ms.
 static int eloc_split(const RcLayout& L, int32_t noff, int64_t ns) {
   const int64_t want = (16 * 512 + ns - 1) / ns;
-  const int64_t most = noff / 4 / ((L.C == 16 && L.N <= 256) ? 16 : 8);
+  const int batch = L.win ? 2 : (rc_own_kernel(L) ? 1 : 4 / rw_pick(L.C, L.N, ns * (noff / 4)).P);
+  const int64_t most = noff / 4 / (8 * batch);
   return (int)std::max<int64_t>(1, std::min(want, most));
 }
 
@@ -1765,9 +1207,10 @@ int qtx_resconv_eloc_ws(void* stream, const qtx_resconv_desc* d, const void* pac
   RcArgs a = rc_args(L, packed);
   hipStream_t st = as_stream(stream);
   double* out = S > 1 ? (double*)ws : eloc;
-  int per = 1;
-  RC_DISPATCH(rc_eloc_kernel, per, dim3((unsigned)(ns * S)), a, *H, s, logabs, S, out, nconn);
-  (void)per;
+  if (rc_own_kernel(L))
+    RC_DISPATCH(rc_eloc_kernel, dim3((unsigned)(ns * S)), a, *H, s, logabs, S, out, nconn);
+  else if ((rc = RW_CALL(rw_eloc, L, st, L, a, *H, s, logabs, ns, S, out, nconn)))
+    return rc;
   if (S > 1)
     hipLaunchKernelGGL(rc_eloc_sum_kernel, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, st, out, ns, S, eloc);
   QTX_LAUNCH_CHECK();

@@ -35,36 +35,6 @@ namespace qtx {
 // through a neighbour table before, and four records per block through HBM).
 constexpr int JAC_THREADS = 256;
 
-// act(sc x) and act'(sc x) of four values, one branch on the activation
-__device__ __forceinline__ v4f act4(v4f x, float sc, int actk) {
-  v4f o;
-  if (actk == QTX_ACT_GELU_TANH) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) o[q] = act_f(x[q] * sc, QTX_ACT_GELU_TANH);
-  } else if (actk == QTX_ACT_RELU) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) o[q] = act_f(x[q] * sc, QTX_ACT_RELU);
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) o[q] = act_f(x[q] * sc, QTX_ACT_GELU_ERF);
-  }
-  return o;
-}
-
-__device__ __forceinline__ v4f act_grad4(v4f x, float sc, int actk) {
-  v4f o;
-  if (actk == QTX_ACT_GELU_TANH) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) o[q] = act_grad_f(x[q] * sc, QTX_ACT_GELU_TANH);
-  } else if (actk == QTX_ACT_RELU) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) o[q] = act_grad_f(x[q] * sc, QTX_ACT_RELU);
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) o[q] = act_grad_f(x[q] * sc, QTX_ACT_GELU_ERF);
-  }
-  return o;
-}
 constexpr int JAC_SLOTS = 768;  // workgroups of a launch: three per CU
 
 struct JacLds {  // byte offsets in the workgroup's dynamic LDS
@@ -142,18 +112,6 @@ __global__ __launch_bounds__(JAC_THREADS, WPS) void rc_jacobian_kernel(RcGeom g,
     // the swizzle key of site 16 t + l16 depends on l16 alone
     if (site(k) < N) *reinterpret_cast<v4f*>(buf + (wv + 4 * k) * (16 * C * 4) + put_off[ct]) = v;
   };
-  // Wait out the last MFMA of acc: the compiler counts the wait states from an
-  // MFMA to the first read of its result along the fall-through path only, so
-  // a short branch over a block that rewrites the same registers (an optional
-  // bias) read element 3 three instructions after the MFMA instead of ten.
-  // The asm statements keep their order, and each use of acc follows its own.
-  auto settle = [&](v4f (&acc)[MAXT][CT]) {
-    asm volatile("s_nop 15" : "+v"(acc[0][0]));
-#pragma unroll
-    for (int k = 0; k < MAXT; ++k)
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) asm volatile("" : "+v"(acc[k][ct]));
-  };
   // acc[k][ct] += the 3 x 3 convolution of the positions in buf with layer l's fragments
   auto conv = [&](const char* buf, int l, int dir, v4f (&acc)[MAXT][CT]) {
     const v4f* fr = reinterpret_cast<const v4f*>(jf + ((int64_t)l * 2 + dir) * per) + lane;
@@ -185,7 +143,7 @@ __global__ __launch_bounds__(JAC_THREADS, WPS) void rc_jacobian_kernel(RcGeom g,
         }
       }
     }
-    settle(acc);
+    mfma_settle<MAXT * CT>(&acc[0][0]);
   };
   auto zero = [&](v4f (&acc)[MAXT][CT]) {
 #pragma unroll

@@ -13,8 +13,6 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-constexpr int RC_WAVES = 4;
-constexpr int RC_THREADS = RC_WAVES * WAVE;
 constexpr int RC_MAXN = 1024;
 
 // ---------------------------------------------------------------- layout
@@ -56,14 +54,6 @@ __host__ __device__ inline void rc_theta_offsets(int nb, int C, int l, int64_t& 
   }
   w = b = -1;
 }
-
-template <int C, int MODE>
-struct RcK {
-  static constexpr int CT = C / 16;                                   // output-channel tiles
-  static constexpr int KS = (MODE == QTX_CONV_FP32) ? (9 * C / 4) : (C == 16 ? 5 : 9);  // K steps
-  static constexpr int CH = C / 4;                                    // 16-byte chunks per position
-  static constexpr int FRAG_WORDS = (MODE == QTX_CONV_FP32) ? 1 : 8;  // 4-byte words per lane per (ct, ks)
-};
 
 inline RcLayout rc_layout(const qtx_resconv_desc* d) {
   RcLayout L;
@@ -135,6 +125,102 @@ __device__ __forceinline__ int tap_pos(const RcGeom& g, int y, int x, int tap) {
   ys = ys < 0 ? ys + g.L0 : (ys >= g.L0 ? ys - g.L0 : ys);
   xs = xs < 0 ? xs + g.L1 : (xs >= g.L1 ? xs - g.L1 : xs);
   return ys * g.L1 + xs;
+}
+
+// act(sc x) and act'(sc x) of four values, one branch on the activation
+__device__ __forceinline__ v4f act4(v4f x, float sc, int actk) {
+  v4f o;
+  if (actk == QTX_ACT_GELU_TANH) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] = act_f(x[q] * sc, QTX_ACT_GELU_TANH);
+  } else if (actk == QTX_ACT_RELU) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] = act_f(x[q] * sc, QTX_ACT_RELU);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] = act_f(x[q] * sc, QTX_ACT_GELU_ERF);
+  }
+  return o;
+}
+
+__device__ __forceinline__ v4f act_grad4(v4f x, float sc, int actk) {
+  v4f o;
+  if (actk == QTX_ACT_GELU_TANH) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] = act_grad_f(x[q] * sc, QTX_ACT_GELU_TANH);
+  } else if (actk == QTX_ACT_RELU) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] = act_grad_f(x[q] * sc, QTX_ACT_RELU);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] = act_grad_f(x[q] * sc, QTX_ACT_GELU_ERF);
+  }
+  return o;
+}
+
+// v = hi + lo + O(2^-16 |v|): hi = bf16(v) (round to nearest even), lo =
+// bf16(v - hi).  v - hi is formed by v_dot2c_f32_bf16 from the packed hi
+// pair, (hi0, hi1) . (-1, 0) + v0 and (hi0, hi1) . (0, -1) + v1, exact
+// (bf16 products are exact in FP32 and v - hi is representable), so hi is
+// never widened back to FP32 by bit moves.
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split_bf16x4(v4f v, v4bf& hi, v4bf& lo) {
+  const v2bf h01 = {(__bf16)v[0], (__bf16)v[1]}, h23 = {(__bf16)v[2], (__bf16)v[3]};
+  // the selectors come from registers: an inline constant here (the
+  // compiler encodes e0 as "-1.0") is not read as (bf16 -1, 0) by the hardware
+  uint32_t u0 = 0x0000bf80u, u1 = 0xbf800000u;
+  asm("" : "+v"(u0), "+v"(u1));
+  const v2bf e0 = __builtin_bit_cast(v2bf, u0), e1 = __builtin_bit_cast(v2bf, u1);
+  const float l0 = __builtin_amdgcn_fdot2_f32_bf16(h01, e0, v[0], false);
+  const float l1 = __builtin_amdgcn_fdot2_f32_bf16(h01, e1, v[1], false);
+  const float l2 = __builtin_amdgcn_fdot2_f32_bf16(h23, e0, v[2], false);
+  const float l3 = __builtin_amdgcn_fdot2_f32_bf16(h23, e1, v[3], false);
+  const v2bf l01 = {(__bf16)l0, (__bf16)l1}, l23 = {(__bf16)l2, (__bf16)l3};
+  hi = v4bf{h01[0], h01[1], h23[0], h23[1]};
+  lo = v4bf{l01[0], l01[1], l23[0], l23[1]};
+}
+
+struct RcArgs {
+  RcGeom g;
+  int nb, actk;
+  const char* packed;
+  int64_t off_l0w, off_l0b, bias_off, off_frag, frag_bytes, off_jac;
+};
+
+// Wait out the MFMAs that wrote acc[0 .. N) before any use of them.  The
+// compiler counts the wait states behind an MFMA along the fall-through path
+// only: a use reached over a short branch can read a result (or overwrite a
+// register) too early.  Volatile asm statements keep their order: the first
+// pass puts every MFMA before the wait, the second every use after it.
+template <int N>
+__device__ __forceinline__ void mfma_settle(v4f* acc) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(acc[i]));
+  asm volatile("s_nop 15" : "+v"(acc[0]));
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(acc[i]));
+}
+
+// log(u) of the acceptance test (metropolis.py:291-322) in FP64, kept out of
+// line: inlined, the constants of FP64 log1p would be hoisted into VGPRs for
+// the whole kernel
+static __device__ __noinline__ double accept_threshold(uint32_t w2, uint32_t w3) {
+  return log1p(-words_to_uniform(w2, w3));
+}
+
+// psi(s') / psi(s) = e^d for the local energy: 2^t, t = d log2(e), split
+// into an integer k applied exactly by ldexp and f = t - k in [-1/2, 1/2]
+// whose 2^f is one FP32 exp2 (about 1 ulp); the FP64 product d log2(e) and
+// the FP32 rounding of f keep the relative error near 1e-7 for any d, where
+// an FP32 exp of d itself would lose |d| * 2^-24 to the rounding of d alone.
+// |t| >= 2100 is exp's overflow (+inf) or underflow (0) outright, and NaN
+// stays NaN: no FP64 exp, whose polynomial constants would otherwise occupy
+// VGPRs for the whole kernel.
+__device__ __forceinline__ double exp_ratio(double d) {
+  const double t = d * 1.4426950408889634;
+  if (!(fabs(t) < 2100.0)) return d > 0.0 ? HUGE_VAL : (d < 0.0 ? 0.0 : d);  // exp's overflow / underflow; NaN stays
+  const double k = rint(t);
+  return ldexp((double)__builtin_amdgcn_exp2f((float)(t - k)), (int)k);
 }
 
 static inline int rc_check(const qtx_resconv_desc* d) {
