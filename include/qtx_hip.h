@@ -425,6 +425,22 @@ int qtx_symm_images(void* stream, const int8_t* s, int64_t ns, int32_t N, const 
 int qtx_symmetrize(void* stream, const double* logabs, const double* sign_in, const double* coef, int64_t ns,
                    int32_t nimg, double* sign, double* logabs_out, double* w);
 
+/* The projected float64 RBM_Dense without materialised images (M, N <= 64,
+ * permutation table within LDS; qtx_symm_rbm_supported tells): sign and
+ * log|psi_sym| of each configuration, as qtx_symm_images + qtx_rbm_logpsi +
+ * qtx_symmetrize, and nsteps Metropolis steps of every chain in one launch, as
+ * qtx_propose + that + qtx_accept per step (sampler/metropolis.py:246-322);
+ * sign / logabs: in = current, out = final.  packed: qtx_rbm_pack, QTX_F64;
+ * perm, nperm, z2: as qtx_symm_images; coef: as qtx_symmetrize. */
+int qtx_symm_rbm_supported(int32_t M, int32_t N, int32_t nperm);
+int qtx_symm_rbm_logpsi(void* stream, const double* packed, int32_t M, int32_t N, const int32_t* perm, int32_t nperm,
+                        int32_t z2, const double* coef, const int8_t* s, int64_t ns, double* sign, double* logabs);
+int qtx_symm_rbm_metropolis(void* stream, const double* packed, int32_t M, int32_t N, const int32_t* perm,
+                            int32_t nperm, int32_t z2, const double* coef, int kind, const int32_t* nbr, int32_t width,
+                            int32_t hopping, const uint32_t* words, int32_t nsteps, int64_t ns, double reweight,
+                            double tie_tol, int8_t* s, double* sign, double* logabs, int32_t* n_accept,
+                            int32_t* n_near);
+
 /* O[s] = sum_g w[s, g] Oimg[s * nimg + g] (rows of np, o_dtype; FP64 sums):
  * the symmetrised Jacobian from the images' Jacobians. */
 int qtx_rows_combine(void* stream, int o_dtype, const void* Oimg, const double* w, int64_t ns, int32_t nimg,

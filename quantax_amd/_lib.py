@@ -95,6 +95,10 @@ PROTOS = {
     "qtx_scale_columns": (C.c_int, [vp, C.c_int, vp, vp, i64, i64, vp]),
     "qtx_symm_images": (C.c_int, [vp, vp, i64, C.c_int32, vp, C.c_int32, C.c_int32, vp]),
     "qtx_symmetrize": (C.c_int, [vp, vp, vp, vp, i64, C.c_int32, vp, vp, vp]),
+    "qtx_symm_rbm_supported": (C.c_int, [i32, i32, i32]),
+    "qtx_symm_rbm_logpsi": (C.c_int, [vp, vp, i32, i32, vp, i32, i32, vp, vp, i64, vp, vp]),
+    "qtx_symm_rbm_metropolis": (C.c_int, [vp, vp, i32, i32, vp, i32, i32, vp, C.c_int, vp, i32, i32, vp, i32, i64, f64,
+                                          f64, vp, vp, vp, vp, vp]),
     "qtx_rows_combine": (C.c_int, [vp, C.c_int, vp, vp, i64, C.c_int32, i64, vp]),
     "qtx_propose": (C.c_int, [vp, C.c_int, vp, C.c_int32, C.c_int32, vp, vp, i64, C.c_int32, vp, vp]),
     "qtx_accept": (C.c_int, [vp, vp, vp, vp, vp, vp, i64, C.c_int32, C.c_double, C.c_double, vp, vp, vp, vp, vp]),

@@ -14,7 +14,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "_lib")
 LIB = os.path.join(LIBDIR, "libqtxhip.so")
 SOURCES = ["qtx_core.hip", "qtx_sr.hip", "qtx_resconv.hip", "qtx_reswave16_fp32.hip",
-           "qtx_reswave16_bf16x3.hip", "qtx_reswave32_fp32.hip", "qtx_reswave32_bf16x3.hip", "qtx_resjac.hip", "qtx_serve.hip", "qtx_symm.hip"]
+           "qtx_reswave16_bf16x3.hip", "qtx_reswave32_fp32.hip", "qtx_reswave32_bf16x3.hip", "qtx_resjac.hip", "qtx_serve.hip", "qtx_symm.hip",
+           "qtx_symm_rbm.hip"]
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 

@@ -135,7 +135,13 @@ class Metropolis:
             ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             ev0.record()
             if self._generic:
-                self._generic_steps(words, nsteps)
+                if self._state.fused_symm and not getattr(self, "force_generic", False):
+                    _lib.call("qtx_symm_rbm_metropolis", _lib.stream(), *self._state._symm.rbm_args(model), self.kind,
+                              _lib.ptr(self._nbr), self._width, self._hopping, words.data_ptr(), nsteps, ns,
+                              self._reweight, self._tie_tol, self._spins.data_ptr(), self._sign.data_ptr(),
+                              self._logabs.data_ptr(), self.n_accept.data_ptr(), self.n_near.data_ptr())
+                else:
+                    self._generic_steps(words, nsteps)
             else:
                 model.metropolis(self.kind, self._nbr, self._width, self._hopping, words, nsteps, self._spins,
                                  self._logabs, self.n_accept, self.n_near, self._reweight, self._tie_tol)

@@ -71,8 +71,17 @@ class Variational:
         if self._symm is None:
             la = self._model.logpsi(s)
             return LogArray(torch.ones_like(la), la)
+        if self.fused_symm:
+            return LogArray(*self._symm.rbm_logpsi(self._model, s.contiguous()))
         sg, la = self._symm.project(self._model.logpsi(self._symm.images(s)))
         return LogArray(sg, la)
+
+    @property
+    def fused_symm(self) -> bool:
+        """A projected float64 RBM whose weights fit the kernels that form no
+        images (float32 ones keep the general path: their amplitudes are
+        rounded in its order)."""
+        return self._symm is not None and self._symm.fuses(self._model)
 
     def jacobian(self, fock_states) -> torch.Tensor:
         s = torch.as_tensor(fock_states, device=_lib.device()).to(torch.int8).reshape(-1, self.Nmodes)

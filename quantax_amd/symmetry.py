@@ -27,6 +27,7 @@ import torch
 
 from . import _lib
 from .global_defs import get_sites
+from .model import RBM_Dense
 
 
 def _group(generators: np.ndarray, sectors: Sequence[int], N: int):
@@ -152,6 +153,26 @@ class Symmetry:
         _lib.call("qtx_symm_images", _lib.stream(), s.data_ptr(), ns, self._N, perm.data_ptr(), perm.shape[0],
                   1 if self._Z2 else 0, out.data_ptr())
         return out
+
+    def fuses(self, model) -> bool:
+        """Whether ``model`` is projected by the kernels without images."""
+        return (isinstance(model, RBM_Dense) and model.theta.dtype == torch.float64 and model.N == self._N
+                and bool(_lib.lib().qtx_symm_rbm_supported(model.M, model.N, self._perm.shape[0])))
+
+    def rbm_args(self, model) -> tuple:
+        """The model and group arguments of ``qtx_symm_rbm_*``."""
+        perm, coef = self._device()
+        return (model.packed.data_ptr(), model.M, model.N, perm.data_ptr(), perm.shape[0], 1 if self._Z2 else 0,
+                coef.data_ptr())
+
+    def rbm_logpsi(self, model, s: torch.Tensor):
+        """(sign, log|psi_sym|) of a float64 RBM on (ns, N) int8 spins."""
+        ns = s.shape[0]
+        sg = torch.empty(ns, dtype=torch.float64, device=s.device)
+        la = torch.empty(ns, dtype=torch.float64, device=s.device)
+        _lib.call("qtx_symm_rbm_logpsi", _lib.stream(), *self.rbm_args(model), s.data_ptr(), ns, sg.data_ptr(),
+                  la.data_ptr())
+        return sg, la
 
     def project(self, logabs: torch.Tensor, weights: bool = False):
         """(ns * nsymm,) image log|psi| -> (sign, logabs) of psi_sym per sample,
