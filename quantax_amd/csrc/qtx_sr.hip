@@ -757,35 +757,69 @@ __global__ __launch_bounds__(1024) void lanczos_init_kernel(int64_t n, double* _
 }
 
 // single block, after w = T v_j: alpha_j = w.v_j, w -= alpha_j v_j + beta_j v_{j-1},
-// one re-orthogonalisation against v_j, beta_{j+1} = |w|, v_{j+1} = w / beta_{j+1}
+// one re-orthogonalisation against v_j, beta_{j+1} = |w|, v_{j+1} = w / beta_{j+1}.
+// n <= 1024 K (K > 0): the vectors are read once and stay in registers, so the
+// block waits for memory once instead of three times (27 -> 16 us at n = 16384,
+// 10.3 -> 6 us at 4096); K = 0 takes any n.
+template <int K>
 __global__ __launch_bounds__(1024) void lanczos_step_kernel(int64_t n, int j, double* __restrict__ w,
                                                             const double* __restrict__ v,
                                                             const double* __restrict__ vp, double* __restrict__ vn,
                                                             double* __restrict__ alpha, double* __restrict__ beta) {
   __shared__ double red[16];
   const double bj = beta[j];
-  double a = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) a += w[i] * v[i];
-  a = block_sum(a, red);
-  double a2 = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-    double t = w[i] - a * v[i] - bj * vp[i];
-    w[i] = t;
-    a2 += t * v[i];
+  double a = 0.0, a2 = 0.0, nn = 0.0;
+  if constexpr (K > 0) {
+    double wr[K], vr[K], pr[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int64_t i = threadIdx.x + 1024 * k;
+      wr[k] = i < n ? w[i] : 0.0;
+      vr[k] = i < n ? v[i] : 0.0;
+      pr[k] = i < n ? vp[i] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) a += wr[k] * vr[k];
+    a = block_sum(a, red);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      wr[k] = wr[k] - a * vr[k] - bj * pr[k];
+      a2 += wr[k] * vr[k];
+    }
+    a2 = block_sum(a2, red);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      wr[k] -= a2 * vr[k];
+      nn += wr[k] * wr[k];
+    }
+    nn = sqrt(block_sum(nn, red));
+    const double inv = nn > 0.0 ? 1.0 / nn : 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int64_t i = threadIdx.x + 1024 * k;
+      if (i < n) vn[i] = wr[k] * inv;
+    }
+  } else {
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) a += w[i] * v[i];
+    a = block_sum(a, red);
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+      double t = w[i] - a * v[i] - bj * vp[i];
+      w[i] = t;
+      a2 += t * v[i];
+    }
+    a2 = block_sum(a2, red);
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+      double t = w[i] - a2 * v[i];
+      w[i] = t;
+      nn += t * t;
+    }
+    nn = sqrt(block_sum(nn, red));
+    const double inv = nn > 0.0 ? 1.0 / nn : 0.0;
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) vn[i] = w[i] * inv;
   }
-  a2 = block_sum(a2, red);
-  double nn = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-    double t = w[i] - a2 * v[i];
-    w[i] = t;
-    nn += t * t;
-  }
-  double b = sqrt(block_sum(nn, red));
-  double inv = b > 0.0 ? 1.0 / b : 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) vn[i] = w[i] * inv;
   if (threadIdx.x == 0) {
     alpha[j] = a + a2;
-    beta[j + 1] = b;
+    beta[j + 1] = nn;
   }
 }
 
@@ -1012,6 +1046,177 @@ __global__ __launch_bounds__(256) void cheb_rows_kernel(const double* __restrict
   if (i >= n) return;
   const double w = wave_sum(wave_row_dot(S + i * n, u, i, n, lane));
   if (lane == 0) {
+    const double tk = tcur[i];
+    const double tn = first ? alpha * tk - beta * w : 2.0 * (alpha * tk - beta * w) - tprev[i];
+    tprev[i] = tn;
+    x[i] = first ? a0 * tk + a * tn : x[i] + a * tn;
+  }
+}
+
+// One read of a triangle for both of its products (n <= kTriPassMax).  A
+// workgroup of 512 threads (one per CU) takes rows c of the lower triangle
+// (row-major, columns j <= c), RB at a time: a thread holds the rows' columns
+// 2 t + 1024 i in registers, x is in LDS, the next rows are in flight while
+// these are used, and the row's multiples are added to the workgroup's partial
+// result in registers.
+//   SYM = false: w = P^T (P x): u_c = row . x, w += u_c row (one barrier a turn
+//                for the sum over the workgroup)
+//   SYM = true:  y = T x for symmetric T: y_c += row . x (columns j < c; the
+//                sums over the workgroup are taken once, at the end), y += x_c row
+// part: (gridDim.x, n) partial results; dots: n (SYM).  HBM-bound: half the
+// bytes of two half-row passes (P) or of full rows (T).
+constexpr int TP_THREADS = 512, TP_WAVES = TP_THREADS / WAVE;
+constexpr int TP_GRID = 256;  // one workgroup per CU (x fills most of the LDS)
+// Where one read of half the matrix wins.  Below, the matrix comes from the
+// last-level cache and the partial results cost more than the second read
+// (us, two reads | one and its sum):
+//   n      T x          P^T P x
+//   3000   13.8 | 18.2   20.5 | 20.8
+//   4096   21.5 | 23.7   30.4 | 26.8
+//   5000   34.2 | 32.0   41.8 | 37.5
+//   6144   46.8 | 38.6   59.2 | 44.5
+//   8192   84.5 | 57.7   98.7 | 63.0
+//   16384   329 |  216    360 |  223  (1.07 GB: 5.0 TB/s)
+constexpr int64_t kTriPassSymMin = 4608, kTriPassMin = 3072, kTriPassMax = 16384;
+typedef double v2d_u __attribute__((ext_vector_type(2), aligned(8)));
+
+template <int NC>
+constexpr int tp_lds() {  // x, then the waves' sums of every row (at most kTriPassMax / TP_GRID turns of one row)
+  return 2 * TP_THREADS * NC * 8 + (int)(kTriPassMax / TP_GRID) * TP_WAVES * 8;
+}
+
+template <int RB, int NC, bool SYM>
+__global__ __launch_bounds__(TP_THREADS) void tri_pass_kernel(const double* __restrict__ S, int64_t n,
+                                                              const double* __restrict__ X,
+                                                              double* __restrict__ part, double* __restrict__ dots) {
+  static_assert(RB * TP_WAVES <= WAVE, "one lane per wave's sum");
+  extern __shared__ __attribute__((aligned(16))) double tp[];
+  double* xs = tp;                         // 2 TP_THREADS NC, zero past n
+  double* red = tp + 2 * TP_THREADS * NC;  // [turn (SYM) or turn % 2][RB][TP_WAVES]
+  const int t = threadIdx.x, lane = t % WAVE, wv = t / WAVE;
+  for (int j = t; j < 2 * TP_THREADS * NC; j += TP_THREADS) xs[j] = j < n ? X[j] : 0.0;
+  __syncthreads();
+  v2d_u w[NC], row[2][RB][NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) w[i] = v2d_u{0.0, 0.0};
+  auto row_of = [&](int turn, int r) { return ((int64_t)turn * TP_GRID + blockIdx.x) * RB + r; };
+  auto load = [&](int turn, v2d_u (&b)[RB][NC]) {
+    int off = 16 * t;
+    asm volatile("" : "+v"(off));  // the NC offsets are formed in every turn, not kept in registers
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      const int64_t c = row_of(turn, r);
+      // the row up to its diagonal; columns past it (and rows past n) read as zero
+      const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)(S + (c < n ? c * n : 0)), 0,
+                                                        c < n ? (int)(c + 1) * 8 : 0, 0x00020000);
+#pragma unroll
+      for (int i = 0; i < NC; ++i)
+        b[r][i] = __builtin_bit_cast(v2d_u, __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16 * TP_THREADS * i, 0, 0));
+    }
+  };
+  auto use = [&](int turn, v2d_u (&b)[RB][NC]) {
+    asm volatile("" ::: "memory");  // x is read from LDS in every turn, not kept in registers
+    double* rd = red + (SYM ? turn : (turn & 1)) * RB * TP_WAVES;
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      int d = 2 * t - (int)row_of(turn, r);  // the diagonal is at column 2 t - d
+      asm volatile("" : "+v"(d));
+      double p = 0.0;
+#pragma unroll
+      for (int i = 0; i < NC; ++i) {
+        if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // few of x's reads at a time
+        const double2 x2 = *reinterpret_cast<const double2*>(xs + 2 * t + 2 * TP_THREADS * i);
+        if (d == -2 * TP_THREADS * i) b[r][i].y = 0.0;  // the second of the last pair, if there is one to read
+        // the diagonal of T belongs to the row's multiple
+        p += (SYM && d == -2 * TP_THREADS * i ? 0.0 : b[r][i].x) * x2.x + (SYM && d == -2 * TP_THREADS * i - 1 ? 0.0 : b[r][i].y) * x2.y;
+      }
+      p = wave_sum(p);
+      if (lane == 0) rd[r * TP_WAVES + wv] = p;
+    }
+    double sums = 0.0;
+    if (!SYM) {
+      __syncthreads();
+      sums = rd[lane % (RB * TP_WAVES)];
+      for (int q = 1; q < TP_WAVES; q *= 2) sums += __shfl_xor(sums, q, WAVE);
+    }
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      const int64_t c = row_of(turn, r);
+      const double u = SYM ? (c < n ? xs[c] : 0.0) : __shfl(sums, r * TP_WAVES, WAVE);
+#pragma unroll
+      for (int i = 0; i < NC; ++i) w[i] += u * b[r][i];
+    }
+  };
+  const int turns = (int)((n + (int64_t)TP_GRID * RB - 1) / ((int64_t)TP_GRID * RB));
+  load(0, row[0]);
+  for (int k = 0; k < turns; k += 2) {  // a turn past the last loads nothing: its rows are past n
+    load(k + 1, row[1]);
+    use(k, row[0]);
+    if (k + 1 == turns) break;
+    load(k + 2, row[0]);
+    use(k + 1, row[1]);
+  }
+  double* out = part + (int64_t)blockIdx.x * n;
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int64_t j = 2 * t + 2 * TP_THREADS * i;
+    if (j < n) out[j] = w[i].x;
+    if (j + 1 < n) out[j + 1] = w[i].y;
+  }
+  if (SYM) {
+    __syncthreads();
+    for (int e = t; e < turns * RB; e += TP_THREADS) {
+      const int64_t c = row_of(e / RB, e % RB);
+      if (c < n) {
+        double u = 0.0;
+#pragma unroll
+        for (int q = 0; q < TP_WAVES; ++q) u += red[e * TP_WAVES + q];
+        dots[c] = u;
+      }
+    }
+  }
+}
+
+// sums over the TP_GRID partial results of TP_COLS columns, for threads t < TP_COLS
+constexpr int TP_COLS = 16;
+__device__ __forceinline__ double tp_column_sum(const double* __restrict__ part, int64_t n, int64_t j) {
+  __shared__ double sh[1024 / WAVE][TP_COLS];
+  const int t = threadIdx.x, grp = t / TP_COLS;
+  double a = 0.0;
+  if (j < n) {
+    double v[TP_GRID * TP_COLS / 1024];
+#pragma unroll
+    for (int k = 0; k < TP_GRID * TP_COLS / 1024; ++k) v[k] = part[(int64_t)(grp + k * (1024 / TP_COLS)) * n + j];
+#pragma unroll
+    for (int k = 0; k < TP_GRID * TP_COLS / 1024; ++k) a += v[k];
+  }
+  a += __shfl_xor(a, 16, WAVE);
+  a += __shfl_xor(a, 32, WAVE);
+  if (t % WAVE < TP_COLS) sh[t / WAVE][t % WAVE] = a;
+  __syncthreads();
+  double s = 0.0;
+  if (t < TP_COLS)
+#pragma unroll
+    for (int q = 0; q < 1024 / WAVE; ++q) s += sh[q][t];
+  return s;
+}
+
+// y = T x from tri_pass_kernel<SYM>
+__global__ __launch_bounds__(1024) void tp_sum_kernel(const double* __restrict__ part, const double* __restrict__ dots,
+                                                      int64_t n, double* __restrict__ y) {
+  const int64_t j = (int64_t)blockIdx.x * TP_COLS + threadIdx.x % TP_COLS;
+  const double s = tp_column_sum(part, n, j);
+  if (threadIdx.x < TP_COLS && j < n) y[j] = s + dots[j];
+}
+
+// the Chebyshev recurrence of cheb_rows_kernel on w = P^T P t_k from tri_pass_kernel
+__global__ __launch_bounds__(1024) void tp_cheb_kernel(const double* __restrict__ part, int64_t n,
+                                                       const double* __restrict__ tcur, double* __restrict__ tprev,
+                                                       double alpha, double beta, double a0, double a, int first,
+                                                       double* __restrict__ x) {
+  const int64_t i = (int64_t)blockIdx.x * TP_COLS + threadIdx.x % TP_COLS;
+  const double w = tp_column_sum(part, n, i);
+  if (threadIdx.x < TP_COLS && i < n) {
     const double tk = tcur[i];
     const double tn = first ? alpha * tk - beta * w : 2.0 * (alpha * tk - beta * w) - tprev[i];
     tprev[i] = tn;
@@ -1760,6 +1965,26 @@ static int tri_inverse(rocblas_handle h, hipStream_t st, int64_t n, double* A, i
   return QTX_OK;
 }
 
+// tri_pass_kernel for this n (tri_pass_ok); part needs TP_GRID n doubles
+template <bool SYM>
+static int launch_tri_pass(hipStream_t st, const double* S, int64_t n, const double* X, double* part, double* dots) {
+#define QTX_TP(RB, NC)                                                                                             \
+  do {                                                                                                             \
+    QTX_HIP(hipFuncSetAttribute((const void*)tri_pass_kernel<RB, NC, SYM>,                                         \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, tp_lds<NC>()));                    \
+    hipLaunchKernelGGL((tri_pass_kernel<RB, NC, SYM>), dim3(TP_GRID), dim3(TP_THREADS), (tp_lds<NC>()), st, S, \
+                       n, X, part, dots);                                                                          \
+  } while (0)
+  if (n <= 4096) QTX_TP(4, 4);
+  else if (n <= 8192) QTX_TP(2, 8);
+  else QTX_TP(1, 16);
+#undef QTX_TP
+  return QTX_OK;
+}
+static bool tri_pass_ok(int64_t n, bool sym) {
+  return n >= (sym ? kTriPassSymMin : kTriPassMin) && n <= kTriPassMax;
+}
+
 // ---------------------------------------------------------------- phased solve
 // A solve runs as three phases so that many solves on different streams can
 // be driven from one host thread with batched host syncs
@@ -1880,8 +2105,18 @@ static int lanczos_enqueue(Task& t, rocblas_handle h, int to) {
     double* v = t.w.V + (j % 3) * t.n;
     double* vp = t.w.V + ((j + 2) % 3) * t.n;
     double* vn = t.w.V + ((j + 1) % 3) * t.n;
-    hipLaunchKernelGGL(matvec_rows_kernel<1>, dim3(gm), dim3(256), 0, t.st, t.w.T, t.n, v, t.w.w);
-    hipLaunchKernelGGL(lanczos_step_kernel, dim3(1), dim3(1024), 0, t.st, t.n, j, t.w.w, v, vp, vn, alpha, beta);
+    if (tri_pass_ok(t.n, true)) {  // T2 is free until the factorisation
+      int rc = launch_tri_pass<true>(t.st, t.w.T, t.n, v, t.w.T2, t.w.R);
+      if (rc) return rc;
+      hipLaunchKernelGGL(tp_sum_kernel, dim3(nblk(t.n, TP_COLS)), dim3(1024), 0, t.st, t.w.T2, t.w.R, t.n, t.w.w);
+    } else {
+      hipLaunchKernelGGL(matvec_rows_kernel<1>, dim3(gm), dim3(256), 0, t.st, t.w.T, t.n, v, t.w.w);
+    }
+    const auto step = t.n <= 1024    ? lanczos_step_kernel<1>
+                      : t.n <= 4096  ? lanczos_step_kernel<4>
+                      : t.n <= 16384 ? lanczos_step_kernel<16>
+                                     : lanczos_step_kernel<0>;
+    hipLaunchKernelGGL(step, dim3(1), dim3(1024), 0, t.st, t.n, j, t.w.w, v, vp, vn, alpha, beta);
   }
   QTX_LAUNCH_CHECK();
   t.done = to;
@@ -2157,6 +2392,12 @@ static int phase2(Task& t, rocblas_handle h) {
       for (int k = 0; k + 1 < t.cheb_terms; ++k) {
         const double* tcur = B[k & 1];
         double* tprev = B[(k + 1) & 1];
+        if (tri_pass_ok(t.n, false)) {  // the third of the n x n buffers is free here
+          if ((rc = launch_tri_pass<false>(t.st, t.w.T2, t.n, tcur, t.w.T2 + 2 * nn, nullptr))) return rc;
+          hipLaunchKernelGGL(tp_cheb_kernel, dim3(nblk(t.n, TP_COLS)), dim3(1024), 0, t.st, t.w.T2 + 2 * nn, t.n, tcur,
+                             tprev, alpha, beta, ca[0], ca[k + 1], k == 0 ? 1 : 0, t.w.x);
+          continue;
+        }
         hipLaunchKernelGGL(tri_rows_kernel<true>, dim3(gm), dim3(256), 0, t.st, t.w.T2, t.n, tcur, u);
         hipLaunchKernelGGL(cheb_rows_kernel, dim3(gm), dim3(256), 0, t.st, t.w.T2, t.n, u, tcur, tprev, alpha, beta,
                            ca[0], ca[k + 1], k == 0 ? 1 : 0, t.w.x);
