@@ -346,7 +346,7 @@ __global__ __launch_bounds__(256) void gram_bf16x3_kernel(const __bf16* __restri
                                                           int ntiles, double* __restrict__ T) {
   __shared__ __attribute__((aligned(16))) char smem[2 * 4 * G3_PLANE];
   int bi, bj;
-  tile_of(xcd_tile(blockIdx.x, ntiles), bi, bj);
+  super_tile_of(xcd_tile(blockIdx.x, ntiles), (int)((n + GT - 1) / GT), bi, bj);
   const int64_t i0 = (int64_t)bi * GT, j0 = (int64_t)bj * GT;
   const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
   const int wr = (wv / 2) * 64, wc = (wv % 2) * 64;
