@@ -38,17 +38,83 @@ __global__ void fill_i32_kernel(int32_t* p, int64_t n, int32_t v) {
   if (i < n) p[i] = v;
 }
 
-// column sums over a chunk of rows, accumulated with FP64 atomics
-template <typename T>
-__global__ __launch_bounds__(256) void colsum_kernel(const T* __restrict__ O, int64_t ns, int64_t np,
-                                                     int64_t rows_per_chunk, double* __restrict__ out) {
-  int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= np) return;
-  int64_t r0 = (int64_t)blockIdx.y * rows_per_chunk;
-  int64_t r1 = r0 + rows_per_chunk < ns ? r0 + rows_per_chunk : ns;
-  double acc = 0.0;
-  for (int64_t r = r0; r < r1; ++r) acc += (double)O[r * np + k];
-  atomicAdd(out + k, acc);
+// Column sums over a chunk of rows, accumulated with FP64 atomics:
+//   W = false: out_k += sum_s O_sk
+//   W = true:  out_k += sum_s (O_sk - mean_k) sqrt(r_s inv_ns) y_s
+// HBM-bound: every element is read once.  A lane takes four neighbouring
+// columns (one load that needs only the element's own alignment), a wave 256
+// columns of every fourth row of the chunk, CS_ROWS rows in flight; the rows'
+// weights are made once, in LDS, CS_PART at a time.  colsum_rows: eight
+// workgroups per CU, of at least CS_MIN rows each: few columns fill the chip too.
+// 4096 x 40400 f32: sum 237 -> 173 us, weighted 257 -> 119 us; 1024 x 272 f64:
+// 33 -> 9.7, 64 -> 8.5 us (one column per thread, one row in flight before).
+constexpr int CS_COLS = 256, CS_ROWS = 8, CS_MIN = 16, CS_PART = 512;
+template <typename TI, bool W>
+__global__ __launch_bounds__(256) void colsum_kernel(const TI* __restrict__ O, const double* __restrict__ mean,
+                                                     const double* __restrict__ r, const double* __restrict__ y,
+                                                     int64_t ns, int64_t np, int64_t rows_per_chunk, double inv_ns,
+                                                     double* __restrict__ out) {
+  typedef TI vt4 __attribute__((ext_vector_type(4), aligned(sizeof(TI))));
+  __shared__ double ws[CS_PART];
+  __shared__ double red[3][CS_COLS];
+  const int tid = threadIdx.x, lane = tid % WAVE, q = tid / WAVE;
+  const int64_t k0 = (int64_t)blockIdx.x * CS_COLS, k = k0 + 4 * lane;
+  const int64_t rc = (int64_t)blockIdx.y * rows_per_chunk;
+  const int64_t re = rc + rows_per_chunk < ns ? rc + rows_per_chunk : ns;
+  const int cols = (int)(k + 4 <= np ? 4 : k < np ? np - k : 0);
+  double acc[4] = {0, 0, 0, 0}, m[4] = {0, 0, 0, 0};
+  if (W)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (c < cols) m[c] = mean[k + c];
+  for (int64_t r0 = rc; r0 < re; r0 += CS_PART) {
+    const int rows = (int)(re - r0 < CS_PART ? re - r0 : CS_PART);
+    if (W) {
+      if (r0 > rc) __syncthreads();  // the last part's weights have been used
+      for (int s = tid; s < rows; s += 256) ws[s] = y[r0 + s] * sqrt((r ? r[r0 + s] : 1.0) * inv_ns);
+      __syncthreads();
+    }
+    const TI* p = O + r0 * np + k;
+    if (cols == 4) {
+      int s = q;
+      for (; s + 4 * (CS_ROWS - 1) < rows; s += 4 * CS_ROWS) {
+        vt4 v[CS_ROWS];
+#pragma unroll
+        for (int i = 0; i < CS_ROWS; ++i) v[i] = *reinterpret_cast<const vt4*>(p + (s + 4 * i) * np);
+#pragma unroll
+        for (int i = 0; i < CS_ROWS; ++i)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) acc[c] += W ? ((double)v[i][c] - m[c]) * ws[s + 4 * i] : (double)v[i][c];
+      }
+      for (; s < rows; s += 4) {
+        const vt4 v = *reinterpret_cast<const vt4*>(p + s * np);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[c] += W ? ((double)v[c] - m[c]) * ws[s] : (double)v[c];
+      }
+    } else if (cols > 0) {
+      for (int s = q; s < rows; s += 4)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          if (c < cols) acc[c] += W ? ((double)p[s * np + c] - m[c]) * ws[s] : (double)p[s * np + c];
+    }
+  }
+  if (q > 0)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) red[q - 1][4 * lane + c] = acc[c];
+  __syncthreads();
+  if (q == 0)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (c < cols) atomicAdd(out + k + c, acc[c] + red[0][4 * lane + c] + red[1][4 * lane + c] + red[2][4 * lane + c]);
+}
+
+// rows per chunk, and the grid
+static int64_t colsum_rows(int64_t ns, int64_t np, dim3& g) {
+  const int64_t gx = (np + CS_COLS - 1) / CS_COLS;
+  const int64_t chunks = std::min<int64_t>(std::max<int64_t>(1, 2048 / gx), (ns + CS_MIN - 1) / CS_MIN);
+  const int64_t rpc = (ns + chunks - 1) / chunks;
+  g = dim3((unsigned)gx, (unsigned)((ns + rpc - 1) / rpc));
+  return rpc;
 }
 
 __global__ void scale_f64_kernel(double* p, int64_t n, double a) {
@@ -479,24 +545,6 @@ __global__ void form_obar_kernel(const TI* __restrict__ O, const double* __restr
     const int64_t s = e / np, k = e - s * np;
     out[e] = ((double)O[e] - mean[k]) * sqrt((r ? r[s] : 1.0) * inv_ns);
   }
-}
-
-// x_k = sum_s (O_sk - mean_k) sqrt(r_s / ns) y_s  (FP64 accumulation)
-template <typename TI>
-__global__ __launch_bounds__(256) void obar_t_y_kernel(const TI* __restrict__ O, const double* __restrict__ mean,
-                                                       const double* __restrict__ r, const double* __restrict__ y,
-                                                       int64_t ns, int64_t np, int64_t rows_per_chunk,
-                                                       double inv_ns, double* __restrict__ x) {
-  int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= np) return;
-  int64_t r0 = (int64_t)blockIdx.y * rows_per_chunk;
-  int64_t r1 = r0 + rows_per_chunk < ns ? r0 + rows_per_chunk : ns;
-  double acc = 0.0, m = mean[k];
-  for (int64_t s = r0; s < r1; ++s) {
-    double w = y[s] * sqrt((r ? r[s] : 1.0) * inv_ns);
-    acc += ((double)O[s * np + k] - m) * w;
-  }
-  atomicAdd(x + k, acc);
 }
 
 // y_s = beta y_s + alpha sqrt(r_s / ns) sum_k (O_sk - mean_k) v_k: the product
@@ -1540,12 +1588,9 @@ template <typename TI>
 static int launch_obar_t_y(hipStream_t st, const TI* O, const double* mean, const double* r, const double* y,
                            int64_t ns, int64_t np, double* x) {
   hipLaunchKernelGGL(fill_f64_kernel, dim3(nblk(np, 256)), dim3(256), 0, st, x, np, 0.0);
-  int64_t chunks = (ns + 255) / 256;
-  if (chunks > 256) chunks = 256;
-  int64_t rpc = (ns + chunks - 1) / chunks;
-  chunks = (ns + rpc - 1) / rpc;
-  dim3 g(nblk(np, 256), (unsigned)chunks);
-  hipLaunchKernelGGL(obar_t_y_kernel<TI>, g, dim3(256), 0, st, O, mean, r, y, ns, np, rpc, 1.0 / (double)ns, x);
+  dim3 g;
+  const int64_t rpc = colsum_rows(ns, np, g);
+  hipLaunchKernelGGL((colsum_kernel<TI, true>), g, dim3(256), 0, st, O, mean, r, y, ns, np, rpc, 1.0 / (double)ns, x);
   QTX_LAUNCH_CHECK();
   return QTX_OK;
 }
@@ -2903,15 +2948,15 @@ int qtx_colmean(void* stream, int o_dtype, const void* O, int64_t ns, int64_t np
   QTX_REQUIRE(ns > 0 && np > 0 && O && mean, "bad arguments");
   hipStream_t st = as_stream(stream);
   hipLaunchKernelGGL(fill_f64_kernel, dim3(nblk(np, 256)), dim3(256), 0, st, mean, np, 0.0);
-  int64_t chunks = (ns + 127) / 128;
-  if (chunks > 128) chunks = 128;
-  int64_t rpc = (ns + chunks - 1) / chunks;
-  chunks = (ns + rpc - 1) / rpc;
-  dim3 g(nblk(np, 256), (unsigned)chunks);
+  dim3 g;
+  const int64_t rpc = colsum_rows(ns, np, g);
+  const double* none = nullptr;
   if (o_dtype == QTX_F32)
-    hipLaunchKernelGGL(colsum_kernel<float>, g, dim3(256), 0, st, (const float*)O, ns, np, rpc, mean);
+    hipLaunchKernelGGL((colsum_kernel<float, false>), g, dim3(256), 0, st, (const float*)O, none, none, none, ns, np,
+                       rpc, 0.0, mean);
   else
-    hipLaunchKernelGGL(colsum_kernel<double>, g, dim3(256), 0, st, (const double*)O, ns, np, rpc, mean);
+    hipLaunchKernelGGL((colsum_kernel<double, false>), g, dim3(256), 0, st, (const double*)O, none, none, none, ns, np,
+                       rpc, 0.0, mean);
   hipLaunchKernelGGL(scale_f64_kernel, dim3(nblk(np, 256)), dim3(256), 0, st, mean, np, 1.0 / (double)ns);
   QTX_LAUNCH_CHECK();
   return QTX_OK;
