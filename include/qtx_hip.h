@@ -83,6 +83,11 @@ int qtx_device_sync(void);
 int qtx_philox_fill(void* stream, uint64_t seed, uint32_t tag, int64_t step0, int64_t nsteps,
                     int64_t chain0, int64_t nchains, uint32_t* words);
 
+/* count[0] = number of chains whose incrementally updated logabs is not close to
+ * the full forward's: neither |e^a - e^b| < 1e-8 nor |e^(a-b) - 1| < 1e-3.
+ * Replaces the check of sampler/metropolis.py:201-213. */
+int qtx_drift_count(void* stream, const double* logabs, const double* full, int64_t ns, int32_t* count);
+
 /* Initial chains: uniform +-1 (nup < 0) or a uniform permutation of nup up
  * spins (Fisher-Yates on Philox draws).  Replaces utils/basis.py:160-219. */
 int qtx_init_spins(void* stream, uint64_t seed, int64_t nchains, int32_t N, int32_t nup, int8_t* s);

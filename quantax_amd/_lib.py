@@ -61,6 +61,7 @@ PROTOS = {
     "qtx_last_error": (C.c_char_p, []),
     "qtx_device_sync": (C.c_int, []),
     "qtx_philox_fill": (C.c_int, [vp, u64, u32, i64, i64, i64, i64, vp]),
+    "qtx_drift_count": (C.c_int, [vp, vp, vp, i64, vp]),
     "qtx_init_spins": (C.c_int, [vp, u64, i64, i32, i32, vp]),
     "qtx_ham_diag": (C.c_int, [vp, C.POINTER(QtxHam), vp, i64, vp]),
     "qtx_conn_count": (C.c_int, [vp, C.POINTER(QtxHam), vp, i64, vp]),

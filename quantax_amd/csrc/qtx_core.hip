@@ -203,6 +203,22 @@ __global__ __launch_bounds__(256) void rbm_jacobian_kernel(const T* __restrict__
   rbm_jacobian_row<T, TO>(packed, M, N, s + n * N, O + n * ((int64_t)M * N + M), tl, tld, sl);
 }
 
+// wavefunctions whose incremental logabs a and full-forward logabs b differ:
+// neither |e^a - e^b| < 1e-8 nor |e^(a - b) - 1| < 1e-3 (NaN counts as different)
+__global__ __launch_bounds__(256) void drift_count_kernel(const double* __restrict__ a, const double* __restrict__ b,
+                                                          int64_t n, int32_t* __restrict__ count) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  bool far = false;
+  if (i < n) {
+    const double x = a[i], y = b[i];
+    far = !(fabs(exp(x) - exp(y)) < 1e-8 || fabs(exp(x - y) - 1.0) < 1e-3);
+  }
+  const int c = __popcll(__ballot(far));
+  if (threadIdx.x % WAVE == 0 && c > 0) atomicAdd(count, c);
+}
+
+__global__ void zero_i32_kernel(int32_t* p) { *p = 0; }
+
 }  // namespace qtx
 
 using namespace qtx;
@@ -236,6 +252,16 @@ int qtx_philox_fill(void* stream, uint64_t seed, uint32_t tag, int64_t step0, in
   if (total == 0) return QTX_OK;
   hipLaunchKernelGGL(philox_fill_kernel, dim3(blocks_for(total, 256)), dim3(256), 0, as_stream(stream), seed, tag,
                      step0, nsteps, chain0, nchains, words);
+  QTX_LAUNCH_CHECK();
+  return QTX_OK;
+}
+
+int qtx_drift_count(void* stream, const double* logabs, const double* full, int64_t ns, int32_t* count) {
+  QTX_REQUIRE(ns >= 0 && count != nullptr && (ns == 0 || (logabs && full)), "bad drift_count arguments");
+  hipLaunchKernelGGL(zero_i32_kernel, dim3(1), dim3(1), 0, as_stream(stream), count);
+  if (ns > 0)
+    hipLaunchKernelGGL(drift_count_kernel, dim3(blocks_for(ns, 256)), dim3(256), 0, as_stream(stream), logabs, full,
+                       ns, count);
   QTX_LAUNCH_CHECK();
   return QTX_OK;
 }

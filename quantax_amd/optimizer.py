@@ -225,7 +225,7 @@ class QNGD:
     def get_step(self, samples) -> torch.Tensor:
         ebar = self.get_Ebar(samples)
         O, mean = self.get_Obar(samples)
-        r = None if samples.reweight_factor is None or self._trivial_r(samples) else samples.reweight_factor
+        r = self._weights(samples)
         ns, np_ = O.shape
         need = self._solver.ws_bytes(ns, np_)
         if self._ws is None or self._ws.numel() < need:
@@ -233,8 +233,17 @@ class QNGD:
         return solve_step(O, mean, ebar, self._solver, r, self._ws)
 
     @staticmethod
-    def _trivial_r(samples) -> bool:
-        return bool(torch.all(samples.reweight_factor == 1.0).item())
+    def _weights(samples) -> Optional[torch.Tensor]:
+        """The reweighting factors as the kernels take them.  Factors of one give
+        the same bits as none, so a tensor that the kernels can read goes to them
+        unseen: looking at its values would make the host wait for the sweep (60
+        us, twice per step).  Any other tensor is looked at: ones need no kernel
+        to read them."""
+        r = samples.reweight_factor
+        if r is None or (r.dtype == torch.float64 and r.is_contiguous() and r.device == samples.spins.device
+                         and r.shape == samples.spins.shape[:1]):
+            return r
+        return None if bool(torch.all(r == 1.0).item()) else r
 
 
 class SR(QNGD):
@@ -263,8 +272,8 @@ class SR(QNGD):
         eloc = self._hamiltonian.Oloc(self._state, samples)
         self._eloc = eloc
         ns = eloc.shape[0]
-        r = samples.reweight_factor
-        r = None if r is None or self._trivial_r(samples) else r.contiguous()
+        r = self._weights(samples)
+        r = None if r is None else r.contiguous()
         ebar = torch.empty(ns, dtype=torch.float64, device=eloc.device)
         out2 = torch.empty(2, dtype=torch.float64, device=eloc.device)
         _lib.call("qtx_ebar", _lib.stream(), eloc.data_ptr(), _lib.ptr(r), ns, ebar.data_ptr(), out2.data_ptr())
@@ -285,7 +294,7 @@ class _MomentumSR(SR):
     def get_step(self, samples) -> torch.Tensor:
         ebar = self.get_Ebar(samples)
         O, mean = self.get_Obar(samples)
-        r = None if samples.reweight_factor is None or self._trivial_r(samples) else samples.reweight_factor
+        r = self._weights(samples)
         return self.solve(O, mean, ebar, r)
 
     def _sr(self, O, mean, ebar, r):

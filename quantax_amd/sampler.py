@@ -156,9 +156,9 @@ class Metropolis:
         if uses_ref:
             # local-update drift check and replacement by the full forward (metropolis.py:201-213)
             full = model.logpsi(self._spins)
-            close = (torch.abs(torch.exp(self._logabs) - torch.exp(full)) < 1e-8) | (
-                torch.abs(torch.exp(self._logabs - full) - 1) < 1e-3)
-            ndiff = int((~close).sum().item())
+            count = torch.empty(1, dtype=torch.int32, device=full.device)
+            _lib.call("qtx_drift_count", _lib.stream(), self._logabs.data_ptr(), full.data_ptr(), ns, count.data_ptr())
+            ndiff = int(count.item())
             self.last_drift = ndiff
             if ndiff > 0:
                 warn(f"{ndiff} out of {ns} wavefunctions are not close in direct forward pass and local updates.")
