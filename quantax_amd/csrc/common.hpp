@@ -101,6 +101,12 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
+__device__ __forceinline__ double readlane_f64(double v, int l) {
+  const int2 u = __builtin_bit_cast(int2, v);
+  const int2 s = int2{__builtin_amdgcn_readlane(u.x, l), __builtin_amdgcn_readlane(u.y, l)};
+  return __builtin_bit_cast(double, s);
+}
+
 // ---------------------------------------------------------------- math
 __device__ __forceinline__ float logcosh(float x) {
   float ax = fabsf(x);
@@ -154,6 +160,13 @@ __host__ __device__ __forceinline__ double words_to_uniform(uint32_t w2, uint32_
   return (double)(v >> 11) * 1.1102230246251565404e-16;
 }
 
+// log(u) of the acceptance test (metropolis.py:291-322) in FP64, kept out of
+// line: inlined, the constants of FP64 log1p would be hoisted into VGPRs for
+// the whole kernel
+static __device__ __noinline__ double accept_threshold(uint32_t w2, uint32_t w3) {
+  return log1p(-words_to_uniform(w2, w3));
+}
+
 constexpr uint32_t TAG_SWEEP = 0x51A7u;
 constexpr uint32_t TAG_INIT = 0x1D17u;
 
@@ -201,6 +214,21 @@ __device__ __forceinline__ void propose_move(int kind, const int8_t* sl, int N, 
   fa = site;
   fb = nb;
   updated = true;
+}
+
+// the sites of sl that hold `hopping`, in order, into pos (wave-cooperative LDS);
+// returns their number
+__device__ __forceinline__ int list_sites(const int8_t* sl, int N, int hopping, uint16_t* pos, int lane) {
+  int n = 0;
+  for (int base = 0; base < N; base += WAVE) {
+    const int i = base + lane;
+    const bool is_hop = (i < N) && (sl[i] == hopping);
+    const uint64_t m = __ballot(is_hop);
+    if (is_hop) pos[n + __popcll(m & ((1ull << lane) - 1))] = (uint16_t)i;
+    n += __popcll(m);
+  }
+  wave_lds_fence();
+  return n;
 }
 
 // ---------------------------------------------------------------- operator tables

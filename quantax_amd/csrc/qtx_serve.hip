@@ -58,11 +58,12 @@ __global__ __launch_bounds__(256) void rbm_group_logpsi_kernel(const qtx_rbm_job
 }
 
 template <int R>
-__global__ __launch_bounds__(256) void rbm_group_metropolis_kernel(const qtx_rbm_job* __restrict__ jobs,
+__global__ __launch_bounds__(256, R <= 8 ? 4 : 1) void rbm_group_metropolis_kernel(const qtx_rbm_job* __restrict__ jobs,
                                                                    const int32_t* __restrict__ idx,
                                                                    const int64_t* __restrict__ vstart, int cnt,
                                                                    int64_t nv) {
   __shared__ int8_t sbuf[WAVES_PER_BLOCK][MAXN];
+  __shared__ uint16_t pbuf[WAVES_PER_BLOCK][MAXN];
   const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
   for (int64_t v = blockIdx.x; v < nv; v += gridDim.x) {
     const int j = g_find(vstart, cnt, v);
@@ -77,7 +78,7 @@ __global__ __launch_bounds__(256) void rbm_group_metropolis_kernel(const qtx_rbm
       return make_uint4(r.x, r.y, r.z, r.w);
     };
     rbm_chain_metropolis<float, R>(J.packed, J.M, J.N, J.kind, J.nbr, J.width, J.hopping, J.nsteps, getw,
-                                   J.reweight, J.tie_tol, J.s + c * J.N, sbuf[wv], lane, J.logabs + c,
+                                   J.reweight, J.tie_tol, J.s + c * J.N, sbuf[wv], pbuf[wv], lane, J.logabs + c,
                                    J.n_accept + c, J.n_near + c);
   }
 }

@@ -1698,12 +1698,6 @@ constexpr int CT = 64;
 constexpr int CL = 80;       // LDS stride of a tile's columns: the four columns of a fragment fall on distinct banks
 constexpr int CI = 18;       // LDS stride of the columns of an inverted 16 x 16 block
 
-__device__ __forceinline__ double readlane_f64(double v, int l) {
-  const int2 u = __builtin_bit_cast(int2, v);
-  const int2 s = int2{__builtin_amdgcn_readlane(u.x, l), __builtin_amdgcn_readlane(u.y, l)};
-  return __builtin_bit_cast(double, s);
-}
-
 // 1 / sqrt(d), d > 0: the hardware's estimate (relative error < 2^-23) and one
 // third-order step; four dependent operations instead of a division after a
 // square root, which every column of a factorisation waits for

@@ -201,13 +201,6 @@ __device__ __forceinline__ void mfma_settle(v4f* acc) {
   for (int i = 0; i < N; ++i) asm volatile("" : "+v"(acc[i]));
 }
 
-// log(u) of the acceptance test (metropolis.py:291-322) in FP64, kept out of
-// line: inlined, the constants of FP64 log1p would be hoisted into VGPRs for
-// the whole kernel
-static __device__ __noinline__ double accept_threshold(uint32_t w2, uint32_t w3) {
-  return log1p(-words_to_uniform(w2, w3));
-}
-
 // psi(s') / psi(s) = e^d for the local energy: 2^t, t = d log2(e), split
 // into an integer k applied exactly by ldexp and f = t - k in [-1/2, 1/2]
 // whose 2^f is one FP32 exp2 (about 1 ulp); the FP64 product d log2(e) and
