@@ -155,7 +155,7 @@ __global__ void rbm_pack_kernel(const T* __restrict__ theta, int M, int N, T* __
 }
 
 template <typename T, int R>
-__global__ __launch_bounds__(256) void rbm_logpsi_kernel(const T* __restrict__ packed, int M, int N,
+__global__ __launch_bounds__(256, sizeof(T) == 4 && R <= 8 ? 4 : 1) void rbm_logpsi_kernel(const T* __restrict__ packed, int M, int N,
                                                          const int8_t* __restrict__ s, int64_t ns,
                                                          double* __restrict__ logabs, T* __restrict__ h_out) {
   __shared__ int8_t sbuf[WAVES_PER_BLOCK][MAXN];
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256) void rbm_logpsi_kernel(const T* __restrict__ p
 }
 
 template <typename T, int R>
-__global__ __launch_bounds__(256) void rbm_metropolis_kernel(
+__global__ __launch_bounds__(256, sizeof(T) == 4 && R <= 8 ? 4 : 1) void rbm_metropolis_kernel(
     const T* __restrict__ packed, int M, int N, int kind, const int32_t* __restrict__ nbr, int width,
     int hopping, const uint32_t* __restrict__ words, int nsteps, int64_t ns, double reweight, double tie_tol,
     int8_t* __restrict__ s, double* __restrict__ logabs, int32_t* __restrict__ n_accept,
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void rbm_metropolis_kernel(
 }
 
 template <typename T, int R>
-__global__ __launch_bounds__(256) void rbm_eloc_kernel(const T* __restrict__ packed, int M, int N, qtx_ham H,
+__global__ __launch_bounds__(256, sizeof(T) == 4 && R <= 8 ? 4 : 1) void rbm_eloc_kernel(const T* __restrict__ packed, int M, int N, qtx_ham H,
                                                        const int8_t* __restrict__ s, int64_t ns,
                                                        double* __restrict__ eloc, int32_t* __restrict__ nconn) {
   __shared__ int8_t sbuf[WAVES_PER_BLOCK][MAXN];

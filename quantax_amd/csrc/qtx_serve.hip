@@ -42,7 +42,7 @@ __device__ __forceinline__ int g_find(const int64_t* __restrict__ vstart, int cn
 }
 
 template <int R>
-__global__ __launch_bounds__(256) void rbm_group_logpsi_kernel(const qtx_rbm_job* __restrict__ jobs,
+__global__ __launch_bounds__(256, R <= 8 ? 4 : 1) void rbm_group_logpsi_kernel(const qtx_rbm_job* __restrict__ jobs,
                                                                const int32_t* __restrict__ idx,
                                                                const int64_t* __restrict__ vstart, int cnt,
                                                                int64_t nv) {
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256, R <= 8 ? 4 : 1) void rbm_group_metropolis_kern
 }
 
 template <int R>
-__global__ __launch_bounds__(256) void rbm_group_eloc_kernel(const qtx_rbm_job* __restrict__ jobs,
+__global__ __launch_bounds__(256, R <= 8 ? 4 : 1) void rbm_group_eloc_kernel(const qtx_rbm_job* __restrict__ jobs,
                                                              const int32_t* __restrict__ idx,
                                                              const int64_t* __restrict__ vstart, int cnt,
                                                              int64_t nv) {
