@@ -212,51 +212,53 @@ __device__ __forceinline__ void super_tile_of(int t, int mt, int& bi, int& bj) {
 
 // FP64 / FP32 Gram on 16x16x4 MFMA.  The FP64 matrix pipe takes 64 cycles per
 // instruction, so LDS and L2 have room for a small tile: 64 x 64 per
-// workgroup (four waves of 32 x 32), four workgroups per CU, which leaves the
-// last round of a 4096-row Gram (2080 tiles on 256 CUs) 90 % full; a 128 x 128
-// tile would leave it at 69 %.  A thread stages four consecutive columns of
-// one row of each operand per 16-column chunk: one four-element load of O
-// (which needs only the element's own alignment, so any np takes it), fetched
-// one chunk ahead into registers and centred in FP64 (the rows' factors are
-// applied to the sums), then written to the other of two LDS buffers: one
-// barrier per chunk.  FP64, 4096 x 40400: 44.3 -> 12.9 ms; 4096 x 34952: 38.3
-// -> 11.2 ms; 16384 x 34952: 331 -> 156 ms (60 TFLOP/s, a library f64 GEMM
+// workgroup (four waves of 32 x 32), four workgroups per CU; a 128 x 128 tile
+// would leave the last round of a 4096-row Gram 69 % full.  A thread stages
+// four consecutive columns of one row of each operand per 16-column chunk: one
+// four-element load of O (which needs only the element's own alignment, so any
+// np takes it), fetched one chunk ahead into registers and centred in FP64 (the
+// rows' factors are applied to the sums), then written to the other of two LDS
+// buffers: one barrier per chunk.  FP64, 4096 x 40400: 44.3 -> 11.7 ms; 4096 x 34952: 38.3
+// -> 10.2 ms; 16384 x 34952: 331 -> 154 ms (60 TFLOP/s, a library f64 GEMM
 // reaches 73).  The matrix pipe is busy 80 % of the time (SQ counters); the
 // FP64 conversions and subtractions, one per MFMA, are most of the rest.
 constexpr int GN_T = 64;    // tile
 constexpr int GN_KC = 16;   // columns per chunk
 constexpr int GN_LD = GN_KC + 1;
 
-template <typename TI, int G>
-__global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ O, const double* __restrict__ mean,
-                                                         const double* __restrict__ r, int64_t n, int64_t np,
-                                                         double inv_ns, int ntiles, double* __restrict__ T) {
-  using ST = typename std::conditional<G == QTX_GRAM_FP64, double, float>::type;
+// one S x S tile (64 or 32) at (i0, j0) by four waves of S/2 x S/2; As, Bs:
+// 2 S GN_LD elements each
+template <typename TI, int G, int S, typename ST>
+__device__ __forceinline__ void gram_nt_tile(const TI* __restrict__ O, const double* __restrict__ mean,
+                                             const double* __restrict__ r, int64_t n, int64_t np, double inv_ns,
+                                             int64_t i0, int64_t j0, ST* As, ST* Bs, double* __restrict__ T) {
+  constexpr int NB = S / 32;  // 16 x 16 blocks per wave and side
   using ACC = typename std::conditional<G == QTX_GRAM_FP64, v4d, v4f>::type;
   typedef TI vt4 __attribute__((ext_vector_type(4), aligned(sizeof(TI))));
-  __shared__ ST As[2][GN_T * GN_LD];
-  __shared__ ST Bs[2][GN_T * GN_LD];
-  int bi, bj;
-  super_tile_of(xcd_tile(blockIdx.x, ntiles), (int)((n + GN_T - 1) / GN_T), bi, bj);
-  const int64_t i0 = (int64_t)bi * GN_T, j0 = (int64_t)bj * GN_T;
   const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
-  const int wr = (wv / 2) * 32, wc = (wv % 2) * 32;  // wave's sub-tile origin
-  // staging: row tid / 4, columns 4 (tid % 4) .. + 3; rows past n repeat row
-  // n - 1 (their outputs are not stored)
-  const int srow = tid / 4, sk = (tid % 4) * 4;
+  const int wr = (wv / 2) * (S / 2), wc = (wv % 2) * (S / 2);  // wave's sub-tile origin
+  // staging: columns 4 (tid % 4) .. + 3 of one row; S = 64: row tid / 4 of both
+  // operands, S = 32: row tid / 4 % 32 of the first (tid < 128) or the second.
+  // Rows past n repeat row n - 1 (their outputs are not stored)
+  const int srow = tid / 4 % S, sk = (tid % 4) * 4;
+  const bool second = S == 32 && tid >= 128;
   const int64_t ra = i0 + srow < n ? i0 + srow : n - 1, rb = j0 + srow < n ? j0 + srow : n - 1;
-  const TI* pa = O + ra * np;
+  const TI* pa = O + (second ? rb : ra) * np;
   const TI* pb = O + rb * np;
+  ST* sa = (second ? Bs : As) + srow * GN_LD + sk;
+  ST* sb = Bs + srow * GN_LD + sk;
   TI av[4], bv[4];
   double mv[4];
   auto fetch = [&](int64_t k0) {
     const int64_t k = k0 + sk;
     if (k + 3 < np) {
-      const vt4 x = *reinterpret_cast<const vt4*>(pa + k), y = *reinterpret_cast<const vt4*>(pb + k);
+      const vt4 x = *reinterpret_cast<const vt4*>(pa + k);
+      vt4 y;
+      if (S == 64) y = *reinterpret_cast<const vt4*>(pb + k);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         av[q] = x[q];
-        bv[q] = y[q];
+        if (S == 64) bv[q] = y[q];
         mv[q] = mean[k + q];
       }
     } else {
@@ -264,7 +266,7 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
       for (int q = 0; q < 4; ++q) {
         const bool ok = k + q < np;
         av[q] = ok ? pa[k + q] : TI(0);
-        bv[q] = ok ? pb[k + q] : TI(0);
+        if (S == 64) bv[q] = ok ? pb[k + q] : TI(0);
         mv[q] = ok ? mean[k + q] : 0.0;
       }
     }
@@ -272,26 +274,26 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
   auto stage = [&](int buf) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      As[buf][srow * GN_LD + sk + q] = (ST)((double)av[q] - mv[q]);
-      Bs[buf][srow * GN_LD + sk + q] = (ST)((double)bv[q] - mv[q]);
+      sa[buf * S * GN_LD + q] = (ST)((double)av[q] - mv[q]);
+      if (S == 64) sb[buf * S * GN_LD + q] = (ST)((double)bv[q] - mv[q]);
     }
   };
 
-  ACC acc[2][2];
+  ACC acc[NB][NB];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < NB; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = ACC{0, 0, 0, 0};
+    for (int b = 0; b < NB; ++b) acc[a][b] = ACC{0, 0, 0, 0};
   // the FP32 mode flushes its MFMA accumulators into FP64 every FLUSH chunks
   // (256 columns), so the rounding error does not grow with np
   constexpr int FLUSH = 256 / GN_KC;
   constexpr bool SHADOW = (G != QTX_GRAM_FP64);
-  v4d dacc[SHADOW ? 2 : 1][SHADOW ? 2 : 1];
+  v4d dacc[SHADOW ? NB : 1][SHADOW ? NB : 1];
   if constexpr (SHADOW) {
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < NB; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) dacc[a][b] = v4d{0, 0, 0, 0};
+      for (int b = 0; b < NB; ++b) dacc[a][b] = v4d{0, 0, 0, 0};
   }
 
   const int nchunks = (int)((np + GN_KC - 1) / GN_KC);
@@ -299,21 +301,21 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
   stage(0);
   __syncthreads();
   for (int c = 0; c < nchunks; ++c) {
-    const ST* Ac = As[c & 1];
-    const ST* Bc = Bs[c & 1];
+    const ST* Ac = As + (c & 1) * S * GN_LD;
+    const ST* Bc = Bs + (c & 1) * S * GN_LD;
     if (c + 1 < nchunks) fetch((int64_t)(c + 1) * GN_KC);
 #pragma unroll
     for (int ks = 0; ks < GN_KC; ks += 4) {
-      ST af[2], bf[2];
+      ST af[NB], bf[NB];
 #pragma unroll
-      for (int a = 0; a < 2; ++a) {
+      for (int a = 0; a < NB; ++a) {
         af[a] = Ac[(wr + a * 16 + lane % 16) * GN_LD + ks + lane / 16];
         bf[a] = Bc[(wc + a * 16 + lane % 16) * GN_LD + ks + lane / 16];
       }
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
+      for (int a = 0; a < NB; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < NB; ++b) {
           if constexpr (G == QTX_GRAM_FP64)
             acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[a], bf[b], acc[a][b], 0, 0, 0);
           else
@@ -323,9 +325,9 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
     if constexpr (SHADOW) {
       if ((c + 1) % FLUSH == 0 || c + 1 == nchunks) {
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+        for (int a = 0; a < NB; ++a)
 #pragma unroll
-          for (int b = 0; b < 2; ++b) {
+          for (int b = 0; b < NB; ++b) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) dacc[a][b][q] += (double)acc[a][b][q];
             acc[a][b] = ACC{0, 0, 0, 0};
@@ -339,9 +341,9 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
   // store, column lane%16 of each 16x16 block; rows of element q:
   //   f32 MFMA: 4 * (lane / 16) + q ;  f64 MFMA: lane / 16 + 4 * q
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < NB; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int rq = (G == QTX_GRAM_FP64) ? (lane / 16 + 4 * q) : (4 * (lane / 16) + q);
@@ -349,7 +351,7 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
         const int64_t gj = j0 + wc + b * 16 + lane % 16;
         // off-diagonal tiles are mirrored; inside diagonal tiles the lower
         // triangle is written to both halves so T is exactly symmetric
-        if (gi < n && gj < n && (bi != bj || gi >= gj)) {
+        if (gi < n && gj < n && (i0 != j0 || gi >= gj)) {
           double v;
           if constexpr (SHADOW)
             v = dacc[a][b][q];
@@ -360,6 +362,38 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
           T[gj * n + gi] = v;
         }
       }
+}
+
+// 32 CUs per XCD take a tile each at a time (four resident at once, so the last
+// ones of an XCD's run would end alone on their CUs, one wave per SIMD).  Where
+// at most 16 tiles are left over after whole rounds, those are dealt out as 32 x
+// 32 quarters, with the same sums: 4096 x 40400 (260 tiles per XCD) 12.9 -> 11.7
+// ms, 4096 x 34952 11.2 -> 10.2 ms.
+// Few rows (less than a round per XCD) spread over four times the CUs.
+__host__ __device__ inline int gram_whole(int per) { return per % 32 <= 16 ? per / 32 * 32 : per; }
+
+template <typename TI, int G>
+__global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ O, const double* __restrict__ mean,
+                                                         const double* __restrict__ r, int64_t n, int64_t np,
+                                                         double inv_ns, int ntiles, double* __restrict__ T) {
+  using ST = typename std::conditional<G == QTX_GRAM_FP64, double, float>::type;
+  __shared__ ST As[2 * GN_T * GN_LD];
+  __shared__ ST Bs[2 * GN_T * GN_LD];
+  const int x = blockIdx.x % 8, loc = blockIdx.x / 8, per = (ntiles + 7) / 8, whole = gram_whole(per);
+  const int tile = loc < whole ? loc : whole + (loc - whole) / 4;
+  const int first = xcd_tile(x, ntiles), mine = ntiles / 8 + (x < ntiles % 8 ? 1 : 0);
+  if (tile >= mine) return;
+  int bi, bj;
+  super_tile_of(first + tile, (int)((n + GN_T - 1) / GN_T), bi, bj);
+  int64_t i0 = (int64_t)bi * GN_T, j0 = (int64_t)bj * GN_T;
+  if (loc < whole) {
+    gram_nt_tile<TI, G, 64>(O, mean, r, n, np, inv_ns, i0, j0, As, Bs, T);
+  } else {
+    i0 += (loc - whole) / 2 % 2 * 32;
+    j0 += (loc - whole) % 2 * 32;
+    if (i0 < j0 || i0 >= n || j0 >= n) return;  // above the diagonal, or past the end
+    gram_nt_tile<TI, G, 32>(O, mean, r, n, np, inv_ns, i0, j0, As, Bs, T);
+  }
 }
 
 // ---------------------------------------------------------------- split-bf16 Gram
@@ -1574,7 +1608,8 @@ static int launch_gram_nt(hipStream_t st, int gram, const TI* O, const double* m
   } else {
     const int64_t mt = (n + GN_T - 1) / GN_T, mtiles = mt * (mt + 1) / 2;
     QTX_REQUIRE(mtiles < 0x7fffffff, "Gram too large");
-    const dim3 gm((unsigned)mtiles);
+    const int64_t per = (mtiles + 7) / 8, whole = gram_whole((int)per);
+    const dim3 gm((unsigned)(8 * (whole + 4 * (per - whole))));
     if (gram == QTX_GRAM_FP32)
       hipLaunchKernelGGL((gram_nt_kernel<TI, QTX_GRAM_FP32>), gm, bl, 0, st, O, mean, r, n, np, inv_ns, (int)mtiles, T);
     else
