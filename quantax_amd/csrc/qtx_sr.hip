@@ -398,16 +398,19 @@ __global__ __launch_bounds__(256, 4) void gram_nt_kernel(const TI* __restrict__ 
 
 // ---------------------------------------------------------------- split-bf16 Gram
 // Pre-pass: Obar = (O - mean) sqrt(r / ns) in FP64, rounded to FP32 x and
-// split into bf16 planes hi = bf16(x), lo = bf16(x - hi), row-major with rows
-// padded to a multiple of GT and K to a multiple of G3_KC (zeros).  The Gram
-// kernel then streams the planes straight into LDS and does only MFMA work:
-// T_ij = sum_k lo_i hi_j + hi_i lo_j + hi_i hi_j (lo * lo dropped).
-constexpr int G3_KC = 64;            // K per LDS stage (two 16x16x32 MFMA steps)
-constexpr int G3_FLUSH = 4;          // stages per FP32 -> FP64 flush (256 K)
-constexpr int G3_PLANE = GT * G3_KC * 2;  // bytes of one bf16 plane of one stage (16 KB)
+// split into bf16 parts hi = bf16(x), lo = bf16(x - hi): per row, 32 hi then their
+// 32 lo (one 128-byte line per K step), rows padded to a multiple of GT and K to
+// a multiple of G3_KPAD (zeros).  The Gram kernel then streams the parts straight
+// into LDS and does only MFMA work: T_ij = sum_k lo_i hi_j + hi_i lo_j + hi_i hi_j
+// (lo * lo dropped).
+constexpr int G3_KC = 32;            // K per LDS stage (one 16x16x32 MFMA step)
+constexpr int G3_FLUSH = 8;          // stages per FP32 -> FP64 flush (256 K)
+constexpr int G3_ROW = 2 * G3_KC * 2;     // bytes of a row's hi and lo parts of one stage (a 128-byte line)
+constexpr int G3_OPER = GT * G3_ROW;      // bytes of one operand of one stage (16 KB)
+constexpr int G3_KPAD = 64;
 
 static inline int64_t g3_rows(int64_t n) { return (n + GT - 1) / GT * GT; }
-static inline int64_t g3_kpad(int64_t np) { return (np + G3_KC - 1) / G3_KC * G3_KC; }
+static inline int64_t g3_kpad(int64_t np) { return (np + G3_KPAD - 1) / G3_KPAD * G3_KPAD; }
 static inline size_t g3_bytes(int64_t n, int64_t np) { return (size_t)g3_rows(n) * g3_kpad(np) * 2 * sizeof(__bf16); }
 
 // Grid-stride over (row, 256-column block) pairs: a launch's work-item count
@@ -416,7 +419,7 @@ template <typename TI>
 __global__ __launch_bounds__(256) void split_bf16x3_kernel(const TI* __restrict__ O, const double* __restrict__ mean,
                                                            const double* __restrict__ r, int64_t n, int64_t np,
                                                            int64_t kpad, int64_t bpr, int64_t nblocks, double inv_ns,
-                                                           __bf16* __restrict__ Hi, __bf16* __restrict__ Lo) {
+                                                           __bf16* __restrict__ HL) {
   for (int64_t blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
     const int64_t row = blk / bpr;
     const int64_t k = (blk % bpr) * 256 + threadIdx.x;
@@ -425,40 +428,47 @@ __global__ __launch_bounds__(256) void split_bf16x3_kernel(const TI* __restrict_
     if (row < n && k < np) v = ((double)O[row * np + k] - mean[k]) * sqrt((r ? r[row] : 1.0) * inv_ns);
     const float f = (float)v;
     const __bf16 hi = (__bf16)f;
-    Hi[row * kpad + k] = hi;
-    Lo[row * kpad + k] = (__bf16)(f - (float)hi);
+    __bf16* p = HL + 2 * (row * kpad + k / G3_KC * G3_KC) + k % G3_KC;
+    p[0] = hi;
+    p[G3_KC] = (__bf16)(f - (float)hi);
   }
 }
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-// 128 x 128 tile, 4 waves (2 x 2, 64 x 64 each).  Operands move HBM -> LDS by
-// LDS DMA (global_load_lds_dwordx4: lane l of a wave writes 16 bytes at the
-// wave's LDS base + 16 l), two 64 KB stages so chunk c + 1 is in flight while
-// chunk c is multiplied.  Wave w fetches plane w (A hi, A lo, B hi, B lo).  A
-// plane is 128 rows x 128 bytes; the 16-byte segment s of row r sits in slot
-// s ^ (r & 7), so the MFMA fragment reads (16 rows, one segment) hit 8
-// distinct slots per 8 lanes: no bank conflicts.  The stage barriers are raw
-// s_barrier with explicit vmcnt waits: a __syncthreads() fence would drain
-// the next chunk's DMA as well.
-__global__ __launch_bounds__(256) void gram_bf16x3_kernel(const __bf16* __restrict__ Hi,
-                                                          const __bf16* __restrict__ Lo, int64_t n, int64_t kpad,
-                                                          int ntiles, double* __restrict__ T) {
-  __shared__ __attribute__((aligned(16))) char smem[2 * 4 * G3_PLANE];
+// 128 x 128 tile, 4 waves (2 x 2, 64 x 64 each), two workgroups per CU so that one
+// multiplies while the other waits.  Operands move HBM -> LDS by LDS DMA
+// (global_load_lds_dwordx4: lane l of a wave writes 16 bytes at the wave's LDS
+// base + 16 l), two 32 KB stages so chunk c + 1 is in flight while chunk c is
+// multiplied.  A row of a stage is one line, hi and lo of 32 K; its 16-byte
+// segment s (hi 0-3, lo 4-7) sits in slot s ^ (r & 7), so the MFMA fragment reads
+// (16 rows, one segment) hit 8 distinct slots per 8 lanes: no bank conflicts.
+// The stage barriers are raw s_barrier with explicit vmcnt waits: a
+// __syncthreads() fence would drain the next chunk's DMA as well.
+// Bound by L2 misses at large n: the 64 tiles an XCD runs together (an 8 x 8
+// super-block) drift apart in K by more than its L2 holds, 154 GB at 4.3 TB/s for
+// 16384 x 34952, where 37 GB would do.  16384 x 34952 with the pass above: 41.7 ->
+// 38.9 ms; 8192: 9.8 ms, 4096: 3.9 -> 3.0 ms (one workgroup per CU with separate
+// planes and K = 64 stages before; half-line stages, 64 bytes per row and plane,
+// took 46.5 ms at 16384).
+__global__ __launch_bounds__(256, 2) void gram_bf16x3_kernel(const __bf16* __restrict__ HL, int64_t n, int64_t kpad,
+                                                             int ntiles, double* __restrict__ T) {
+  __shared__ __attribute__((aligned(16))) char smem[2 * 2 * G3_OPER];
   int bi, bj;
   super_tile_of(xcd_tile(blockIdx.x, ntiles), (int)((n + GT - 1) / GT), bi, bj);
   const int64_t i0 = (int64_t)bi * GT, j0 = (int64_t)bj * GT;
   const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
   const int wr = (wv / 2) * 64, wc = (wv % 2) * 64;
-  const __bf16* src = (wv == 0) ? Hi + i0 * kpad : (wv == 1) ? Lo + i0 * kpad : (wv == 2) ? Hi + j0 * kpad : Lo + j0 * kpad;
-  // one DMA instruction covers rows 8q .. 8q+7: lane l -> row 8q + l/8, slot l%8,
-  // which holds logical segment (l%8) ^ (l/8)
+  // wave w fetches rows 64 (w % 2) .. of the first (w < 2) or the second operand.
+  // One DMA instruction covers rows 8 q .. 8 q + 7: lane l -> row 8 q + l / 8, slot
+  // l % 8, which holds logical segment (l % 8) ^ (l / 8)
   const int lrow = lane / 8, lseg = (lane % 8) ^ (lane / 8);
+  const __bf16* src = HL + 2 * ((wv < 2 ? i0 : j0) + 64 * (wv % 2) + lrow) * kpad + lseg * 8;
   auto issue = [&](int64_t k0, int stage) {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const __bf16* g = src + (int64_t)(q * 8 + lrow) * kpad + k0 + lseg * 8;
-      char* dst = smem + (stage * 4 + wv) * G3_PLANE + q * 1024;
+    for (int q = 0; q < 8; ++q) {
+      const __bf16* g = src + 2 * (q * 8 * kpad + k0);
+      char* dst = smem + (stage * 2 + wv / 2) * G3_OPER + (wv % 2) * (G3_OPER / 2) + q * 1024;
       __builtin_amdgcn_global_load_lds((const void*)g, (lds_void*)dst, 16, 0, 0);
     }
   };
@@ -476,41 +486,32 @@ __global__ __launch_bounds__(256) void gram_bf16x3_kernel(const __bf16* __restri
   issue(0, 0);
   if (nchunks > 1) issue(G3_KC, 1);
   for (int c = 0; c < nchunks; ++c) {
-    // this wave's DMA for chunk c is done (16 newer ones may be in flight), then
+    // this wave's DMA for chunk c is done (8 newer ones may be in flight), then
     // every wave's is
     if (c + 1 < nchunks)
-      asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
+      asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
     else
       asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    const char* stg = smem + (c & 1) * 4 * G3_PLANE;
+    const char* stg = smem + (c & 1) * 2 * G3_OPER;
+    const int hs = ((lane / 16) ^ (lane & 7)) * 16, ls = hs ^ 64;  // slots of hi and lo, the same for every 16-row block
+    v8bf bh[4], bl[4];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      v8bf ah[4], al[4], bh[4], bl[4];
+    for (int b = 0; b < 4; ++b) {
+      const char* row = stg + G3_OPER + (wc + b * 16 + lane % 16) * G3_ROW;
+      bh[b] = *(const v8bf*)(row + hs);
+      bl[b] = *(const v8bf*)(row + ls);
+    }
 #pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const int row = wr + a * 16 + lane % 16, slot = (ks * 4 + lane / 16) ^ (row & 7);
-        ah[a] = *(const v8bf*)(stg + 0 * G3_PLANE + row * 128 + slot * 16);
-        al[a] = *(const v8bf*)(stg + 1 * G3_PLANE + row * 128 + slot * 16);
-      }
+    for (int a = 0; a < 4; ++a) {
+      const char* row = stg + (wr + a * 16 + lane % 16) * G3_ROW;
+      const v8bf ah = *(const v8bf*)(row + hs), al = *(const v8bf*)(row + ls);
+      // the three products of a block are 4 MFMAs apart (no back-to-back dependency)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int row = wc + b * 16 + lane % 16, slot = (ks * 4 + lane / 16) ^ (row & 7);
-        bh[b] = *(const v8bf*)(stg + 2 * G3_PLANE + row * 128 + slot * 16);
-        bl[b] = *(const v8bf*)(stg + 3 * G3_PLANE + row * 128 + slot * 16);
-      }
-      // the three products of a block are 16 MFMAs apart (no back-to-back dependency)
+      for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[b], acc[a][b], 0, 0, 0);
 #pragma unroll
-      for (int a = 0; a < 4; ++a)
+      for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl[b], acc[a][b], 0, 0, 0);
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[a], bh[b], acc[a][b], 0, 0, 0);
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[a], bl[b], acc[a][b], 0, 0, 0);
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[a], bh[b], acc[a][b], 0, 0, 0);
+      for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh[b], acc[a][b], 0, 0, 0);
     }
     if ((c + 1) % G3_FLUSH == 0 || c + 1 == nchunks) {
 #pragma unroll
@@ -1599,12 +1600,10 @@ static int launch_gram_nt(hipStream_t st, int gram, const TI* O, const double* m
     QTX_REQUIRE(split_ws != nullptr, "split-bf16 Gram needs its workspace");
     const int64_t rows = g3_rows(n), kpad = g3_kpad(np), bpr = (kpad + 255) / 256;
     const int64_t nblocks = rows * bpr;
-    __bf16* Hi = (__bf16*)split_ws;
-    __bf16* Lo = Hi + rows * kpad;
+    __bf16* HL = (__bf16*)split_ws;
     hipLaunchKernelGGL(split_bf16x3_kernel<TI>, dim3((unsigned)std::min<int64_t>(nblocks, kGridCap)), dim3(256), 0,
-                       st, O, mean, r, n, np, kpad, bpr, nblocks, inv_ns, Hi, Lo);
-    hipLaunchKernelGGL(gram_bf16x3_kernel, g, bl, 0, st, (const __bf16*)Hi, (const __bf16*)Lo, n, kpad, (int)ntiles,
-                       T);
+                       st, O, mean, r, n, np, kpad, bpr, nblocks, inv_ns, HL);
+    hipLaunchKernelGGL(gram_bf16x3_kernel, g, bl, 0, st, (const __bf16*)HL, n, kpad, (int)ntiles, T);
   } else {
     const int64_t mt = (n + GN_T - 1) / GN_T, mtiles = mt * (mt + 1) / 2;
     QTX_REQUIRE(mtiles < 0x7fffffff, "Gram too large");
