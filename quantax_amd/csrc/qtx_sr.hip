@@ -1136,6 +1136,18 @@ __global__ __launch_bounds__(256) void cheb_rows_kernel(const double* __restrict
   }
 }
 
+// p: 2 H values per lane, summed over lane pairs S H apart; lanes with that bit
+// set keep the upper half of the values
+template <int H, int S>
+__device__ __forceinline__ void halve_columns(double* p, int lane) {
+  const bool up = lane & (S * H);
+#pragma unroll
+  for (int i = 0; i < H; ++i) {
+    const double keep = up ? p[i + H] : p[i], send = up ? p[i] : p[i + H];
+    p[i] = keep + __shfl_xor(send, S * H, WAVE);
+  }
+}
+
 // One read of a triangle for both of its products (n <= kTriPassMax).  A
 // workgroup of 512 threads (one per CU) takes rows c of the lower triangle
 // (row-major, columns j <= c), RB at a time: a thread holds the rows' columns
@@ -1154,13 +1166,13 @@ constexpr int TP_GRID = 256;  // one workgroup per CU (x fills most of the LDS)
 // last-level cache and the partial results cost more than the second read
 // (us, two reads | one and its sum):
 //   n      T x          P^T P x
-//   3000   13.8 | 18.2   20.5 | 20.8
-//   4096   21.5 | 23.7   30.4 | 26.8
-//   5000   34.2 | 32.0   41.8 | 37.5
-//   6144   46.8 | 38.6   59.2 | 44.5
-//   8192   84.5 | 57.7   98.7 | 63.0
+//   2560    9.8 | 16.4   17.2 | 16.9
+//   3072   12.2 | 17.6   21.1 | 17.9
+//   4096   21.6 | 21.7   30.2 | 22.6
+//   5000   34.2 | 30.6   41.8 | 33.1
+//   8192   84.5 | 56.8   98.7 | 60.3
 //   16384   329 |  216    360 |  223  (1.07 GB: 5.0 TB/s)
-constexpr int64_t kTriPassSymMin = 4608, kTriPassMin = 3072, kTriPassMax = 16384;
+constexpr int64_t kTriPassSymMin = 4608, kTriPassMin = 2560, kTriPassMax = 16384;
 typedef double v2d_u __attribute__((ext_vector_type(2), aligned(8)));
 
 template <int NC>
@@ -1200,22 +1212,27 @@ __global__ __launch_bounds__(TP_THREADS) void tri_pass_kernel(const double* __re
   auto use = [&](int turn, v2d_u (&b)[RB][NC]) {
     asm volatile("" ::: "memory");  // x is read from LDS in every turn, not kept in registers
     double* rd = red + (SYM ? turn : (turn & 1)) * RB * TP_WAVES;
+    double p[RB];
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
       int d = 2 * t - (int)row_of(turn, r);  // the diagonal is at column 2 t - d
       asm volatile("" : "+v"(d));
-      double p = 0.0;
+      p[r] = 0.0;
 #pragma unroll
       for (int i = 0; i < NC; ++i) {
-        if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // few of x's reads at a time
+        if (NC > 4 && i % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // few of x's reads at a time
         const double2 x2 = *reinterpret_cast<const double2*>(xs + 2 * t + 2 * TP_THREADS * i);
         if (d == -2 * TP_THREADS * i) b[r][i].y = 0.0;  // the second of the last pair, if there is one to read
         // the diagonal of T belongs to the row's multiple
-        p += (SYM && d == -2 * TP_THREADS * i ? 0.0 : b[r][i].x) * x2.x + (SYM && d == -2 * TP_THREADS * i - 1 ? 0.0 : b[r][i].y) * x2.y;
+        p[r] += (SYM && d == -2 * TP_THREADS * i ? 0.0 : b[r][i].x) * x2.x +
+                (SYM && d == -2 * TP_THREADS * i - 1 ? 0.0 : b[r][i].y) * x2.y;
       }
-      p = wave_sum(p);
-      if (lane == 0) rd[r * TP_WAVES + wv] = p;
     }
+    // the RB sums of a wave by one butterfly; row r ends in the r-th WAVE / RB lanes
+    if constexpr (RB == 4) halve_columns<2, 16>(p, lane);
+    if constexpr (RB >= 2) halve_columns<1, RB == 4 ? 16 : 32>(p, lane);
+    for (int q = WAVE / RB / 2; q >= 1; q /= 2) p[0] += __shfl_xor(p[0], q, WAVE);
+    if (lane % (WAVE / RB) == 0) rd[lane / (WAVE / RB) * TP_WAVES + wv] = p[0];
     double sums = 0.0;
     if (!SYM) {
       __syncthreads();
@@ -1225,7 +1242,7 @@ __global__ __launch_bounds__(TP_THREADS) void tri_pass_kernel(const double* __re
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
       const int64_t c = row_of(turn, r);
-      const double u = SYM ? (c < n ? xs[c] : 0.0) : __shfl(sums, r * TP_WAVES, WAVE);
+      const double u = SYM ? (c < n ? xs[c] : 0.0) : readlane_f64(sums, r * TP_WAVES);
 #pragma unroll
       for (int i = 0; i < NC; ++i) w[i] += u * b[r][i];
     }
@@ -2036,18 +2053,6 @@ __global__ __launch_bounds__(1024) void chol_fwd_gemv_kernel(const double* __res
   }
 }
 
-// p: 2 H column values per lane, summed over lane pairs 4 H apart; lanes with
-// that bit set keep the upper half of the columns
-template <int H>
-__device__ __forceinline__ void halve_columns(double* p, int lane) {
-  const bool up = lane & (4 * H);
-#pragma unroll
-  for (int i = 0; i < H; ++i) {
-    const double keep = up ? p[i + H] : p[i], send = up ? p[i] : p[i + H];
-    p[i] = keep + __shfl_xor(send, 4 * H, WAVE);
-  }
-}
-
 // One 64-row step of x = L^-T y from the last block up: x_b = L_bb^-T y_b, then
 // y_j -= L_bj^T x_b for the blocks j < b, one per workgroup.  Every workgroup
 // solves the 64 x 64 triangle (a chain of 64 lane reads; cheaper than a launch
@@ -2092,10 +2097,10 @@ __global__ __launch_bounds__(256) void chol_back_kernel(const double* __restrict
   const double xr = xb[lane];
 #pragma unroll
   for (int i = 0; i < 16; ++i) p[i] *= xr;
-  halve_columns<8>(p, lane);
-  halve_columns<4>(p, lane);
-  halve_columns<2>(p, lane);
-  halve_columns<1>(p, lane);
+  halve_columns<8, 4>(p, lane);
+  halve_columns<4, 4>(p, lane);
+  halve_columns<2, 4>(p, lane);
+  halve_columns<1, 4>(p, lane);
   double s = p[0];
   s += __shfl_xor(s, 1, WAVE);
   s += __shfl_xor(s, 2, WAVE);

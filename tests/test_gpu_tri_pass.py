@@ -1,5 +1,5 @@
 """The one-read triangle passes of the solver: the symmetric product of the
-Lanczos steps (n >= 4608) and P^T (P x) of the Chebyshev terms (n >= 3072), on
+Lanczos steps (n >= 4608) and P^T (P x) of the Chebyshev terms (n >= 2560), on
 both sides of their lines, at the edges of their column classes (n <= 4096,
 n <= 8192, above) and at odd n (rows that end inside a pair of columns and are
 not 16-byte aligned), with the register forms of the Lanczos step.
@@ -22,7 +22,7 @@ def _reflector(gen, n):
     return v / v.norm()
 
 
-@pytest.mark.parametrize("n", [3071, 3072, 3073, 4096, 4099, 4607, 4608, 8192, 8193, 9001])
+@pytest.mark.parametrize("n", [2559, 2560, 2561, 3073, 4096, 4099, 4607, 4608, 8192, 8193, 9001])
 def test_solve_closed_form(n):
     gen = torch.Generator(device="cuda").manual_seed(n)
     np_ = n + 7
