@@ -24,7 +24,6 @@ import time
 
 import numpy as np
 
-HBM_PEAK_GBS = 8000.0
 MFMA_PEAK = {"bf16": 2500.0, "fp32": 157.3, "fp64": 78.6}  # dense TFLOP/s
 
 
@@ -92,16 +91,6 @@ CONFIGS = {
                workload="J1-J2 20x20 (J2=0.5, MSR, Sz=0), ResConv(16 blocks, 32 ch), 32768 chains, MinSR "
                         "(T 32768^2); sampling cut to 8 proposals per chain, no thermalisation"),
 }
-
-
-# HBM traffic of one rc_metropolis_kernel launch at the 16x16 workload (mixed,
-# 512 steps, 16384 chains): NOT measured by this run.  It comes from two
-# rocprofv3 --pmc runs of this script (FETCH_SIZE, then WRITE_SIZE), each
-# scaled by what the counter reads for a 256 MiB device copy; the commands,
-# raw counts and the calibration are in the profile named below, and the
-# bench line reports the figure with that source.
-PMC_C3_MIXED = {"fetch_kib": 68745.5, "write_kib": 4352.0, "fetch_scale": 262144.0 / 131092.8125, "write_scale": 1.0,
-                "source": "profiles/rc_metropolis_16x16_c16_nb8_hbm_traffic.md"}
 
 
 def conv_flops_per_forward(nblocks, C, N):
@@ -484,12 +473,12 @@ def profile_kernels(cfg, args, torch, qtx):
     nconn = float(nc.float().mean().item())
     print(json.dumps({"profile": args.config, "mode": mode, "sweep_steps": args.sweep_steps, "chains": cfg["ns"],
                       "metropolis_ms": round(ms_sweep, 3),
-                      "metropolis_tflops": round(cfg["ns"] * args.sweep_steps * fwd / ms_sweep / 1e9, 1),
+                      "proposals_per_s": round(cfg["ns"] * args.sweep_steps / ms_sweep * 1e3),
                       "eloc_samples": n, "eloc_ms": round(ms_e, 3), "mean_nconn": round(nconn, 1),
                       "eloc_tflops": round(n * nconn * fwd / ms_e / 1e9, 1)}))
 
 
-def relu_variant(cfg, args, torch, qtx, flops_per_sweep):
+def relu_variant(cfg, args, torch, qtx, fwd):
     """The same VMC step, both modes, with the opt-in ReLU activation (the
     reference's network uses GELU); timed like the headline."""
     va = argparse.Namespace(**vars(args))
@@ -500,14 +489,15 @@ def relu_variant(cfg, args, torch, qtx, flops_per_sweep):
         print(f"[bench] building {args.config} {m} (ReLU variant)", file=sys.stderr, flush=True)
         res[m] = run_mode(cfg, m, va, torch, qtx)
     r, p = res["mixed"], res["plain"]
-    ach = flops_per_sweep / (r["metropolis_kernel_ms"] / 1e3) / 1e12
+    ach = cfg["ns"] * r["nconn"] * fwd / (r["eloc_ms"] / 1e3) / 1e12
     out = {"activation": "relu", "value": round(r["steps_per_s"], 5), "ms_per_step": round(r["ms_per_step"], 2),
            "stages_ms": {k: round(v, 2) for k, v in r["stages"].items()},
            "plain": {"value": round(p["steps_per_s"], 5), "ms_per_step": round(p["ms_per_step"], 2),
                      "stages_ms": {k: round(v, 2) for k, v in p["stages"].items()}},
            "mixed_over_plain": round(r["steps_per_s"] / p["steps_per_s"], 3),
-           "metropolis_kernel": {"avg_launch_ms": round(r["metropolis_kernel_ms"], 3),
-                                 "achieved_tflops": round(ach, 2), "frac": round(ach / MFMA_PEAK["bf16"], 4)}}
+           "metropolis_kernel_ms": round(r["metropolis_kernel_ms"], 3),
+           "eloc_kernel": {"avg_launch_ms": round(r["eloc_ms"], 3), "achieved_tflops": round(ach, 2),
+                           "frac": round(ach / MFMA_PEAK["bf16"], 4)}}
     if "precision" in r:
         out["precision"] = {k: r["precision"][k] for k in ("update_vector_rel_err", "energy_rel_err",
                                                            "logpsi_max_abs_diff") if k in r["precision"]}
@@ -557,35 +547,20 @@ def main():
     N = cfg["L"] ** 2 if cfg["model"] != "rbm1d" else cfg["L"]
     sweep_steps = args.sweep_steps or 2 * N
     roof = None
-    if cfg["model"] == "resconv" and args.config == "c4":
-        # sampling is cut here, so the dominant kernel is the fused E_loc (one
-        # forward per valid connected configuration); HIP events on its stream
+    if cfg["model"] == "resconv":
+        # the fused E_loc: one forward per valid connected configuration, so its
+        # FLOPs are known exactly (the Metropolis kernel, about as long, runs a
+        # forward only for proposals that change the spins); HIP events on its stream
         fwd = conv_flops_per_forward(cfg["nblocks"], cfg["channels"], N)
         flops = cfg["ns"] * r["nconn"] * fwd
         ach = flops / (r["eloc_ms"] / 1e3) / 1e12
         peak = MFMA_PEAK["bf16"] if main_mode == "mixed" else MFMA_PEAK["fp32"]
         roof = {"bound": "mfma", "achieved": round(ach, 2), "peak": peak, "unit": "TFLOP/s",
-                "frac": round(ach / peak, 4), "traffic": None, "kernel": "rc_eloc_kernel",
+                "frac": round(ach / peak, 4), "traffic": None, "kernel": "E_loc",
                 "flops_per_launch": flops, "avg_launch_ms": round(r["eloc_ms"], 3)}
-    elif cfg["model"] == "resconv":
-        fwd = conv_flops_per_forward(cfg["nblocks"], cfg["channels"], N)
-        flops = cfg["ns"] * sweep_steps * fwd  # one Metropolis launch = one sweep
-        t = r["metropolis_kernel_ms"] / 1e3  # HIP events around the kernel launch, same stream
-        ach = flops / t / 1e12
-        peak = MFMA_PEAK["bf16"] if main_mode == "mixed" else MFMA_PEAK["fp32"]
-        traffic = None
-        if args.config == "c3" and main_mode == "mixed" and sweep_steps == 512:
-            p = PMC_C3_MIXED
-            traffic = int(1024 * (p["fetch_kib"] * p["fetch_scale"] + p["write_kib"] * p["write_scale"]))
-        roof = {"bound": "mfma", "achieved": round(ach, 2), "peak": peak, "unit": "TFLOP/s",
-                "frac": round(ach / peak, 4), "traffic": traffic,
-                "traffic_source": None if traffic is None else
-                "not measured in this run: rocprofv3 --pmc FETCH_SIZE/WRITE_SIZE of this kernel, " + PMC_C3_MIXED["source"],
-                "hbm_gbps": None if traffic is None else round(traffic / t / 1e9, 3),
-                "hbm_peak_gbps": HBM_PEAK_GBS,
-                "traffic_algorithmic": cfg["ns"] * sweep_steps * 16 + 2 * cfg["ns"] * N + 24 * cfg["ns"],
-                "kernel": "rc_metropolis_kernel", "flops_per_launch": flops,
-                "avg_launch_ms": round(r["metropolis_kernel_ms"], 3)}
+        if r["metropolis_kernel_ms"]:
+            roof["metropolis"] = {"avg_launch_ms": round(r["metropolis_kernel_ms"], 3),
+                                  "proposals_per_s": round(cfg["ns"] * sweep_steps / r["metropolis_kernel_ms"] * 1e3)}
     out = {
         "metric": "VMC steps/s, 16x16 J1J2 ResConv MinSR (mixed vs FP64); served p50/p99 latency"
         if args.config == "c3" else
@@ -630,12 +605,12 @@ def main():
         fwd = conv_flops_per_forward(cfg["nblocks"], cfg["channels"], N)
         t_e = r["eloc_ms"] / 1e3
         nbytes = cfg["ns"] * (N + 8 + 8 + 4)
-        out["eloc"] = {"kernel": "rc_eloc_kernel", "ms": round(r["eloc_ms"], 2),
+        out["eloc"] = {"kernel": "E_loc", "ms": round(r["eloc_ms"], 2),
                        "achieved_tflops": round(cfg["ns"] * r["nconn"] * fwd / t_e / 1e12, 1),
                        "hbm_algorithmic_bytes": nbytes, "hbm_gbps": round(nbytes / t_e / 1e9, 4)}
     if (args.config == "c3" and args.activation == "gelu" and args.mode == "both" and
             not args.no_relu_variant):
-        out["relu_variant"] = relu_variant(cfg, args, torch, qtx, fwd * cfg["ns"] * sweep_steps)
+        out["relu_variant"] = relu_variant(cfg, args, torch, qtx, fwd)
     if not args.no_cpu_baseline:
         out["cpu_baseline"] = cpu_baseline(cfg, args.cpu_seconds, sweep_steps)
     if not args.no_serve and args.config == "c3":
