@@ -544,30 +544,97 @@ __global__ __launch_bounds__(256, 2) void gram_bf16x3_kernel(const __bf16* __res
       }
 }
 
-// S = Obar^T Obar (np x np), FP64, small np (SR branch, ns >= np)
+// No use of an accumulator before its MFMA is done, whatever branch follows:
+// the distance is kept here, not counted along one path
+template <int N>
+__device__ __forceinline__ void mfma_settle_f64(v4d* acc) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(acc[i]));
+  asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]));
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(acc[i]));
+}
+
+// S = Obar^T Obar (np x np), FP64 (SR branch, ns >= np).  One 16 x 16 tile of
+// the lower triangle per workgroup, its 16 waves a part of the samples each (every
+// 16th group of four): an MFMA's operands are 16 neighbouring columns
+// of four samples, read from O as they lie (no staging, no Obar in memory), TN_U
+// steps in flight.  Bound by the FP64 matrix pipe and the L1 (64 B per cycle) once
+// there are enough tiles; by the loads' latency with few samples.
+// 1024 x 272 f64: 10.7 us (43 with Obar formed and a library DGEMM, which is what
+// larger np take in a solve, kGramTnMax).
+constexpr int TN_U = 4, TN_W = 16;
 template <typename TI>
-__global__ __launch_bounds__(256) void gram_tn_kernel(const TI* __restrict__ O, const double* __restrict__ mean,
+__global__ __launch_bounds__(WAVE * TN_W) void gram_tn_kernel(const TI* __restrict__ O, const double* __restrict__ mean,
                                                       const double* __restrict__ r, int64_t ns, int64_t np,
                                                       double inv_ns, double* __restrict__ S) {
-  __shared__ double As[32][17], Bs[32][17];
-  int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-  int64_t k = (int64_t)blockIdx.y * 16 + ty, l = (int64_t)blockIdx.x * 16 + tx;
-  double acc = 0.0;
-  for (int64_t s0 = 0; s0 < ns; s0 += 32) {
-    for (int e = threadIdx.x; e < 32 * 16; e += 256) {
-      int ss = e / 16, c = e % 16;
-      int64_t s = s0 + ss;
-      int64_t ka = (int64_t)blockIdx.y * 16 + c, kb = (int64_t)blockIdx.x * 16 + c;
-      double sc = (s < ns) ? sqrt((r ? r[s] : 1.0) * inv_ns) : 0.0;
-      As[ss][c] = (s < ns && ka < np) ? ((double)O[s * np + ka] - mean[ka]) * sc : 0.0;
-      Bs[ss][c] = (s < ns && kb < np) ? ((double)O[s * np + kb] - mean[kb]) * sc : 0.0;
+  __shared__ double red[TN_W - 1][4][WAVE];
+  int bi, bj;
+  tile_of(blockIdx.x, bi, bj);
+  const int lane = threadIdx.x % WAVE, g = lane / 16, m = lane % 16;
+  const int q = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int64_t k = 16 * (int64_t)bi + m, l = 16 * (int64_t)bj + m;
+  const int64_t kc = k < np ? k : np - 1, lc = l < np ? l : np - 1;  // columns past np: not stored
+  const double mk = mean[kc], ml = mean[lc];
+  v4d acc[1] = {v4d{0, 0, 0, 0}};
+  TI a[2][TN_U], b[2][TN_U];
+  double w[2][TN_U];
+  auto load = [&](int64_t s0, int p) {  // samples past ns: weight 0
+#pragma unroll
+    for (int u = 0; u < TN_U; ++u) {
+      const int64_t s = s0 + 4 * TN_W * u + 4 * q + g, sc = s < ns ? s : ns - 1;
+      a[p][u] = O[sc * np + kc];
+      b[p][u] = O[sc * np + lc];
+      w[p][u] = s < ns ? (r ? r[sc] : 1.0) * inv_ns : 0.0;
     }
-    __syncthreads();
-#pragma unroll 8
-    for (int ss = 0; ss < 32; ++ss) acc += As[ss][ty] * Bs[ss][tx];
-    __syncthreads();
+  };
+  auto use = [&](int p) {
+#pragma unroll
+    for (int u = 0; u < TN_U; ++u)
+      acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(((double)a[p][u] - mk) * w[p][u], (double)b[p][u] - ml, acc[0], 0,
+                                                    0, 0);
+  };
+  constexpr int STEP = 4 * TN_W * TN_U;
+  load(0, 0);
+  for (int64_t s0 = 0; s0 < ns; s0 += 2 * STEP) {  // the next part is on its way during this one's products
+    load(s0 + STEP, 1);
+    use(0);
+    load(s0 + 2 * STEP, 0);
+    use(1);
   }
-  if (k < np && l < np) S[k * np + l] = acc;
+  mfma_settle_f64<1>(acc);
+  if (q > 0)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[q - 1][v][lane] = acc[0][v];
+  __syncthreads();
+  if (q > 0) return;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    double x = acc[0][v];
+#pragma unroll
+    for (int p = 0; p < TN_W - 1; ++p) x += red[p][v][lane];
+    const int64_t row = 16 * (int64_t)bi + 4 * v + g;
+    if (row < np && l < np && row >= l) {
+      S[row * np + l] = x;
+      S[l * np + row] = x;
+    }
+  }
+}
+
+// np up to which a solve forms S by gram_tn_kernel (us, it | Obar and DGEMM): 1024 x
+// 272 10.7 | 43, 4096 x 272 35 | 137, 8192 x 272 63 | 232, 4096 x 512 94 | 135, 4096
+// x 1000 250 | 144, 8192 x 1000 482 | 911, 4096 x 2000 942 | 495
+constexpr int64_t kGramTnMax = 512;
+
+template <typename TI>
+static int launch_gram_tn(hipStream_t st, const TI* O, const double* mean, const double* r, int64_t ns, int64_t np,
+                          double* S) {
+  const int64_t nt = (np + 15) / 16, tiles = nt * (nt + 1) / 2;
+  QTX_REQUIRE(tiles < 0x7fffffff, "Gram too large");
+  hipLaunchKernelGGL(gram_tn_kernel<TI>, dim3((unsigned)tiles), dim3(WAVE * TN_W), 0, st, O, mean, r, ns, np,
+                     1.0 / (double)ns, S);
+  QTX_LAUNCH_CHECK();
+  return QTX_OK;
 }
 
 // out[s, k] = (O[s, k] - mean[k]) sqrt(r_s / ns) in FP64 (grid-stride)
@@ -1758,17 +1825,6 @@ __device__ __forceinline__ double rsqrt_f64(double d) {
   return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
 }
 
-// No use of an accumulator before its MFMA is done, whatever branch follows:
-// the distance is kept here, not counted along one path
-template <int N>
-__device__ __forceinline__ void mfma_settle_f64(v4d* acc) {
-#pragma unroll
-  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(acc[i]));
-  asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]));
-#pragma unroll
-  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(acc[i]));
-}
-
 // base[off], 0 where !ok (base[0] is always readable): an address select instead
 // of a branch around each load
 __device__ __forceinline__ double load_or_zero(const double* base, int64_t off, bool ok) {
@@ -2440,22 +2496,26 @@ static int phase1(Task& t, rocblas_handle h) {
     if (rc) return rc;
     hipLaunchKernelGGL(copy_f64_kernel, dim3(nblk(io.ns, 256)), dim3(256), 0, t.st, io.ebar, t.w.y, io.ns);
   } else {
-    // S = Obar^T Obar: Obar formed in FP64 a row block at a time, each block
-    // accumulated by one rocBLAS DGEMM (a row-major rows x np block is the
-    // column-major np x rows matrix B, S += B B^T)
-    const int64_t rows = obar_rows(io.ns, io.np);
-    const double one = 1.0, zero = 0.0;
-    for (int64_t s0 = 0; s0 < io.ns; s0 += rows) {
-      const int64_t nr = std::min(rows, io.ns - s0), tot = nr * io.np;
-      hipLaunchKernelGGL(form_obar_kernel<TI>, dim3((unsigned)std::min<int64_t>((tot + 255) / 256, kGridCap)),
-                         dim3(256), 0, t.st, O + s0 * io.np, io.mean, io.r ? io.r + s0 : nullptr, nr, io.np,
-                         1.0 / (double)io.ns, t.w.obar);
-      QTX_LAUNCH_CHECK();
-      rc = rb(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_transpose, (rocblas_int)io.np,
-                            (rocblas_int)io.np, (rocblas_int)nr, &one, t.w.obar, (rocblas_int)io.np, t.w.obar,
-                            (rocblas_int)io.np, s0 ? &one : &zero, t.w.T, (rocblas_int)io.np),
-              "rocblas_dgemm");
-      if (rc) return rc;
+    // S = Obar^T Obar; beyond kGramTnMax Obar formed in FP64 a row block at a time,
+    // each block accumulated by one rocBLAS DGEMM (a row-major rows x np block is
+    // the column-major np x rows matrix B, S += B B^T)
+    if (io.np <= kGramTnMax) {
+      if ((rc = launch_gram_tn<TI>(t.st, O, io.mean, io.r, io.ns, io.np, t.w.T))) return rc;
+    } else {
+      const int64_t rows = obar_rows(io.ns, io.np);
+      const double one = 1.0, zero = 0.0;
+      for (int64_t s0 = 0; s0 < io.ns; s0 += rows) {
+        const int64_t nr = std::min(rows, io.ns - s0), tot = nr * io.np;
+        hipLaunchKernelGGL(form_obar_kernel<TI>, dim3((unsigned)std::min<int64_t>((tot + 255) / 256, kGridCap)),
+                           dim3(256), 0, t.st, O + s0 * io.np, io.mean, io.r ? io.r + s0 : nullptr, nr, io.np,
+                           1.0 / (double)io.ns, t.w.obar);
+        QTX_LAUNCH_CHECK();
+        rc = rb(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_transpose, (rocblas_int)io.np,
+                              (rocblas_int)io.np, (rocblas_int)nr, &one, t.w.obar, (rocblas_int)io.np, t.w.obar,
+                              (rocblas_int)io.np, s0 ? &one : &zero, t.w.T, (rocblas_int)io.np),
+                "rocblas_dgemm");
+        if (rc) return rc;
+      }
     }
     rc = launch_obar_t_y<TI>(t.st, O, io.mean, io.r, io.ebar, io.ns, io.np, t.w.y);  // F = Obar^T ebar
     if (rc) return rc;
@@ -3097,15 +3157,8 @@ int qtx_gram(void* stream, int o_dtype, const void* O, const double* mean, const
     if (o_dtype == QTX_F32) return launch_gram_nt<float>(st, gram, (const float*)O, mean, r, ns, np, T, ws);
     return launch_gram_nt<double>(st, gram, (const double*)O, mean, r, ns, np, T, ws);
   }
-  dim3 g(nblk(np, 16), nblk(np, 16));
-  if (o_dtype == QTX_F32)
-    hipLaunchKernelGGL(gram_tn_kernel<float>, g, dim3(256), 0, st, (const float*)O, mean, r, ns, np,
-                       1.0 / (double)ns, T);
-  else
-    hipLaunchKernelGGL(gram_tn_kernel<double>, g, dim3(256), 0, st, (const double*)O, mean, r, ns, np,
-                       1.0 / (double)ns, T);
-  QTX_LAUNCH_CHECK();
-  return QTX_OK;
+  if (o_dtype == QTX_F32) return launch_gram_tn<float>(st, (const float*)O, mean, r, ns, np, T);
+  return launch_gram_tn<double>(st, (const double*)O, mean, r, ns, np, T);
 }
 
 int qtx_apply_update(void* stream, int dtype, void* theta, const double* step, double lr, int64_t np,
