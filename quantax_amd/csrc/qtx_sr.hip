@@ -1889,8 +1889,13 @@ __global__ __launch_bounds__(256) void chol_panel_kernel(double* A, int64_t lda,
       x[b][v] = load_or_zero(Xp, xr + xc * xs, xr < h && xc < w);
     }
   int bad = -1;
+  const int groups = (w + 7) / 8;  // a short last panel: the rest is the identity
+  for (int c8 = 8 * groups + q; c8 < CT; c8 += 4) {
+    Ls[c8 * CL + lane] = lane == c8 ? 1.0 : 0.0;
+    rdg[c8] = 1.0;
+  }
 #pragma unroll 1
-  for (int gb = 0; gb < 8; ++gb) {
+  for (int gb = 0; gb < groups; ++gb) {
     if (q == gb / 2) {
       // to one row per lane through these columns of Ls
 #pragma unroll
