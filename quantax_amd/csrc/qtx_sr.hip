@@ -408,6 +408,12 @@ constexpr int G3_FLUSH = 8;          // stages per FP32 -> FP64 flush (256 K)
 constexpr int G3_ROW = 2 * G3_KC * 2;     // bytes of a row's hi and lo parts of one stage (a 128-byte line)
 constexpr int G3_OPER = GT * G3_ROW;      // bytes of one operand of one stage (16 KB)
 constexpr int G3_KPAD = 64;
+// From this many tile rows on the super-blocks are dealt to the XCDs one by one:
+// the eight that run together then share their row panels, and the last-level
+// cache serves what the L2s miss (16384 x 34952: 38.9 -> 37.2 ms, 32768 x 286976:
+// 1472 -> 1429).  Below, an XCD takes a contiguous run of tiles: few super-blocks
+// do not divide evenly (64 tile rows: 12 % more tiles on one XCD than on average).
+constexpr int G3_DEAL = 96;
 
 static inline int64_t g3_rows(int64_t n) { return (n + GT - 1) / GT * GT; }
 static inline int64_t g3_kpad(int64_t np) { return (np + G3_KPAD - 1) / G3_KPAD * G3_KPAD; }
@@ -448,14 +454,30 @@ typedef __attribute__((address_space(3))) void lds_void;
 // Bound by L2 misses at large n: the 64 tiles an XCD runs together (an 8 x 8
 // super-block) drift apart in K by more than its L2 holds, 154 GB at 4.3 TB/s for
 // 16384 x 34952, where 37 GB would do.  16384 x 34952 with the pass above: 41.7 ->
-// 38.9 ms; 8192: 9.8 ms, 4096: 3.9 -> 3.0 ms (one workgroup per CU with separate
+// 37.2 ms; 8192: 9.8 ms, 4096: 3.9 -> 3.0 ms (one workgroup per CU with separate
 // planes and K = 64 stages before; half-line stages, 64 bytes per row and plane,
 // took 46.5 ms at 16384).
 __global__ __launch_bounds__(256, 2) void gram_bf16x3_kernel(const __bf16* __restrict__ HL, int64_t n, int64_t kpad,
                                                              int ntiles, double* __restrict__ T) {
   __shared__ __attribute__((aligned(16))) char smem[2 * 2 * G3_OPER];
   int bi, bj;
-  super_tile_of(xcd_tile(blockIdx.x, ntiles), (int)((n + GT - 1) / GT), bi, bj);
+  const int mt = (int)((n + GT - 1) / GT);
+  if (mt < G3_DEAL) {
+    super_tile_of(xcd_tile(blockIdx.x, ntiles), mt, bi, bj);
+  } else {
+    const int x = blockIdx.x % 8, loc = blockIdx.x / 8, in = loc % 64;
+    int R, C;
+    tile_of(loc / 64 * 8 + x, R, C);
+    bi = in / 8;
+    bj = in % 8;
+    if (R == C) {
+      if (in >= 36) return;
+      tile_of(in, bi, bj);
+    }
+    bi += 8 * R;
+    bj += 8 * C;
+    if (bi >= mt) return;
+  }
   const int64_t i0 = (int64_t)bi * GT, j0 = (int64_t)bj * GT;
   const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
   const int wr = (wv / 2) * 64, wc = (wv % 2) * 64;
@@ -1687,6 +1709,11 @@ static int launch_gram_nt(hipStream_t st, int gram, const TI* O, const double* m
     __bf16* HL = (__bf16*)split_ws;
     hipLaunchKernelGGL(split_bf16x3_kernel<TI>, dim3((unsigned)std::min<int64_t>(nblocks, kGridCap)), dim3(256), 0,
                        st, O, mean, r, n, np, kpad, bpr, nblocks, inv_ns, HL);
+    if (nt >= G3_DEAL) {
+      const int64_t ms = (nt + 7) / 8, sb = ms * (ms + 1) / 2;
+      QTX_REQUIRE((sb + 7) / 8 * 512 < 0x7fffffff, "Gram too large");
+      g = dim3((unsigned)((sb + 7) / 8 * 512));
+    }
     hipLaunchKernelGGL(gram_bf16x3_kernel, g, bl, 0, st, (const __bf16*)HL, n, kpad, (int)ntiles, T);
   } else {
     const int64_t mt = (n + GN_T - 1) / GN_T, mtiles = mt * (mt + 1) / 2;
@@ -2359,7 +2386,8 @@ static bool tri_pass_ok(int64_t n, bool sym) {
 // (qtx_minsr_solve_many): every task's phase p is enqueued before any task's
 // phase p + 1 reads results back.
 //   phase 1: Gram (and for SR the right-hand side Obar^T ebar); CHOL_SHIFT:
-//            shift + potrf + potrs; EIGH_PINV: the first Lanczos steps.
+//            shift, factorisation and both substitutions; EIGH_PINV: the first
+//            Lanczos steps.
 //   phase 2: EIGH_PINV: read the Lanczos coefficients (sync), extend until the
 //            largest Ritz value settles, then syrk + three (potrf, refinement)
 //            for the partial fractions; dsyevd where that route does not apply.
