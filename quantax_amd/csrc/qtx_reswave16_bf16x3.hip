@@ -53,7 +53,7 @@ int rw_metropolis<16, QTX_CONV_BF16X3>(hipStream_t st, const RcLayout& L, const 
                                     int width, int hopping, const uint32_t* words, int nsteps, int64_t ns,
                                     double reweight, double tie_tol, int8_t* s, double* logabs, int32_t* n_accept,
                                     int32_t* n_near) {
-  const RwPick pk = rw_pick(16, L.N, ns);
+  const RwPick pk = rw_pick(16, L.N, ns, true);
   if (pk.P == 1 && pk.maxt == 4) {
     RW_LAUNCH(rw_metropolis_kernel, 16, QTX_CONV_BF16X3, 4, 1, 1, 0, (ns + G - 1) / G,
               kind, nbr, width, hopping, words, nsteps, ns, reweight, tie_tol, s, logabs, n_accept, n_near);

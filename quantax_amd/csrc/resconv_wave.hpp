@@ -11,7 +11,7 @@
 // after the start of the kernel, every chain or candidate proceeds on its own
 // and the waves of a SIMD overlap one's activations with another's MFMAs.
 // P grows with the lattice (registers) and when there are too few
-// configurations to give every SIMD two waves (rw_pick).
+// configurations for the SIMDs (rw_pick).
 //
 // Per layer the K loop runs over the taps outside the tile loop: one tap's
 // weights serve all tiles.  With 16 channels a layer's weights are in
@@ -28,10 +28,10 @@
 // Measured against the previous any-lattice kernels (two configurations per
 // workgroup, tap addresses formed per tile on VALU, ping-pong activations, a
 // barrier per layer): J1-J2 E_loc of 1000 samples 10 x 10, 16 channels, 4
-// blocks, FP32 16.4 -> 7.5 ms; a forward of 1000 6 x 6 configurations 50 -> 32 us; forwards of 10000 6 x 6 configurations 533 ->
-// 215 us, 8000 of 10 x 10 718 -> 360 us (split-bf16 323 -> 195), 3000 of 10 x
-// 10 with 32 channels 554 -> 346 us (split-bf16 313 -> 142), 2000 of 18 x 18
-// 510 -> 313 us.
+// blocks, FP32 16.4 -> 7.5 ms; a forward of 1000 6 x 6 configurations 50 -> 25
+// us; forwards of 10000 6 x 6 configurations 533 -> 215 us, 8000 of 10 x 10 718 ->
+// 360 us (split-bf16 323 -> 195), 3000 of 10 x 10 with 32 channels 554 -> 346 us
+// (split-bf16 313 -> 142), 2000 of 18 x 18 510 -> 313 us.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -666,25 +666,37 @@ __global__ __launch_bounds__(RW_THREADS, 2) void rw_eloc_kernel(RcArgs a, RwMerg
 }
 
 // ---------------------------------------------------------------- dispatch
-// Waves per configuration and tiles per wave.  P = 1 as long as the tiles'
-// registers (8 C / 16 per tile and lane, besides offsets and weights) leave
-// two waves per SIMD and there are at least two configurations per SIMD
-// (2048); fewer configurations are spread over four waves each (200
-// configurations of 10 x 10, 32 channels, split-bf16: 41 us; one wave each
-// would run the whole network in sequence on 200 of 1024 SIMDs).
+// Waves per configuration and tiles per wave.  P = 1 (2 where the tiles'
+// registers would not leave two waves per SIMD) does the least work, but a pass
+// then takes as long as one wave needs for a whole network, for 1 to 1024
+// configurations (one wave per SIMD) and half as long again up to 2048; P = 4
+// takes time in proportion, in steps of 256 (a workgroup per CU).  So P = 4 is
+// for fewer than 768 and between 1025 and 1536.  us, P = 4 | P = 1, four blocks:
+//                       768         1000        1250        1640        2000
+//   6 x 6, 16, FP32   22 | 25     31 | 25     35 | 37     48 | 37     53 | 37
+//   8 x 8, 16, FP32   24 | 31     32 | 31     37 | 47     51 | 47     56 | 47
+//   8 x 8, 32, bf16   31 | 42     51 | 41     57 | 50     76 | 50     83 | 52
+//   10 x 10, 16, FP32 37 | 49     51 | 49     60 | 78     83 | 78     92 | 78
+//   12 x 12, 16 (P 2) 55 | 56     66 | 57     85 | 89    116 | 110   131 | 112
+// (10 x 10 in split-bf16 at 1000: 31 | 34, so five to eight tiles start at 1537.)
+// A single tile leaves three of four waves idle: P = 1 from 512 on.  In a sweep the
+// chains whose proposal does not move leave their waves' time to the others, so
+// P = 4 stays best up to 1536 (8 x 8, FP32, 24 steps of 1000 chains: 535 | 625 us;
+// of 2000: 949 | 855) and P = 2 starts at 1793.
 struct RwPick {
   int P, maxt;
 };
-inline RwPick rw_pick(int C, int N, int64_t units) {
+inline RwPick rw_pick(int C, int N, int64_t units, bool sweep = false) {
   const int nt = (N + 15) / 16;
-  const bool many = units >= 2048;
+  const bool late = units > 1536, full = late || (!sweep && units > 768 && units <= 1024);
+  if (nt == 1 && units >= 512) return {1, 4};
+  if (full && nt <= 4) return {1, 4};
   if (C == 16) {
-    if (many && nt <= 8) return {1, nt <= 4 ? 4 : 8};
-    if (many && nt <= 16) return {2, 8};
+    if (late && nt <= 8) return {1, 8};
+    if ((sweep ? units > 1792 : full) && nt > 8 && nt <= 16) return {2, 8};
     return {4, nt <= 8 ? 2 : (nt <= 16 ? 4 : 8)};
   }
-  if (many && nt <= 4) return {1, 4};
-  if (many && nt <= 8) return {2, 4};
+  if (units > 1792 && nt <= 8) return {2, 4};
   return {4, nt <= 8 ? 2 : (nt <= 16 ? 4 : 7)};
 }
 
