@@ -419,24 +419,55 @@ static inline int64_t g3_rows(int64_t n) { return (n + GT - 1) / GT * GT; }
 static inline int64_t g3_kpad(int64_t np) { return (np + G3_KPAD - 1) / G3_KPAD * G3_KPAD; }
 static inline size_t g3_bytes(int64_t n, int64_t np) { return (size_t)g3_rows(n) * g3_kpad(np) * 2 * sizeof(__bf16); }
 
-// Grid-stride over (row, 256-column block) pairs: a launch's work-item count
-// is a 32-bit quantity, and rows * kpad passes 2^32 at 32768 x 286976.
+// Eight columns per thread: one row factor for them, two loads that need only the
+// element's own alignment, one 16-byte store per part.  HBM-bound: 16384 x 34952
+// 1.57 -> 1.13 ms (one column, a square root and two 2-byte stores per thread
+// before).  Grid-stride over (row, 2048-column block) pairs: a launch's work-item
+// count is a 32-bit quantity, and rows * kpad passes 2^32 at 32768 x 286976.
+constexpr int SP_COLS = 8;
 template <typename TI>
 __global__ __launch_bounds__(256) void split_bf16x3_kernel(const TI* __restrict__ O, const double* __restrict__ mean,
                                                            const double* __restrict__ r, int64_t n, int64_t np,
                                                            int64_t kpad, int64_t bpr, int64_t nblocks, double inv_ns,
                                                            __bf16* __restrict__ HL) {
+  typedef TI vt4 __attribute__((ext_vector_type(4), aligned(sizeof(TI))));
   for (int64_t blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
     const int64_t row = blk / bpr;
-    const int64_t k = (blk % bpr) * 256 + threadIdx.x;
+    const int64_t k = ((blk % bpr) * 256 + threadIdx.x) * SP_COLS;
     if (k >= kpad) continue;
-    double v = 0.0;
-    if (row < n && k < np) v = ((double)O[row * np + k] - mean[k]) * sqrt((r ? r[row] : 1.0) * inv_ns);
-    const float f = (float)v;
-    const __bf16 hi = (__bf16)f;
-    __bf16* p = HL + 2 * (row * kpad + k / G3_KC * G3_KC) + k % G3_KC;
-    p[0] = hi;
-    p[G3_KC] = (__bf16)(f - (float)hi);
+    TI o[SP_COLS];
+    double m[SP_COLS];
+    const TI* p = O + row * np + k;
+    const bool in = row < n;
+    if (in && k + SP_COLS <= np) {
+      const vt4 x = *reinterpret_cast<const vt4*>(p), y = *reinterpret_cast<const vt4*>(p + 4);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        o[c] = x[c];
+        o[c + 4] = y[c];
+      }
+#pragma unroll
+      for (int c = 0; c < SP_COLS; ++c) m[c] = mean[k + c];
+    } else {
+#pragma unroll
+      for (int c = 0; c < SP_COLS; ++c) {
+        const bool ok = in && k + c < np;
+        o[c] = ok ? p[c] : TI(0);
+        m[c] = ok ? mean[k + c] : 0.0;
+      }
+    }
+    const double f = sqrt((r && in ? r[row] : 1.0) * inv_ns);
+    v8bf hi, lo;
+#pragma unroll
+    for (int c = 0; c < SP_COLS; ++c) {
+      float x = (float)(((double)o[c] - m[c]) * f);
+      asm("" : "+v"(x));  // rounded to single precision first: not folded into FP64 -> bf16
+      hi[c] = (__bf16)x;
+      lo[c] = (__bf16)(x - (float)hi[c]);
+    }
+    __bf16* q = HL + 2 * (row * kpad + k / G3_KC * G3_KC) + k % G3_KC;
+    *reinterpret_cast<v8bf*>(q) = hi;
+    *reinterpret_cast<v8bf*>(q + G3_KC) = lo;
   }
 }
 
@@ -454,7 +485,7 @@ typedef __attribute__((address_space(3))) void lds_void;
 // Bound by L2 misses at large n: the 64 tiles an XCD runs together (an 8 x 8
 // super-block) drift apart in K by more than its L2 holds, 154 GB at 4.3 TB/s for
 // 16384 x 34952, where 37 GB would do.  16384 x 34952 with the pass above: 41.7 ->
-// 37.2 ms; 8192: 9.8 ms, 4096: 3.9 -> 3.0 ms (one workgroup per CU with separate
+// 36.5 ms; 8192: 9.8 ms, 4096: 3.9 -> 2.9 ms (one workgroup per CU with separate
 // planes and K = 64 stages before; half-line stages, 64 bytes per row and plane,
 // took 46.5 ms at 16384).
 __global__ __launch_bounds__(256, 2) void gram_bf16x3_kernel(const __bf16* __restrict__ HL, int64_t n, int64_t kpad,
@@ -1704,7 +1735,7 @@ static int launch_gram_nt(hipStream_t st, int gram, const TI* O, const double* m
   double inv_ns = 1.0 / (double)n;
   if (gram == QTX_GRAM_BF16X3) {
     QTX_REQUIRE(split_ws != nullptr, "split-bf16 Gram needs its workspace");
-    const int64_t rows = g3_rows(n), kpad = g3_kpad(np), bpr = (kpad + 255) / 256;
+    const int64_t rows = g3_rows(n), kpad = g3_kpad(np), bpr = (kpad + 256 * SP_COLS - 1) / (256 * SP_COLS);
     const int64_t nblocks = rows * bpr;
     __bf16* HL = (__bf16*)split_ws;
     hipLaunchKernelGGL(split_bf16x3_kernel<TI>, dim3((unsigned)std::min<int64_t>(nblocks, kGridCap)), dim3(256), 0,
