@@ -2197,7 +2197,7 @@ __global__ __launch_bounds__(256) void chol_back_kernel(const double* __restrict
 #pragma unroll
   for (int i = 0; i < 16; ++i) Ls[(16 * q + i) * (CT + 1) + lane] = p[i];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) p[i] = load_or_zero(A + p0 + j0 * n, lane + i * n, b > 0 && lane < w);
+  for (int i = 0; i < 16; ++i) p[i] = load_or_zero(A + p0, lane + (j0 + i) * n, b > 0 && lane < w);
   __syncthreads();
   if (q == 0) {
     double z = lane < w ? y[p0 + lane] : 0.0, xi = 0.0;
