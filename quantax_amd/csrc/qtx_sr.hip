@@ -1583,6 +1583,14 @@ constexpr int kLanczosMax = 512;  // Lanczos steps for lambda_max before giving 
 #define QTX_CHOL_BLOCK 1024
 #endif
 constexpr int64_t kCholBlock = QTX_CHOL_BLOCK;  // diagonal block of the blocked Cholesky
+// Width of the diagonal block that starts with `rem` columns left: the rest of the
+// matrix once the panel and update kernels do it faster than dtrsm and dsyrk on
+// its blocks (the rank-64 updates then come from the last-level cache): 4096 3.85
+// -> 2.99 ms, 6144 7.7 -> 6.4, the last 6144 of 12288 31.0 -> 29.7, of 16384 58.6
+// -> 57.5 (8192: 58.4); three matrices of 2000 7.0 -> 5.35 ms for their solve.
+static int64_t chol_block(int64_t rem, int batch) {
+  return rem <= (batch == 1 ? 6144 : 2048) ? rem : kCholBlock;
+}
 constexpr int kInfoPerFactor = (int)((131072 + kCholBlock - 1) / kCholBlock);  // status slots: n <= 131072
 
 // Rows of FP64 Obar formed per DGEMM chunk in the SR branch (<= 256 MiB)
@@ -1858,8 +1866,8 @@ static int pinv_syevd(hipStream_t st, rocblas_handle h, int64_t n, double rtol, 
 
 // ---------------------------------------------------------------- Cholesky
 // Right-looking blocked Cholesky (lower, column-major, leading dimension n) of
-// `batch` matrices `stride` elements apart.  Each kCholBlock-wide diagonal
-// block is factored in CT-column panels by two kernels of this file (panel:
+// `batch` matrices `stride` elements apart.  Each diagonal block (kCholBlock
+// columns, or all that is left: chol_block) is factored in CT-column panels by two kernels of this file (panel:
 // factor the CT x CT diagonal tile in LDS and solve the tiles below it inside
 // the block; update: the rank-CT update of the block's remaining tiles), all
 // matrices in one launch, so the latency-bound diagonal work of one matrix
@@ -2233,8 +2241,8 @@ static int blocked_potrf(rocblas_handle h, hipStream_t st, int64_t n, double* A,
   const double one = 1.0, minus_one = -1.0;
   const rocblas_int ld = (rocblas_int)n;
   int b = 0;
-  for (int64_t k = 0; k < n; k += kCholBlock, ++b) {
-    const int64_t kb = (n - k < kCholBlock) ? n - k : kCholBlock;
+  for (int64_t k = 0, kb; k < n; k += kb, ++b) {
+    kb = chol_block(n - k, batch);
     const int nt = (int)((kb + CT - 1) / CT);
     for (int kp = 0; kp < nt; ++kp) {
       hipLaunchKernelGGL(chol_panel_kernel, dim3((unsigned)(nt - kp + (y ? 1 : 0)), (unsigned)batch), dim3(256), 0, st,
@@ -2983,8 +2991,9 @@ static int blas_query(rocblas_handle h, int64_t ns, int64_t np, int mode, SolveW
   }
   if (bm == QTX_SOLVE_CHOL_SHIFT || bm == QTX_SOLVE_EIGH_PINV) {  // panels of the blocked Cholesky
     double* A = (bm == QTX_SOLVE_CHOL_SHIFT) ? w.T : w.T2;
-    for (int64_t k = 0; k < n; k += kCholBlock) {
-      const int64_t kb = (n - k < kCholBlock) ? n - k : kCholBlock, m = n - k - kb;
+    for (int64_t k = 0, kb; k < n; k += kb) {
+      kb = chol_block(n - k, bm == QTX_SOLVE_CHOL_SHIFT ? 1 : 3);  // the smaller blocks: every call of either
+      const int64_t m = n - k - kb;
       if (m == 0) break;
       double* Akk = A + k * n + k;
       good &= ok(rocblas_dtrsm(h, rocblas_side_right, rocblas_fill_lower, rocblas_operation_transpose,

@@ -1,5 +1,6 @@
 """The blocked Cholesky factorisation and its fused substitutions at the edges
-of their tiles: 16-column groups, 64-column panels, 1024-column diagonal blocks.
+of their tiles: 16-column groups, 64-column panels, the diagonal blocks (one up
+to 6144 columns, 1024 and the rest beyond).
 
 The shifted solve is compared with the same solve in float64 on the CPU.
 Tolerance: 8 (n + np) u cond(T + shift), u = 2^-53: the usual bounds of the
@@ -34,3 +35,33 @@ def test_shifted_solve(n):
     tol = 8 * (n + np_) * 2.0**-53 * cond
     print(f"n {n}: cond {cond:.1e} err {err:.2e} tol {tol:.2e}")
     assert err <= tol, (err, tol)
+
+
+@pytest.mark.parametrize("n", [6143, 6144, 6145, 7300])
+def test_shifted_solve_closed_form(n):
+    """O = sqrt(n) H1 D H2 with reflections H1, H2 and known singular values, so
+    x = H2 D^T (D^2 + shift)^-1 H1 y.  The same tolerance."""
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    np_ = n + 7
+    u, v = (torch.randn(k, dtype=torch.float64, device="cuda", generator=gen) for k in (n, np_))
+    u, v = u / u.norm(), v / v.norm()
+    s = torch.logspace(0, -2, n, dtype=torch.float64, device="cuda")
+    s = s[torch.randperm(n, device="cuda", generator=gen)]
+    dv, ud = s * v[:n], torch.zeros(np_, dtype=torch.float64, device="cuda")
+    ud[:n] = u * s
+    O = torch.zeros(n, np_, dtype=torch.float64, device="cuda")
+    O[torch.arange(n), torch.arange(n)] = s
+    O -= 2 * torch.outer(u, ud) + 2 * torch.outer(dv, v) - 4 * (u @ dv) * torch.outer(u, v)
+    O *= n**0.5
+    y = torch.randn(n, dtype=torch.float64, device="cuda", generator=gen)
+    mean = torch.zeros(np_, dtype=torch.float64, device="cuda")
+    x = qtx.optimizer.solve_step(O, mean, y, qtx.optimizer.minnorm_shift_eig(rshift=1e-8, ashift=1e-6, gram="fp64"))
+    shift = 1e-8 * float((s * s).sum()) + 1e-6
+    z = torch.zeros(np_, dtype=torch.float64, device="cuda")
+    z[:n] = s / (s * s + shift) * (y - 2 * u * (u @ y))
+    ref = z - 2 * v * (v @ z)
+    err = float((x - ref).norm() / ref.norm())
+    cond = (1.0 + shift) / (float((s * s).min()) + shift)
+    tol = 8 * (n + np_) * 2.0**-53 * cond
+    print(f"n {n}: cond {cond:.1e} err {err:.2e} tol {tol:.2e}")
+    assert err <= tol
