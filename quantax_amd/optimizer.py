@@ -234,16 +234,24 @@ class QNGD:
 
     @staticmethod
     def _weights(samples) -> Optional[torch.Tensor]:
-        """The reweighting factors as the kernels take them.  Factors of one give
-        the same bits as none, so a tensor that the kernels can read goes to them
-        unseen: looking at its values would make the host wait for the sweep (60
-        us, twice per step).  Any other tensor is looked at: ones need no kernel
-        to read them."""
+        """The reweighting factors as the kernels read them: float64, contiguous, one
+        per sample, on this GPU.  A tensor of that kind goes to them unseen: looking
+        at its values would make the host wait for the sweep (60 us, twice per
+        step).  Any other tensor is looked at, wherever it and the spins live: ones
+        need no kernel to read them, others are copied into that form."""
         r = samples.reweight_factor
-        if r is None or (r.dtype == torch.float64 and r.is_contiguous() and r.device == samples.spins.device
-                         and r.shape == samples.spins.shape[:1]):
+        if r is None:
+            return None
+        r = torch.as_tensor(r)
+        ns = len(samples.spins)
+        if (r.is_cuda and r.device == _lib.device() and r.dtype == torch.float64 and r.is_contiguous()
+                and r.shape == (ns,)):
             return r
-        return None if bool(torch.all(r == 1.0).item()) else r
+        if bool(torch.all(r == 1.0).item()):
+            return None
+        if r.shape != (ns,):
+            raise ValueError(f"expected one reweighting factor for each of the {ns} samples, got {tuple(r.shape)}")
+        return r.to(_lib.device(), torch.float64).contiguous()
 
 
 class SR(QNGD):
@@ -273,7 +281,6 @@ class SR(QNGD):
         self._eloc = eloc
         ns = eloc.shape[0]
         r = self._weights(samples)
-        r = None if r is None else r.contiguous()
         ebar = torch.empty(ns, dtype=torch.float64, device=eloc.device)
         out2 = torch.empty(2, dtype=torch.float64, device=eloc.device)
         _lib.call("qtx_ebar", _lib.stream(), eloc.data_ptr(), _lib.ptr(r), ns, ebar.data_ptr(), out2.data_ptr())
