@@ -268,14 +268,16 @@ def reference_default_solve(last, solver, torch, qtx):
     (``optimizer/solver.py:12-21``), below 1e-5 lambda_max: the shifted
     Cholesky route when T allows it, else dsyevd; and the same solve forced
     through dsyevd (EIGH_PINV_DIRECT) for its time and the two results'
-    relative difference.  HIP events around each call, the step's own O and
-    Ebar, the faster of two calls."""
+    relative difference.  HIP events around each call, the step's own O, Ebar
+    and reweighting factors, the faster of two calls."""
+    r = qtx.optimizer.QNGD._weights(last["samples"])
+
     def timed(s):
         ms, x = [], None
         for _ in range(2):
             a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             a.record()
-            x = qtx.optimizer.solve_step(last["O"], last["mean"], last["ebar"], s)
+            x = qtx.optimizer.solve_step(last["O"], last["mean"], last["ebar"], s, r)
             b.record()
             torch.cuda.synchronize()
             ms.append(a.elapsed_time(b))

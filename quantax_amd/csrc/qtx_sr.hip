@@ -165,6 +165,15 @@ __global__ __launch_bounds__(1024) void ebar_kernel(const double* __restrict__ E
   }
 }
 
+// single block: out[0] = 1 if every r_i is one, else 0
+__global__ __launch_bounds__(1024) void all_ones_kernel(const double* __restrict__ r, int64_t n,
+                                                        double* __restrict__ out) {
+  bool other = false;
+  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) other |= !(r[i] == 1.0);
+  const int any = __syncthreads_or(other ? 1 : 0);
+  if (threadIdx.x == 0) out[0] = any ? 0.0 : 1.0;
+}
+
 // ---------------------------------------------------------------- Gram T = A A^T
 // A = Obar (n x np) from O rows; only tiles with bi >= bj are computed and
 // mirrored.  Output T is FP64 (n x n, symmetric).
@@ -1640,7 +1649,7 @@ struct SolveWs {
   double* z;       // max(ns, np)
   double* D;       // n
   double* E;       // n
-  double* scalars; // 8
+  double* scalars; // 8: trace, power-of-two scale, whether the weights are one (MinSR), -, four norms
   int32_t* info;   // 4 (+pad)
   double* dtile;   // 3 x 64 x 64: factored diagonal tiles of the blocked Cholesky, staged
   // partial-fraction soft inverse (EIGH_PINV modes only)
@@ -2618,6 +2627,9 @@ static int phase1(Task& t, rocblas_handle h) {
   // recurrence; the largest Ritz value is checked every 32 steps)
   hipLaunchKernelGGL(lanczos_init_kernel, dim3(1), dim3(1024), 0, t.st, t.n, t.w.V, t.w.ab + kLanczosMax);
   t.mcap = (int)(t.n < kLanczosMax ? t.n : kLanczosMax);
+  // whether the weights are all one, for phase 2 (the small-cutoff route)
+  if (t.minnorm && io.r)
+    hipLaunchKernelGGL(all_ones_kernel, dim3(1), dim3(1024), 0, t.st, io.r, io.ns, t.w.scalars + 2);
   // convergence checks every 16 steps when one product streams more than
   // 512 MB of T (n > 8192: 16 products cost far more than the host round
   // trip of a check; a VMC Gram's top eigenvalue, well separated, settles
@@ -2710,6 +2722,9 @@ static int phase2(Task& t, rocblas_handle h) {
     double lmax = 0.0;
     int msteps = 0;
     bool bad = false;
+    double ones = 1.0;  // read with the coefficients: no further wait
+    if (t.minnorm && io.r)
+      QTX_HIP(hipMemcpyAsync(&ones, t.w.scalars + 2, sizeof(double), hipMemcpyDeviceToHost, t.st));
     for (;;) {
       QTX_HIP(hipMemcpyAsync(ha.data(), t.w.ab, (size_t)t.done * 8, hipMemcpyDeviceToHost, t.st));
       QTX_HIP(hipMemcpyAsync(hb.data(), t.w.ab + kLanczosMax, (size_t)(t.done + 1) * 8, hipMemcpyDeviceToHost, t.st));
@@ -2744,7 +2759,7 @@ static int phase2(Task& t, rocblas_handle h) {
       t.fallback = 2;
     } else if (!(lmax > 0.0) || !std::isfinite(lmax)) {
       t.fallback = 3;
-    } else if (!std::isfinite(c) || (!(rel >= 1e-5) && t.minnorm && io.r != nullptr)) {
+    } else if (!std::isfinite(c) || (!(rel >= 1e-5) && t.minnorm && ones == 0.0)) {
       t.fallback = 1;  // (reweighted MinSR: the null direction of T is not 1)
     }
     if (t.fallback) {
