@@ -2058,11 +2058,13 @@ __global__ __launch_bounds__(256) void chol_panel_kernel(double* A, int64_t lda,
   __syncthreads();
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
+    v4d lx = v4d{0, 0, 0, 0};
 #pragma unroll
     for (int p = 0; p < b; ++p)
 #pragma unroll
       for (int s = 0; s < 4; ++s)
-        x[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-Ls[(16 * p + 4 * s + g) * CL + 16 * b + m], x[p][s], x[b], 0, 0, 0);
+        lx = __builtin_amdgcn_mfma_f64_16x16x4f64(-Ls[(16 * p + 4 * s + g) * CL + 16 * b + m], x[p][s], lx, 0, 0, 0);
+    x[b] += lx;
     double inv[4];
     v4d t = v4d{0, 0, 0, 0}, r = x[b];
 #pragma unroll
@@ -2150,20 +2152,23 @@ __global__ __launch_bounds__(256) void chol_update_kernel(double* A, int64_t lda
   }
   __syncthreads();
   if (16 * q >= hi) return;
+  // the products are summed by themselves and taken off at once: 64 roundings the
+  // size of the sum instead of the size of A_ij
+  v4d ll[4] = {v4d{0, 0, 0, 0}, v4d{0, 0, 0, 0}, v4d{0, 0, 0, 0}, v4d{0, 0, 0, 0}};
 #pragma unroll 2
   for (int s = 0; s < 16; ++s) {
     const double l = Li[(4 * s + g) * CL + row];
 #pragma unroll
     for (int b = 0; b < 4; ++b)
-      c[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(Lj[(4 * s + g) * CL + 16 * b + m], l, c[b], 0, 0, 0);
+      ll[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(Lj[(4 * s + g) * CL + 16 * b + m], l, ll[b], 0, 0, 0);
   }
-  mfma_settle_f64<4>(c);
+  mfma_settle_f64<4>(ll);
 #pragma unroll
   for (int b = 0; b < 4; ++b)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int col = 16 * b + 4 * v + g;
-      if (row < hi && col < hj && (ti != tj || row >= col)) Cp[row + col * cs] = c[b][v];
+      if (row < hi && col < hj && (ti != tj || row >= col)) Cp[row + col * cs] = c[b][v] + ll[b][v];
     }
 }
 
