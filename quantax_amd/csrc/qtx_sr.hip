@@ -225,8 +225,8 @@ __device__ __forceinline__ void super_tile_of(int t, int mt, int& bi, int& bj) {
 // would leave the last round of a 4096-row Gram 69 % full.  A thread stages
 // four consecutive columns of one row of each operand per 16-column chunk: one
 // four-element load of O (which needs only the element's own alignment, so any
-// np takes it), fetched one chunk ahead into registers and centred in FP64 (the
-// rows' factors are applied to the sums), then written to the other of two LDS
+// np takes it), fetched one chunk ahead into registers and centred in FP64,
+// then written to the other of two LDS
 // buffers: one barrier per chunk.  FP64, 4096 x 40400: 44.3 -> 11.7 ms; 4096 x 34952: 38.3
 // -> 10.2 ms; 16384 x 34952: 331 -> 154 ms (60 TFLOP/s, a library f64 GEMM
 // reaches 73).  The matrix pipe is busy 80 % of the time (SQ counters); the
@@ -256,6 +256,11 @@ __device__ __forceinline__ void gram_nt_tile(const TI* __restrict__ O, const dou
   const TI* pb = O + rb * np;
   ST* sa = (second ? Bs : As) + srow * GN_LD + sk;
   ST* sb = Bs + srow * GN_LD + sk;
+  // FP32: the row factors go to the staged values, which keeps the products of
+  // large O in range (2 to 4 % of its time); FP64: to the sums
+  constexpr bool SHADOW = (G != QTX_GRAM_FP64);
+  const double fa = SHADOW ? sqrt((r ? r[second ? rb : ra] : 1.0) * inv_ns) : 1.0;
+  const double fb = SHADOW ? sqrt((r ? r[rb] : 1.0) * inv_ns) : 1.0;
   TI av[4], bv[4];
   double mv[4];
   auto fetch = [&](int64_t k0) {
@@ -283,8 +288,12 @@ __device__ __forceinline__ void gram_nt_tile(const TI* __restrict__ O, const dou
   auto stage = [&](int buf) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      sa[buf * S * GN_LD + q] = (ST)((double)av[q] - mv[q]);
-      if (S == 64) sb[buf * S * GN_LD + q] = (ST)((double)bv[q] - mv[q]);
+      const double x = (double)av[q] - mv[q];
+      sa[buf * S * GN_LD + q] = (ST)(SHADOW ? x * fa : x);
+      if (S == 64) {
+        const double y = (double)bv[q] - mv[q];
+        sb[buf * S * GN_LD + q] = (ST)(SHADOW ? y * fb : y);
+      }
     }
   };
 
@@ -296,7 +305,6 @@ __device__ __forceinline__ void gram_nt_tile(const TI* __restrict__ O, const dou
   // the FP32 mode flushes its MFMA accumulators into FP64 every FLUSH chunks
   // (256 columns), so the rounding error does not grow with np
   constexpr int FLUSH = 256 / GN_KC;
-  constexpr bool SHADOW = (G != QTX_GRAM_FP64);
   v4d dacc[SHADOW ? NB : 1][SHADOW ? NB : 1];
   if constexpr (SHADOW) {
 #pragma unroll
@@ -365,8 +373,7 @@ __device__ __forceinline__ void gram_nt_tile(const TI* __restrict__ O, const dou
           if constexpr (SHADOW)
             v = dacc[a][b][q];
           else
-            v = acc[a][b][q];
-          v *= r ? sqrt(r[gi] * r[gj]) * inv_ns : inv_ns;
+            v = acc[a][b][q] * (r ? sqrt(r[gi]) * sqrt(r[gj]) * inv_ns : inv_ns);
           T[gi * n + gj] = v;
           T[gj * n + gi] = v;
         }
@@ -647,7 +654,8 @@ __global__ __launch_bounds__(WAVE * TN_W) void gram_tn_kernel(const TI* __restri
       const int64_t s = s0 + 4 * TN_W * u + 4 * q + g, sc = s < ns ? s : ns - 1;
       a[p][u] = O[sc * np + kc];
       b[p][u] = O[sc * np + lc];
-      w[p][u] = s < ns ? (r ? r[sc] : 1.0) * inv_ns : 0.0;
+      const double rs = r ? r[sc] : 1.0;
+      w[p][u] = s < ns ? (rs < 0.0 ? NAN : rs) * inv_ns : 0.0;  // of a negative factor there is no root
     }
   };
   auto use = [&](int p) {
