@@ -80,8 +80,9 @@ class Variational:
     def fused_symm(self) -> bool:
         """A projected float64 RBM whose weights fit the kernels that form no
         images (float32 ones keep the general path: their amplitudes are
-        rounded in its order)."""
-        return self._symm is not None and self._symm.fuses(self._model)
+        rounded in its order), under a state with this class's own amplitudes."""
+        return (self._symm is not None and type(self).__call__ is Variational.__call__
+                and self._symm.fuses(self._model))
 
     def jacobian(self, fock_states) -> torch.Tensor:
         s = torch.as_tensor(fock_states, device=_lib.device()).to(torch.int8).reshape(-1, self.Nmodes)

@@ -155,8 +155,12 @@ class Symmetry:
         return out
 
     def fuses(self, model) -> bool:
-        """Whether ``model`` is projected by the kernels without images."""
-        return (isinstance(model, RBM_Dense) and model.theta.dtype == torch.float64 and model.N == self._N
+        """Whether ``model`` is projected by the kernels without images: an RBM_Dense
+        whose ``logpsi`` is the class's own, under this class's own images and
+        projection (they take the place of all three)."""
+        return (isinstance(model, RBM_Dense) and getattr(model.logpsi, "__func__", None) is RBM_Dense.logpsi
+                and type(self).images is Symmetry.images and type(self).project is Symmetry.project
+                and model.theta.dtype == torch.float64 and model.N == self._N
                 and bool(_lib.lib().qtx_symm_rbm_supported(model.M, model.N, self._perm.shape[0])))
 
     def rbm_args(self, model) -> tuple:
