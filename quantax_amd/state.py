@@ -71,7 +71,7 @@ class Variational:
         if self._symm is None:
             la = self._model.logpsi(s)
             return LogArray(torch.ones_like(la), la)
-        if self.fused_symm:
+        if self.fused_symm and not self._symm.images_faster(self._model, s.shape[0]):
             return LogArray(*self._symm.rbm_logpsi(self._model, s.contiguous()))
         sg, la = self._symm.project(self._model.logpsi(self._symm.images(s)))
         return LogArray(sg, la)

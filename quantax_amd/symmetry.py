@@ -163,6 +163,21 @@ class Symmetry:
                 and model.theta.dtype == torch.float64 and model.N == self._N
                 and bool(_lib.lib().qtx_symm_rbm_supported(model.M, model.N, self._perm.shape[0])))
 
+    def images_faster(self, model, ns: int) -> bool:
+        """Whether images -> forward -> projection is faster than those kernels for ns
+        configurations: small groups, which leave most of a tile of 16 permutations
+        idle, in large batches.  Per configuration the kernels take about 60 + 3/4 N +
+        6 (M / 4) units of 26 ps without spin inversion and 72 + 3/4 N + 9 (M / 4) with
+        it, the images N + 20 each; three launches and their waits are worth 8e5 units
+        (us for 131072 configurations, these kernels | images): 6 x 6, M = 36,
+        inversion alone 620 | 384, two permutations 486 | 385, three 487 | 547, two and
+        inversion 622 | 706; M = 64: 830 | 385, 626 | 384, 626 | 546, 829 | 706; M = 12:
+        419 | 381, 356 | 384; 8192 configurations, M = 36, inversion 45 | 34, 4096: 27 |
+        30.  A sweep's steps cost the images two more launches each: never faster."""
+        groups = (model.M + 3) // 4
+        fused = 0.75 * self._N + (72 + 9 * groups if self._Z2 else 60 + 6 * groups)
+        return ns * fused > 8e5 and self.nsymm * (self._N + 20) < fused
+
     def rbm_args(self, model) -> tuple:
         """The model and group arguments of ``qtx_symm_rbm_*``."""
         perm, coef = self._device()
