@@ -42,23 +42,28 @@ __global__ void fill_i32_kernel(int32_t* p, int64_t n, int32_t v) {
 //   W = false: out_k += sum_s O_sk
 //   W = true:  out_k += sum_s (O_sk - mean_k) sqrt(r_s inv_ns) y_s
 // HBM-bound: every element is read once.  A lane takes four neighbouring
-// columns (one load that needs only the element's own alignment), a wave 256
-// columns of every fourth row of the chunk, CS_ROWS rows in flight; the rows'
-// weights are made once, in LDS, CS_PART at a time.  colsum_rows: eight
-// workgroups per CU, of at least CS_MIN rows each: few columns fill the chip too.
-// 4096 x 40400 f32: sum 237 -> 173 us, weighted 257 -> 119 us; 1024 x 272 f64:
-// 33 -> 9.7, 64 -> 8.5 us (one column per thread, one row in flight before).
-constexpr int CS_COLS = 256, CS_ROWS = 8, CS_MIN = 16, CS_PART = 512;
+// columns (one load that needs only the element's own alignment), 2^lg lanes a
+// row (64, fewer where np <= 128, so that narrow rows fill the wave too), CS_ROWS
+// rows per lane in flight, the last ones of a chunk masked; the rows'
+// weights are made once, in LDS, CS_PART at a time.  The sums leave by one column
+// per thread: an atomic of a wave touches 512 bytes, where a lane's four columns
+// one after another touched 2 KB each time.
+// us, means of f32 (one column per thread and row before | this): 4096 x 40400 204 |
+// 118, 4096 x 5000 41 | 19, 16384 x 1000 40 | 17, 65536 x 256 132 | 17, 100000 x 8 58 |
+// 14, 16 x 1000000 24 | 20, 1024 x 272 17.5 | 13.5.
+constexpr int CS_COLS = 256, CS_ROWS = 8, CS_MIN = 16, CS_CHUNKS = 128, CS_PART = 2048;
 template <typename TI, bool W>
 __global__ __launch_bounds__(256) void colsum_kernel(const TI* __restrict__ O, const double* __restrict__ mean,
                                                      const double* __restrict__ r, const double* __restrict__ y,
-                                                     int64_t ns, int64_t np, int64_t rows_per_chunk, double inv_ns,
-                                                     double* __restrict__ out) {
+                                                     int64_t ns, int64_t np, int64_t rows_per_chunk, int lg,
+                                                     double inv_ns, double* __restrict__ out) {
   typedef TI vt4 __attribute__((ext_vector_type(4), aligned(sizeof(TI))));
-  __shared__ double ws[CS_PART];
-  __shared__ double red[3][CS_COLS];
+  __shared__ double ws[W ? CS_PART : 1];
+  __shared__ double red[4][CS_COLS];
   const int tid = threadIdx.x, lane = tid % WAVE, q = tid / WAVE;
-  const int64_t k0 = (int64_t)blockIdx.x * CS_COLS, k = k0 + 4 * lane;
+  const int cl = lane & ((1 << lg) - 1), rw = WAVE >> lg;  // column group of the lane, rows of a wave
+  const int first = q * rw + (lane >> lg), step = 4 * rw;
+  const int64_t k0 = (int64_t)blockIdx.x * CS_COLS, k = k0 + 4 * cl;
   const int64_t rc = (int64_t)blockIdx.y * rows_per_chunk;
   const int64_t re = rc + rows_per_chunk < ns ? rc + rows_per_chunk : ns;
   const int cols = (int)(k + 4 <= np ? 4 : k < np ? np - k : 0);
@@ -76,42 +81,56 @@ __global__ __launch_bounds__(256) void colsum_kernel(const TI* __restrict__ O, c
     }
     const TI* p = O + r0 * np + k;
     if (cols == 4) {
-      int s = q;
-      for (; s + 4 * (CS_ROWS - 1) < rows; s += 4 * CS_ROWS) {
+      int s = first;
+      for (; s + step * (CS_ROWS - 1) < rows; s += step * CS_ROWS) {
         vt4 v[CS_ROWS];
 #pragma unroll
-        for (int i = 0; i < CS_ROWS; ++i) v[i] = *reinterpret_cast<const vt4*>(p + (s + 4 * i) * np);
+        for (int i = 0; i < CS_ROWS; ++i) v[i] = *reinterpret_cast<const vt4*>(p + (s + step * i) * np);
 #pragma unroll
         for (int i = 0; i < CS_ROWS; ++i)
 #pragma unroll
-          for (int c = 0; c < 4; ++c) acc[c] += W ? ((double)v[i][c] - m[c]) * ws[s + 4 * i] : (double)v[i][c];
+          for (int c = 0; c < 4; ++c) acc[c] += W ? ((double)v[i][c] - m[c]) * ws[s + step * i] : (double)v[i][c];
       }
-      for (; s < rows; s += 4) {
-        const vt4 v = *reinterpret_cast<const vt4*>(p + s * np);
+      if (s < rows) {
+        vt4 v[CS_ROWS];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[c] += W ? ((double)v[c] - m[c]) * ws[s] : (double)v[c];
+        for (int i = 0; i < CS_ROWS; ++i)
+          v[i] = *reinterpret_cast<const vt4*>(p + (s + step * i < rows ? s + step * i : s) * np);
+#pragma unroll
+        for (int i = 0; i < CS_ROWS; ++i)
+          if (s + step * i < rows)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc[c] += W ? ((double)v[i][c] - m[c]) * ws[s + step * i] : (double)v[i][c];
       }
     } else if (cols > 0) {
-      for (int s = q; s < rows; s += 4)
+#pragma unroll 4
+      for (int s = first; s < rows; s += step)
 #pragma unroll
         for (int c = 0; c < 3; ++c)
           if (c < cols) acc[c] += W ? ((double)p[s * np + c] - m[c]) * ws[s] : (double)p[s * np + c];
     }
   }
-  if (q > 0)
+  for (int d = 1 << lg; d < WAVE; d *= 2)  // over the rows of a wave
 #pragma unroll
-    for (int c = 0; c < 4; ++c) red[q - 1][4 * lane + c] = acc[c];
+    for (int c = 0; c < 4; ++c) acc[c] += __shfl_xor(acc[c], d, WAVE);
+  if (lane < 1 << lg)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) red[q][4 * cl + c] = acc[c];
   __syncthreads();
-  if (q == 0)
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      if (c < cols) atomicAdd(out + k + c, acc[c] + red[0][4 * lane + c] + red[1][4 * lane + c] + red[2][4 * lane + c]);
+  // one column per thread: neighbouring atomics
+  if (tid < 4 << lg && k0 + tid < np) atomicAdd(out + k0 + tid, red[0][tid] + red[1][tid] + red[2][tid] + red[3][tid]);
 }
 
-// rows per chunk, and the grid
-static int64_t colsum_rows(int64_t ns, int64_t np, dim3& g) {
-  const int64_t gx = (np + CS_COLS - 1) / CS_COLS;
-  const int64_t chunks = std::min<int64_t>(std::max<int64_t>(1, 2048 / gx), (ns + CS_MIN - 1) / CS_MIN);
+// rows per chunk, the grid and lg: workgroups of at least CS_MIN wave rows, eight per
+// CU, but at most CS_CHUNKS of them, whose atomics on one sum wait for each other (us
+// with 32 | 64 | 128 | 256: 1000000 x 3 41 | 24 | 15 | 14, 65536 x 256 39 | 23 | 17 | 19,
+// 16384 x 1000 17 | 16 | 17 | 17)
+static int64_t colsum_rows(int64_t ns, int64_t np, dim3& g, int& lg) {
+  lg = 0;
+  while (lg < 6 && (4 << lg) < np) ++lg;
+  const int64_t gx = (np + CS_COLS - 1) / CS_COLS, least = (int64_t)CS_MIN * (WAVE >> lg);
+  const int64_t fill = std::min<int64_t>(CS_CHUNKS, std::max<int64_t>(1, 2048 / gx));
+  const int64_t chunks = std::min<int64_t>(fill, (ns + least - 1) / least);
   const int64_t rpc = (ns + chunks - 1) / chunks;
   g = dim3((unsigned)gx, (unsigned)((ns + rpc - 1) / rpc));
   return rpc;
@@ -1790,8 +1809,10 @@ static int launch_obar_t_y(hipStream_t st, const TI* O, const double* mean, cons
                            int64_t ns, int64_t np, double* x) {
   hipLaunchKernelGGL(fill_f64_kernel, dim3(nblk(np, 256)), dim3(256), 0, st, x, np, 0.0);
   dim3 g;
-  const int64_t rpc = colsum_rows(ns, np, g);
-  hipLaunchKernelGGL((colsum_kernel<TI, true>), g, dim3(256), 0, st, O, mean, r, y, ns, np, rpc, 1.0 / (double)ns, x);
+  int lg;
+  const int64_t rpc = colsum_rows(ns, np, g, lg);
+  hipLaunchKernelGGL((colsum_kernel<TI, true>), g, dim3(256), 0, st, O, mean, r, y, ns, np, rpc, lg, 1.0 / (double)ns,
+                     x);
   QTX_LAUNCH_CHECK();
   return QTX_OK;
 }
@@ -3143,14 +3164,15 @@ int qtx_colmean(void* stream, int o_dtype, const void* O, int64_t ns, int64_t np
   hipStream_t st = as_stream(stream);
   hipLaunchKernelGGL(fill_f64_kernel, dim3(nblk(np, 256)), dim3(256), 0, st, mean, np, 0.0);
   dim3 g;
-  const int64_t rpc = colsum_rows(ns, np, g);
+  int lg;
+  const int64_t rpc = colsum_rows(ns, np, g, lg);
   const double* none = nullptr;
   if (o_dtype == QTX_F32)
     hipLaunchKernelGGL((colsum_kernel<float, false>), g, dim3(256), 0, st, (const float*)O, none, none, none, ns, np,
-                       rpc, 0.0, mean);
+                       rpc, lg, 0.0, mean);
   else
     hipLaunchKernelGGL((colsum_kernel<double, false>), g, dim3(256), 0, st, (const double*)O, none, none, none, ns, np,
-                       rpc, 0.0, mean);
+                       rpc, lg, 0.0, mean);
   hipLaunchKernelGGL(scale_f64_kernel, dim3(nblk(np, 256)), dim3(256), 0, st, mean, np, 1.0 / (double)ns);
   QTX_LAUNCH_CHECK();
   return QTX_OK;
