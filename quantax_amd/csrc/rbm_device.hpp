@@ -28,16 +28,21 @@ __device__ __forceinline__ void rbm_hidden(const T* __restrict__ Wt, const T* __
     h[r] = (i < M) ? b[i] : T(0);
   }
   // J rows in flight at once, added in order: one row at a time, the wave waits
-  // for the L2 in every one (4096 samples, 100 x 400: 90 -> 36 us)
+  // for the L2 in every one (4096 samples, 100 x 400: 90 -> 36 us).  Lanes past M load
+  // nothing, because a load takes the L1 for as many lanes as it has (8192 samples, us
+  // with the last unit's weights in their place | without: 36 x 144 FP64 41 | 33, 100 x
+  // 400 188 | 163, FP32 63 | 54), but for single rows, whose many loads a branch each
+  // would hold up (1000 samples, 100 x 1000 FP64: 62 | 77)
   constexpr int J = sizeof(T) * R <= 16 ? 8 : sizeof(T) * R <= 32 ? 4 : sizeof(T) * R <= 64 ? 2 : 1;
   int j = 0;
   for (; j + J <= N; j += J) {
     T w[J][R];
+    const T* row = Wt + (int64_t)j * M + lane;
 #pragma unroll
-    for (int u = 0; u < J; ++u) {
-      const T* row = Wt + (int64_t)(j + u) * M;
+    for (int r = 0; r < R; ++r) {
+      if (J > 1 && lane + WAVE * r >= M) continue;
 #pragma unroll
-      for (int r = 0; r < R; ++r) w[u][r] = row[lane + WAVE * r < M ? lane + WAVE * r : M - 1];
+      for (int u = 0; u < J; ++u) w[u][r] = row[u * M + (lane + WAVE * r < M ? WAVE * r : M - 1 - lane)];
     }
 #pragma unroll
     for (int u = 0; u < J; ++u) {
