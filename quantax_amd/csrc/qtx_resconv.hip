@@ -104,41 +104,50 @@ __global__ void rc_pack_frag_kernel(const float* __restrict__ theta, int nb, cha
   }
 }
 
-// The Jacobian's FP32 A fragments of layers 1 .. 2nb-1, whatever the forward's
-// precision: per layer and direction (0: forward, 1: input gradient, with the
-// two channel indices exchanged and the taps mirrored) [tap][row tile][column
-// half][lane][4]: row = 16 ct + lane % 16, column = 16 h + 4 (lane / 16) + j,
-// so a lane reads its four K values of a tap in one 16-byte load
+// Everything but the fragments of rc_pack_frag_kernel, in one launch: the copy of
+// theta, layer 0's weights and bias, the layers' biases, and the FP32 A fragments
+// of layers 1 .. 2nb-1, which the Jacobian reads whatever the forward's precision and
+// the any-lattice FP32 forward reads too: per layer and direction (0: forward, 1:
+// input gradient, with the two channel indices exchanged and the taps mirrored)
+// [tap][row tile][column half][lane][4]: row = 16 ct + lane % 16, column = 16 h +
+// 4 (lane / 16) + j, so a lane reads its four K values of a tap in one 16-byte load
 template <int C>
-__global__ void rc_pack_jac_kernel(const float* __restrict__ theta, int nb, float* __restrict__ dst) {
+__global__ void rc_pack_kernel(const float* __restrict__ theta, int nb, int64_t nparams, float* __restrict__ packed,
+                               int64_t off_l0w, int64_t off_l0b, int64_t bias_off, float* __restrict__ frag) {
   constexpr int CT = C / 16;
-  const int64_t per = (int64_t)C * C * 9;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)(2 * nb - 1) * 2 * per) return;
-  const int l = 1 + (int)(idx / (2 * per)), dir = (int)(idx / per) & 1;
-  const int e = (int)(idx % per);
-  const int j = e % 4, lane = (e / 4) % WAVE, h = (e / 256) % CT, ct = (e / 256 / CT) % CT, tap = e / 256 / CT / CT;
-  const int row = 16 * ct + lane % 16, col = 16 * h + 4 * (lane / 16) + j;
-  const int64_t w0 = 10 * C + (int64_t)(l - 1) * (per + C);  // layer l >= 1 of rc_theta_offsets
-  dst[((int64_t)l * 2 + dir) * per + e] =
-      dir == 0 ? theta[w0 + ((int64_t)row * C + col) * 9 + tap] : theta[w0 + ((int64_t)col * C + row) * 9 + (8 - tap)];
-}
-
-__global__ void rc_pack_misc_kernel(const float* __restrict__ theta, int nb, int C, int64_t nparams,
-                                    float* __restrict__ packed, int64_t off_l0w, int64_t off_l0b, int64_t bias_off) {
-  int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx < nparams) packed[idx] = theta[idx];
-  int64_t j = idx - nparams;
-  if (j >= 0 && j < (int64_t)C * 9) packed[off_l0w + j] = theta[j];  // layer 0 weights start at 0
-  j -= (int64_t)C * 9;
-  if (j >= 0 && j < C) packed[off_l0b + j] = theta[(int64_t)C * 9 + j];
+  constexpr int64_t per = (int64_t)C * C * 9;
+  int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < nparams) {
+    packed[j] = theta[j];
+    return;
+  }
+  j -= nparams;
+  if (j < C * 9) {
+    packed[off_l0w + j] = theta[j];  // layer 0 weights start at 0
+    return;
+  }
+  j -= C * 9;
+  if (j < C) {
+    packed[off_l0b + j] = theta[C * 9 + j];
+    return;
+  }
   j -= C;
-  if (j >= 0 && j < (int64_t)2 * nb * C) {
-    int l = (int)(j / C), co = (int)(j % C);
+  if (j < (int64_t)2 * nb * C) {
+    const int l = (int)(j / C), co = (int)(j % C);
     int64_t w0, b0;
     rc_theta_offsets(nb, C, l, w0, b0);
     packed[bias_off + j] = (b0 >= 0) ? theta[b0 + co] : 0.0f;
+    return;
   }
+  j -= (int64_t)2 * nb * C;
+  if (j >= (int64_t)(2 * nb - 1) * 2 * per) return;
+  const int l = 1 + (int)(j / (2 * per)), dir = (int)(j / per) & 1;
+  const int e = (int)(j % per);
+  const int i = e % 4, lane = (e / 4) % WAVE, h = (e / 256) % CT, ct = (e / 256 / CT) % CT, tap = e / 256 / CT / CT;
+  const int row = 16 * ct + lane % 16, col = 16 * h + 4 * (lane / 16) + i;
+  const int64_t w0 = 10 * C + (int64_t)(l - 1) * (per + C);  // layer l >= 1 of rc_theta_offsets
+  frag[((int64_t)l * 2 + dir) * per + e] =
+      dir == 0 ? theta[w0 + ((int64_t)row * C + col) * 9 + tap] : theta[w0 + ((int64_t)col * C + row) * 9 + (8 - tap)];
 }
 
 // ---------------------------------------------------------------- forwards
@@ -1082,31 +1091,25 @@ int qtx_resconv_pack(void* stream, const qtx_resconv_desc* d, const float* theta
   QTX_REQUIRE(theta && packed, "null pointer");
   RcLayout L = rc_layout(d);
   hipStream_t st = as_stream(stream);
-  int64_t misc = L.nparams + (int64_t)L.C * 10 + (int64_t)2 * L.nb * L.C;
-  hipLaunchKernelGGL(rc_pack_misc_kernel, dim3((unsigned)((misc + 255) / 256)), dim3(256), 0, st, theta, L.nb, L.C,
-                     L.nparams, (float*)packed, L.off_l0w, L.off_l0b, L.bias_off);
-  const int64_t jac = (int64_t)(2 * L.nb - 1) * 2 * L.C * L.C * 9;
-  float* jf = (float*)((char*)packed + L.off_jac);
+  const int64_t n = L.nparams + (int64_t)L.C * 10 + (int64_t)2 * L.nb * L.C + (int64_t)(2 * L.nb - 1) * 2 * L.C * L.C * 9;
+  float* frag = (float*)((char*)packed + L.off_jac);
+  const dim3 b(256), gp((unsigned)((n + 255) / 256));
   if (L.C == 16)
-    hipLaunchKernelGGL(rc_pack_jac_kernel<16>, dim3((unsigned)((jac + 255) / 256)), dim3(256), 0, st, theta, L.nb, jf);
+    hipLaunchKernelGGL(rc_pack_kernel<16>, gp, b, 0, st, theta, L.nb, L.nparams, (float*)packed, L.off_l0w, L.off_l0b,
+                       L.bias_off, frag);
   else
-    hipLaunchKernelGGL(rc_pack_jac_kernel<32>, dim3((unsigned)((jac + 255) / 256)), dim3(256), 0, st, theta, L.nb, jf);
-  int ct = L.C / 16;
-  int ks = (L.mode == QTX_CONV_FP32) ? 9 * L.C / 4 : (L.C == 16 ? (L.win ? 6 : 5) : 9);
-  int64_t total = (int64_t)ct * ks * WAVE * (2 * L.nb - 1);
-  if (total > 0) {
-    dim3 g((unsigned)((total + 255) / 256)), b(256);
-    if (L.C == 16 && L.mode == QTX_CONV_FP32)
-      hipLaunchKernelGGL((rc_pack_frag_kernel<16, QTX_CONV_FP32, 0>), g, b, 0, st, theta, L.nb, (char*)packed,
+    hipLaunchKernelGGL(rc_pack_kernel<32>, gp, b, 0, st, theta, L.nb, L.nparams, (float*)packed, L.off_l0w, L.off_l0b,
+                       L.bias_off, frag);
+  if (L.frag_bytes > 0) {
+    const dim3 g((unsigned)((rc_frag_steps(L) * WAVE * (2 * L.nb - 1) + 255) / 256));
+    if (L.mode == QTX_CONV_FP32)
+      hipLaunchKernelGGL((rc_pack_frag_kernel<16, QTX_CONV_FP32, 1>), g, b, 0, st, theta, L.nb, (char*)packed,
                          L.off_frag, L.frag_bytes);
-    else if (L.C == 16 && L.win)
+    else if (L.win)
       hipLaunchKernelGGL((rc_pack_frag_kernel<16, QTX_CONV_BF16X3, 1>), g, b, 0, st, theta, L.nb, (char*)packed,
                          L.off_frag, L.frag_bytes);
     else if (L.C == 16)
       hipLaunchKernelGGL((rc_pack_frag_kernel<16, QTX_CONV_BF16X3, 0>), g, b, 0, st, theta, L.nb, (char*)packed,
-                         L.off_frag, L.frag_bytes);
-    else if (L.mode == QTX_CONV_FP32)
-      hipLaunchKernelGGL((rc_pack_frag_kernel<32, QTX_CONV_FP32, 0>), g, b, 0, st, theta, L.nb, (char*)packed,
                          L.off_frag, L.frag_bytes);
     else
       hipLaunchKernelGGL((rc_pack_frag_kernel<32, QTX_CONV_BF16X3, 0>), g, b, 0, st, theta, L.nb, (char*)packed,

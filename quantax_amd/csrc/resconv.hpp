@@ -22,9 +22,9 @@ struct RcLayout {
   int64_t nparams;
   int64_t off_l0w, off_l0b;  // first conv (Cin = 1): W (C, 9), b (C) in floats
   int64_t off_frag;          // start of per-layer fragment blocks (bytes)
-  int64_t frag_bytes;        // bytes of one layer's fragments
+  int64_t frag_bytes;        // bytes of one layer's fragments, see rc_frag_steps
   int64_t bias_off;          // start of per-layer biases (floats, (2nb) x C)
-  int64_t off_jac;           // start of the Jacobian's FP32 fragments (bytes), see rc_pack_jac_kernel
+  int64_t off_jac;           // start of the Jacobian's FP32 fragments (bytes), see rc_pack_kernel
   int64_t total_bytes;
 };
 
@@ -55,6 +55,14 @@ __host__ __device__ inline void rc_theta_offsets(int nb, int C, int l, int64_t& 
   w = b = -1;
 }
 
+// 64-lane fragments of one layer at off_frag: none for the any-lattice FP32 kernels,
+// which read the Jacobian's
+inline int64_t rc_frag_steps(const RcLayout& L) {
+  const int ct = L.C / 16;
+  if (L.mode == QTX_CONV_FP32) return L.win ? ct * 9 * L.C / 4 : 0;
+  return ct * (L.C == 16 ? (L.win ? 6 : 5) : 9);
+}
+
 inline RcLayout rc_layout(const qtx_resconv_desc* d) {
   RcLayout L;
   L.nb = d->nblocks;
@@ -77,10 +85,7 @@ inline RcLayout rc_layout(const qtx_resconv_desc* d) {
   off += (int64_t)2 * L.nb * L.C * 4;
   off = (off + 255) & ~(int64_t)255;
   L.off_frag = off;
-  int ct = L.C / 16;
-  int ks = (L.mode == QTX_CONV_FP32) ? 9 * L.C / 4 : (L.C == 16 ? (L.win ? 6 : 5) : 9);
-  int words = (L.mode == QTX_CONV_FP32) ? 1 : 8;
-  L.frag_bytes = (int64_t)ct * ks * WAVE * words * 4;
+  L.frag_bytes = rc_frag_steps(L) * WAVE * (L.mode == QTX_CONV_FP32 ? 1 : 8) * 4;
   off += L.frag_bytes * 2 * L.nb;  // slot per layer index (slot 0 unused)
   off = (off + 255) & ~(int64_t)255;
   L.off_jac = off;
