@@ -23,11 +23,6 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 // ---------------------------------------------------------------- helpers
-template <typename T>
-__device__ __forceinline__ double ld_as_double(const T* p, int64_t i) {
-  return (double)p[i];
-}
-
 __global__ void fill_f64_kernel(double* p, int64_t n, double v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -714,6 +709,8 @@ __global__ __launch_bounds__(WAVE * TN_W) void gram_tn_kernel(const TI* __restri
 // 272 10.7 | 43, 4096 x 272 35 | 137, 8192 x 272 63 | 232, 4096 x 512 94 | 135, 4096
 // x 1000 250 | 144, 8192 x 1000 482 | 911, 4096 x 2000 942 | 495
 constexpr int64_t kGramTnMax = 512;
+// whether the SR branch forms Obar in memory: S of more parameters, the SNR products
+static inline bool needs_obar(int64_t np, int mode) { return np > kGramTnMax || (mode & QTX_SOLVE_SNR); }
 
 template <typename TI>
 static int launch_gram_tn(hipStream_t st, const TI* O, const double* mean, const double* r, int64_t ns, int64_t np,
@@ -1690,7 +1687,7 @@ struct SolveWs {
   double* w;       // n: Lanczos work vector
   double* ab;      // alpha[kLanczosMax], beta[kLanczosMax + 1]
   void* split;     // bf16 hi / lo planes of Obar (split-bf16 Gram only)
-  double* obar;    // ns x np FP64 Obar (SR branch, ns >= np: S = Obar^T Obar by DGEMM)
+  double* obar;    // obar_rows x np FP64 Obar of a row block (SR branch, where needs_obar)
   double* var2;    // n: SNR truncation, sums of squared deviations (QTX_SOLVE_SNR)
   double* cbuf;    // obar_rows x np: Obar V of a row block (SR branch with QTX_SOLVE_SNR)
 };
@@ -1725,7 +1722,7 @@ static size_t ws_layout(int64_t ns, int64_t np, int mode, int gram, SolveWs* w, 
     s.ab = (double*)take((size_t)(2 * kLanczosMax + 1) * 8);
   }
   if (gram == QTX_GRAM_BF16X3 && mn) s.split = take(g3_bytes(ns, np));
-  if (!mn) s.obar = (double*)take((size_t)obar_rows(ns, np) * np * 8);
+  if (!mn && needs_obar(np, mode)) s.obar = (double*)take((size_t)obar_rows(ns, np) * np * 8);
   if (mode & QTX_SOLVE_SNR) {
     s.var2 = (double*)take((size_t)n * 8);
     if (!mn) s.cbuf = (double*)take((size_t)obar_rows(ns, np) * np * 8);
@@ -3032,8 +3029,9 @@ static int blas_query(rocblas_handle h, int64_t ns, int64_t np, int mode, SolveW
   bool good = true;
   if (!mn) {  // SR branch: S by row blocks of Obar, and the SNR products
     const rocblas_int npi = (rocblas_int)np, rows = (rocblas_int)obar_rows(ns, np);
-    good &= ok(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_transpose, npi, npi, rows, &one, w.obar,
-                             npi, w.obar, npi, &zero, w.T, npi));
+    if (np > kGramTnMax)
+      good &= ok(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_transpose, npi, npi, rows, &one, w.obar,
+                               npi, w.obar, npi, &zero, w.T, npi));
     if (mode & QTX_SOLVE_SNR)
       good &= ok(rocblas_dgemm(h, rocblas_operation_transpose, rocblas_operation_none, npi, rows, npi, &one, w.T, npi,
                                w.obar, npi, &zero, w.cbuf, npi));
