@@ -51,6 +51,21 @@ def test_sweep_samples_take_the_route_without_factors(ns, opt):
         assert np.linalg.norm(out[1][0] - out[0][0]) <= tol * np.linalg.norm(out[0][0])
 
 
+@pytest.mark.parametrize("solver", ["shift", "pinv"])
+@pytest.mark.parametrize("form", ["device", "single", "one", "strided", "host"])
+def test_ones_give_the_step_without_factors(solver, form):
+    """In whatever form; solvers whose route does not look at the factors."""
+    H, state, smp = _state(40)
+    one = torch.ones(40, dtype=torch.float64, device="cuda")
+    r = {"device": one, "single": one.float(), "one": one[:1], "strided": one[:1].expand(40), "host": one.cpu()}[form]
+    sv = qtx.optimizer.auto_shift_eig(rshift=1e-2, ashift=0.0) if solver == "shift" else qtx.optimizer.auto_pinv_eig(1e-2)
+    steps = [qtx.optimizer.SR(state, H, solver=sv).get_step(qtx.sampler.Samples(smp.spins, smp.psi, None, f))
+             for f in (None, r)]
+    # a condition number of at most 1e2 (40 rows of trace 1 at most, or the cutoff's)
+    tol = 32 * (40 + state.nparams) * 2.0**-53 * 1e2 * float(steps[0].norm())
+    assert float((steps[1] - steps[0]).norm()) <= tol
+
+
 def test_other_factors_take_dsyevd():
     H, state, smp = _state(40, reweight=1.5)
     assert not bool((smp.reweight_factor == 1.0).all())
