@@ -6,6 +6,8 @@
 // is one contiguous row of Wt.  One wavefront owns one chain / sample; lane l
 // holds hidden units l, l + 64, ... (R = ceil(M / 64) registers per lane).
 #pragma once
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace qtx {
@@ -31,28 +33,35 @@ __device__ __forceinline__ void rbm_hidden(const T* __restrict__ Wt, const T* __
   // for the L2 in every one (4096 samples, 100 x 400: 90 -> 36 us).  Lanes past M load
   // nothing, because a load takes the L1 for as many lanes as it has (8192 samples, us
   // with the last unit's weights in their place | without: 36 x 144 FP64 41 | 33, 100 x
-  // 400 188 | 163, FP32 63 | 54), but for single rows, whose many loads a branch each
-  // would hold up (1000 samples, 100 x 1000 FP64: 62 | 77)
+  // 400 188 | 163, FP32 63 | 54).  Single rows, whose many loads a branch on the lane
+  // each would hold up (1000 samples, 100 x 1000 FP64: 62 | 77), branch on registers
+  // that lie past M as a whole, where there are two of them at least (100 x 513, 1000
+  // and 32768 samples: 57, 1404 | 53, 850; x 800 58, 1415 | 68, 1191; x 960 60, 1417 |
+  // 76, 1357)
   constexpr int J = sizeof(T) * R <= 16 ? 8 : sizeof(T) * R <= 32 ? 4 : sizeof(T) * R <= 64 ? 2 : 1;
   int j = 0;
-  for (; j + J <= N; j += J) {
-    T w[J][R];
-    const T* row = Wt + (int64_t)j * M + lane;
+  auto batches = [&](auto skip) {
+    for (; j + J <= N; j += J) {
+      T w[J][R];
+      const T* row = Wt + (int64_t)j * M + lane;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      if (J > 1 && lane + WAVE * r >= M) continue;
+      for (int r = 0; r < R; ++r) {
+        if (skip.value && (J > 1 ? lane : 0) + WAVE * r >= M) continue;
 #pragma unroll
-      for (int u = 0; u < J; ++u) w[u][r] = row[u * M + (lane + WAVE * r < M ? WAVE * r : M - 1 - lane)];
+        for (int u = 0; u < J; ++u) w[u][r] = row[u * M + (lane + WAVE * r < M ? WAVE * r : M - 1 - lane)];
+      }
+#pragma unroll
+      for (int u = 0; u < J; ++u) {
+        const T sj = (T)sl[j + u];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          if (lane + WAVE * r < M) h[r] += w[u][r] * sj;
+      }
+      __builtin_amdgcn_sched_barrier(0);  // no second batch in registers
     }
-#pragma unroll
-    for (int u = 0; u < J; ++u) {
-      const T sj = (T)sl[j + u];
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        if (lane + WAVE * r < M) h[r] += w[u][r] * sj;
-    }
-    __builtin_amdgcn_sched_barrier(0);  // no second batch in registers
-  }
+  };
+  if (J == 1 && M > WAVE * (R - 2)) batches(std::false_type{});
+  else batches(std::true_type{});
   for (; j < N; ++j) {
     T sj = (T)sl[j];
     const T* row = Wt + (int64_t)j * M;
