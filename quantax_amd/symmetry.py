@@ -165,18 +165,36 @@ class Symmetry:
 
     def images_faster(self, model, ns: int) -> bool:
         """Whether images -> forward -> projection is faster than those kernels for ns
-        configurations: small groups, which leave most of a tile of 16 permutations
-        idle, in large batches.  Per configuration the kernels take about 60 + 3/4 N +
+        configurations.
+
+        Small groups, which leave most of a tile of 16 permutations idle, in large
+        batches.  Per configuration the kernels take about 60 + 3/4 N +
         6 (M / 4) units of 26 ps without spin inversion and 72 + 3/4 N + 9 (M / 4) with
         it, the images N + 20 each; three launches and their waits are worth 8e5 units
         (us for 131072 configurations, these kernels | images): 6 x 6, M = 36,
         inversion alone 620 | 384, two permutations 486 | 385, three 487 | 547, two and
         inversion 622 | 706; M = 64: 830 | 385, 626 | 384, 626 | 546, 829 | 706; M = 12:
         419 | 381, 356 | 384; 8192 configurations, M = 36, inversion 45 | 34, 4096: 27 |
-        30.  A sweep's steps cost the images two more launches each: never faster."""
-        groups = (model.M + 3) // 4
+        30.
+
+        Few configurations of a large group: a workgroup fills its table of the group
+        and takes the tiles of a configuration eight at a time, ``one`` units for the
+        first configuration, where the images spread over the card and their three calls
+        take 1.1e6 units from the host (us, one configuration, these kernels | images):
+        8 x 8, 512 permutations and inversion, M = 64: 62 | 29, M = 36: 48 | 29, M = 4:
+        29 | 29; 16 configurations, M = 64: 63 | 54; 8 x 8 without inversion, M = 64:
+        51 | 29, 16 configurations 52 | 31, 32: 52 | 48; 6 x 6, 288 permutations and
+        inversion, M = 64: 30 | 29; 64 permutations: at most 17 | 29.
+
+        A sweep's steps cost the images two more launches each: never faster."""
+        groups, nperm = (model.M + 3) // 4, len(self._perm)
         fused = 0.75 * self._N + (72 + 9 * groups if self._Z2 else 60 + 6 * groups)
-        return ns * fused > 8e5 and self.nsymm * (self._N + 20) < fused
+        images = self.nsymm * (self._N + 20)
+        if ns * fused > 8e5 and images < fused:
+            return True
+        tiles, ksteps = (nperm + 15) // 16, 4 if self._N <= 16 else 9 if self._N <= 36 else 16
+        one = 1.9e5 + 1600 * tiles * ksteps + tiles / 8 * groups * (850 * ksteps + (6500 if self._Z2 else 1900))
+        return one > max(1.2e6, 5e5 + ns * images)
 
     def rbm_args(self, model) -> tuple:
         """The model and group arguments of ``qtx_symm_rbm_*``."""
