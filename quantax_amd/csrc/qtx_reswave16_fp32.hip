@@ -8,7 +8,7 @@ namespace qtx {
 template <>
 int rw_logpsi<16, QTX_CONV_FP32>(hipStream_t st, const RcLayout& L, const RcArgs& a, const int8_t* s, int64_t ns,
                                 double* logabs) {
-  const RwPick pk = rw_pick(16, L.N, ns);
+  const RwPick pk = rw_pick(16, L.N, ns, false, true);
   if (pk.P == 1 && pk.maxt == 4) {
     RW_LAUNCH(rw_logpsi_kernel, 16, QTX_CONV_FP32, 4, 1, 1, 0, (ns + G - 1) / G,
               s, ns, logabs);

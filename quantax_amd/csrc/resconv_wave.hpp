@@ -412,19 +412,24 @@ struct RwFwd {
   }
 };
 
-// The source table: by every thread of the workgroup, barrier after it
+// The source table: by every thread of the workgroup, barrier after it.  A site per
+// thread and one division for its nine taps: a workgroup forms it for 4 / P forwards
+// (1300 of 10 x 16, one block, FP32: 31.1 -> 28.3 us against a division per entry)
 template <int C, int MODE>
 __device__ __forceinline__ void rw_build_tab(const RcGeom& g, uint16_t* tab) {
   using K = RwK<C, MODE>;
   const int npad = 16 * g.NT;
-  for (int e = threadIdx.x; e < K::ROWS * npad; e += RW_THREADS) {
-    const int row = e / npad, p = e - row * npad;
-    uint16_t v = 0;
-    if (p < g.N) {
-      const int src = row < 9 ? tap_pos(g, p / g.L1, p % g.L1, row) : p;  // row 9: zero weights, any finite input
-      v = (uint16_t)(src * (C * 4) + (((src / (8 / K::CH)) & (K::CH - 1)) << 4));
+  for (int p = threadIdx.x; p < npad; p += RW_THREADS) {
+    const int y = p / g.L1, x = p - y * g.L1;
+    const int ym = y == 0 ? g.L0 - 1 : y - 1, yp = y + 1 == g.L0 ? 0 : y + 1;
+    const int xm = x == 0 ? g.L1 - 1 : x - 1, xp = x + 1 == g.L1 ? 0 : x + 1;
+#pragma unroll
+    for (int row = 0; row < K::ROWS; ++row) {
+      const int ys = row / 3 == 0 ? ym : (row / 3 == 1 ? y : yp), xs = row % 3 == 0 ? xm : (row % 3 == 1 ? x : xp);
+      const int src = row < 9 ? ys * g.L1 + xs : p;  // row 9: zero weights, any finite input
+      const int v = src * (C * 4) + (((src / (8 / K::CH)) & (K::CH - 1)) << 4);
+      tab[row * npad + p] = (uint16_t)(p < g.N ? v : 0);
     }
-    tab[e] = v;
   }
 }
 
@@ -683,11 +688,23 @@ __global__ __launch_bounds__(RW_THREADS, 2) void rw_eloc_kernel(RcArgs a, RwMerg
 // chains whose proposal does not move leave their waves' time to the others, so
 // P = 4 stays best up to 1536 (8 x 8, FP32, 24 steps of 1000 chains: 535 | 625 us;
 // of 2000: 949 | 855) and P = 2 starts at 1793.
+// A forward of 16 channels in FP32 (fp32 set) goes by its tiles too: P = 4 leaves half the
+// waves of two tiles idle, half those of the second turn with five and six, the last
+// turn's with nine and more, where 768 and 1280 configurations (three and five per CU)
+// do not hide it.  us, one | four | eight blocks, P = 4 and the choice here: 2 x 16 at 1300
+// 12.6 | 34.7 | 62.7 and 9.1 | 27.4 | 51.3; 6 x 16 at 1000 14.8 | 46.0 | 88.3 and 12.8 | 42.6
+// | 81.9; 10 x 16 at 1300 28.2 | 103.5 | 204 and 24.0 | 91.1 | 181; 14 x 14 32.2 | 125 | 246
+// and 29.7 | 117 | 234.  Split-bf16 loses up to a tenth by it.
 struct RwPick {
   int P, maxt;
 };
-inline RwPick rw_pick(int C, int N, int64_t units, bool sweep = false) {
+inline RwPick rw_pick(int C, int N, int64_t units, bool sweep = false, bool fp32 = false) {
   const int nt = (N + 15) / 16;
+  if (fp32 && C == 16) {
+    if (nt == 2 && units > 768) return {1, 4};
+    if (nt > 4 && nt <= 6 && units > 768 && units <= 1024) return {1, 8};
+    if (nt > 8 && nt <= 16 && units > 1280) return {2, 8};
+  }
   const bool late = units > 1536, full = late || (!sweep && units > 768 && units <= 1024);
   if (nt == 1 && units >= 512) return {1, 4};
   if (full && nt <= 4) return {1, 4};
