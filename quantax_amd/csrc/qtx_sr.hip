@@ -707,7 +707,9 @@ __global__ __launch_bounds__(WAVE * TN_W) void gram_tn_kernel(const TI* __restri
 
 // np up to which a solve forms S by gram_tn_kernel (us, it | Obar and DGEMM): 1024 x
 // 272 10.7 | 43, 4096 x 272 35 | 137, 8192 x 272 63 | 232, 4096 x 512 94 | 135, 4096
-// x 1000 250 | 144, 8192 x 1000 482 | 911, 4096 x 2000 942 | 495
+// x 1000 250 | 144, 8192 x 1000 482 | 911, 4096 x 2000 942 | 495.  Many samples do not
+// move it, though a tile is one workgroup over all of them (whole shifted solves, ms):
+// 65536 x 72 0.45 | 7.3, 262144 x 272 1.7 | 14.9, 65536 x 512 1.4 | 8.0, 1000000 x 8 5.2 | 54
 constexpr int64_t kGramTnMax = 512;
 // whether the SR branch forms Obar in memory: S of more parameters, the SNR products
 static inline bool needs_obar(int64_t np, int mode) { return np > kGramTnMax || (mode & QTX_SOLVE_SNR); }
@@ -2121,7 +2123,8 @@ __global__ __launch_bounds__(256) void chol_panel_kernel(double* A, int64_t lda,
 // tiles), the last mt (with a right-hand side) the same for y as one more row.
 // One 64 x 64 tile per workgroup on transposed 16 x 16 MFMA tiles, wave q the
 // rows 16 q ..; all loads in flight at once, the products in a rolled loop.
-// 19 -> 8 us (4 x 4 register tiles before).
+// 19 -> 8 us in a block of 1024 columns (4 x 4 register tiles before); 22 on average in
+// one of 4096.
 __global__ __launch_bounds__(256) void chol_update_kernel(double* A, int64_t lda, int64_t stride, int64_t d0,
                                                           int64_t kb, int kp, const double* __restrict__ dtile,
                                                           double* y) {
