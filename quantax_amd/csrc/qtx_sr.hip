@@ -2568,6 +2568,10 @@ struct Task {
   int path = -1, fallback = 0;
 };
 
+// whether the weights' values choose the route: only below a cutoff of 1e-5 (a copy of
+// the flag costs about 20 us)
+static bool ones_asked(const Task& t) { return t.minnorm && t.io->r && !(t.io->rtol >= 1e-5); }
+
 static int task_fail(Task& t, int rc) {
   t.failed = true;
   t.io->status = rc;
@@ -2661,8 +2665,8 @@ static int phase1(Task& t, rocblas_handle h) {
   // recurrence; the largest Ritz value is checked every 32 steps)
   hipLaunchKernelGGL(lanczos_init_kernel, dim3(1), dim3(1024), 0, t.st, t.n, t.w.V, t.w.ab + kLanczosMax);
   t.mcap = (int)(t.n < kLanczosMax ? t.n : kLanczosMax);
-  // whether the weights are all one, for phase 2 (the small-cutoff route)
-  if (t.minnorm && io.r)
+  // whether the weights are all one, for the small-cutoff route of phase 2
+  if (ones_asked(t))
     hipLaunchKernelGGL(all_ones_kernel, dim3(1), dim3(1024), 0, t.st, io.r, io.ns, t.w.scalars + 2);
   // convergence checks every 16 steps when one product streams more than
   // 512 MB of T (n > 8192: 16 products cost far more than the host round
@@ -2756,8 +2760,8 @@ static int phase2(Task& t, rocblas_handle h) {
     double lmax = 0.0;
     int msteps = 0;
     bool bad = false;
-    double ones = 1.0;  // read with the coefficients: no further wait
-    if (t.minnorm && io.r)
+    double ones = io.r ? 0.0 : 1.0;  // read with the coefficients: no further wait
+    if (ones_asked(t))
       QTX_HIP(hipMemcpyAsync(&ones, t.w.scalars + 2, sizeof(double), hipMemcpyDeviceToHost, t.st));
     for (;;) {
       QTX_HIP(hipMemcpyAsync(ha.data(), t.w.ab, (size_t)t.done * 8, hipMemcpyDeviceToHost, t.st));
