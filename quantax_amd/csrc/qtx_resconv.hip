@@ -1173,7 +1173,7 @@ int qtx_resconv_metropolis(void* stream, const qtx_resconv_desc* d, const void* 
 // 10 x 10, 4 blocks (FP32) 17.6 -> 17.0 ms.
 static int eloc_split(const RcLayout& L, int32_t noff, int64_t ns) {
   const int64_t want = (16 * 512 + ns - 1) / ns;
-  const int batch = L.win ? 2 : (rc_own_kernel(L) ? 1 : 4 / rw_pick(L.C, L.N, ns * (noff / 4)).P);
+  const int batch = L.win ? 2 : (rc_own_kernel(L) ? 1 : 4 / rw_eloc_pick(L.C, L.N, noff, ns).P);
   const int64_t most = noff / 4 / (8 * batch);
   return (int)std::max<int64_t>(1, std::min(want, most));
 }

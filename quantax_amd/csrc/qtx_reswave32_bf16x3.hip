@@ -72,8 +72,7 @@ int rw_metropolis<32, QTX_CONV_BF16X3>(hipStream_t st, const RcLayout& L, const 
 template <>
 int rw_eloc<32, QTX_CONV_BF16X3>(hipStream_t st, const RcLayout& L, const RcArgs& a, const qtx_ham& H, const int8_t* s,
                               const double* logabs, int64_t ns, int S, double* eloc, int32_t* nconn) {
-  // about a quarter of an exchange Hamiltonian's candidates are valid
-  const RwPick pk = rw_pick(32, L.N, ns * (H.noff / 4));
+  const RwPick pk = rw_eloc_pick(32, L.N, H.noff, ns);
   if (pk.P == 1 && pk.maxt == 4) {
     RW_LAUNCH(rw_eloc_kernel, 32, QTX_CONV_BF16X3, 4, 1, 1, H.noff, ns * S,
               H, s, logabs, S, eloc, nconn);

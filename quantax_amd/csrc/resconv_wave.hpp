@@ -717,6 +717,18 @@ inline RwPick rw_pick(int C, int N, int64_t units, bool sweep = false, bool fp32
   return {4, nt <= 8 ? 2 : (nt <= 16 ? 4 : 7)};
 }
 
+// The choice for a local energy of ns samples: about a quarter of an exchange
+// Hamiltonian's candidates are valid.  On one or two tiles, where P = 4 leaves two or
+// three waves of each configuration idle, a table too short to be split over workgroups
+// with P = 4 (eloc_split) takes P = 1, four candidates at a time (us, 16 channels, four
+// blocks, P = 4 | P = 1, 3 to 200 samples: transverse-field Ising 3 x 5 FP32 140 | 45,
+// split-bf16 112 | 35, 4 x 8 309 | 135, 250 | 94; Heisenberg 3 x 5 168 | 55, 134 | 42; split
+// in two or more, 4 x 8 104 | 167, 85 | 116).
+inline RwPick rw_eloc_pick(int C, int N, int64_t noff, int64_t ns) {
+  if (C == 16 && N <= 32 && noff < 64) return {1, 4};
+  return rw_pick(C, N, ns * (noff / 4));
+}
+
 inline RwMerge rw_merge(const RcLayout& L) {
   return RwMerge{(L.C == 16 && L.L1 == 16 && L.L0 <= 16) ? 8 : 4, (L.C == 16 && L.N <= 256) ? 1 : 0};
 }
